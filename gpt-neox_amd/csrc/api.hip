@@ -120,7 +120,7 @@ struct SoftmaxCall {
             return;
         }
         a.mask = m;
-        a.rows_per_mask_batch = (uint32_t)((int64_t)np * a.sq);
+        a.by_mask_batch = FastDiv::by((uint32_t)((int64_t)np * a.sq));
         a.mask_bcast = (mask_b == 1 && b != 1) ? 1 : 0;
         a.mask_bytes = fits32((uint64_t)mask_b * (uint64_t)a.sq * (uint64_t)a.sk);
         vec_ok = vec_ok && aligned(m, 8);
@@ -138,7 +138,7 @@ struct SoftmaxCall {
         }
         vec_ok = vec_ok && aligned(t, 16);
         a.bias = t;
-        a.bias_rows = (bias_b == 1 && b != 1) ? (uint32_t)((int64_t)np * a.sq) : 0u;
+        if (bias_b == 1 && b != 1) a.by_bias_rows = FastDiv::by((uint32_t)((int64_t)np * a.sq));
         a.bias_bytes = fits32((uint64_t)bias_b * (uint64_t)np * (uint64_t)a.sq * (uint64_t)a.sk * 2u);
         features |= kBias;
     }
@@ -149,7 +149,7 @@ struct SoftmaxCall {
             status = fail(NEOX_ERR_BAD_SHAPE, "%s: mask batch dim %d must be 1 or b=%d", what, mask_b, b);
             return;
         }
-        a.rows_per_mask_batch = (uint32_t)((int64_t)np * a.sq);
+        a.by_mask_batch = FastDiv::by((uint32_t)((int64_t)np * a.sq));
         a.mask_bcast = (mask_b == 1 && b != 1) ? 1 : 0;
     }
     // where the visible keys of every mask row end, int32 [mask_b * sq]; null = no hint
@@ -169,7 +169,7 @@ struct SoftmaxCall {
             return;
         }
         a.slopes = slopes;
-        a.np = (uint32_t)np;
+        a.by_np = FastDiv::by((uint32_t)np);
         features |= kAlibi;
     }
     void dropout(float p, uint64_t seed, uint64_t offset, const uint64_t* device_state) {
@@ -215,6 +215,7 @@ struct SoftmaxCall {
         }
         a.rows = (uint32_t)n;
         a.sq = sq;
+        a.by_sq = FastDiv::by((uint32_t)sq);
         a.sk = sk;
     }
     // size of a tensor the packed kernels address through one buffer, 0 if it needs more than 32 bits

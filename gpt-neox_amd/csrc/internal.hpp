@@ -18,7 +18,7 @@ int fail(int status, const char* fmt, ...) __attribute__((format(printf, 2, 3)))
 // aligned); without it the launchers of a feature set without kRagged use their element-wise
 // kernels, and those with kRagged (8 <= sk < kMaxStagedRow) ignore it.
 // One specialisation per feature set, each in a translation unit of its own: FLAGS combines
-// kAlibi (a.slopes, a.np), kBias (a.bias, a.bias_rows, a.bias_bytes), kDropout (a.drop, and a.out2
+// kAlibi (a.slopes, a.by_np), kBias (a.bias, a.by_bias_rows, a.bias_bytes), kDropout (a.drop, and a.out2
 // in the forward pass) and kRagged for the forward pass, kDropout and kRagged for the backward pass.
 template <int FLAGS>
 hipError_t launch_softmax_fwd_flags(const SoftmaxArgs& a, Mask mask, int dtype, bool vec_ok, hipStream_t stream);

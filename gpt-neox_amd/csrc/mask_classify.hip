@@ -42,16 +42,17 @@ constexpr int kScanWaves = 16;  // waves per block
 // instead of several per row (which cost more than reading the mask: about 12 ns each).
 template <bool WIDE>
 __global__ __launch_bounds__(kScanWaves * kWave) void mask_classify_kernel(int32_t* record, int32_t* row_end,
-                                                                           const uint8_t* mask, uint32_t rows, int sq, int sk) {
+                                                                           const uint8_t* mask, uint32_t rows, FastDiv by_sq, int sk) {
     __shared__ int s_bad[kScanWaves], s_min[kScanWaves], s_max[kScanWaves], s_top[kScanWaves];
     __shared__ unsigned long long s_tail[kScanWaves];
     const int lane = threadIdx.x & (kWave - 1);
     const int wib = threadIdx.x >> 6;
     const uint32_t waves = gridDim.x * kScanWaves;
+    const int sq = (int)by_sq.d;
     int bad = 0, wmin = INT_MAX, wmax = -1, top = -1;  // wave-uniform, as in the record
     unsigned long long tail = 0;
     for (uint32_t row = blockIdx.x * kScanWaves + wib; row < rows; row += waves) {
-        const int i = (int)(row % (uint32_t)sq);
+        const int i = (int)by_sq.mod(row);
         const uint8_t* m = mask + (size_t)row * sk;
         int count = 0, first = INT_MAX, last = -1;
         if constexpr (WIDE) {  // sk % 8 == 0 and the tensor 8-byte aligned: 8 bytes per lane, 4 loads in flight
@@ -140,9 +141,10 @@ hipError_t launch_mask_classify(int32_t* record, int32_t* row_end, const uint8_t
     // two blocks per CU at most: the record takes a handful of atomic operations per block
     const uint32_t blocks = (rows + kScanWaves - 1) / kScanWaves;
     const dim3 grid(blocks < 512u ? blocks : 512u), block(kScanWaves * kWave);
+    const FastDiv by_sq = FastDiv::by((uint32_t)sq);
     const bool wide = sk % 8 == 0 && (reinterpret_cast<uintptr_t>(mask) & 7u) == 0;
-    if (wide) hipLaunchKernelGGL((mask_classify_kernel<true>), grid, block, 0, st, record, row_end, mask, rows, sq, sk);
-    else hipLaunchKernelGGL((mask_classify_kernel<false>), grid, block, 0, st, record, row_end, mask, rows, sq, sk);
+    if (wide) hipLaunchKernelGGL((mask_classify_kernel<true>), grid, block, 0, st, record, row_end, mask, rows, by_sq, sk);
+    else hipLaunchKernelGGL((mask_classify_kernel<false>), grid, block, 0, st, record, row_end, mask, rows, by_sq, sk);
     return hipGetLastError();
 }
 

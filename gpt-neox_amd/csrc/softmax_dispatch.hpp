@@ -43,14 +43,14 @@ namespace neox {
 // the output starts on a 4 KiB boundary.
 static SoftmaxArgs with_xcd_mapping(const SoftmaxArgs& a, uint64_t unit_bytes, uint32_t units, uint32_t blocks) {
     SoftmaxArgs b = a;
-    b.units_per_piece = 0;
+    b.piece_shift = 0;
     b.affine_blocks = 0;
     const bool aligned = (reinterpret_cast<uintptr_t>(a.out) & 4095u) == 0 &&
                          (a.out2 == nullptr || (reinterpret_cast<uintptr_t>(a.out2) & 4095u) == 0);
     if (aligned && unit_bytes > 0 && unit_bytes <= 4096 && 4096 % unit_bytes == 0 && blocks >= 8) {
         const uint32_t upp = (uint32_t)(4096 / unit_bytes);
         if (units % upp == 0 && units / upp >= 1) {
-            b.units_per_piece = upp;
+            b.piece_shift = (uint32_t)__builtin_ctz(upp);  // unit_bytes divides 4096: a power of two
             b.affine_blocks = blocks & ~7u;
         }
     }
