@@ -112,6 +112,73 @@ static bool try_launch_rope_piece(const RopeArgs& a, int s, int n_outer, hipStre
     return true;
 }
 
+template <typename T, typename CS, int PW, bool BWD>
+static hipError_t launch_rope_run(const RopeRunArgs& r, int nt, hipStream_t st) {
+    const uint32_t slots = nt > 1 && r.slots[1] > r.slots[0] ? r.slots[1] : r.slots[0];
+    const uint32_t pieces = (slots + kPieceSlots - 1) / kPieceSlots;
+    hipLaunchKernelGGL((rope_run_kernel<T, CS, PW, BWD>), dim3((pieces + 3) / 4, nt), dim3(256),
+                       4 * r.wave_floats * sizeof(float), st, r);
+    return hipGetLastError();
+}
+
+// Whole heads of dense tensors, out of place: the run kernel (see rope_run_kernel).  Returns false if the
+// call does not qualify.
+template <typename T, typename CS, bool BWD>
+static bool try_launch_rope_run(const RopeArgs& a, int s, int n_outer, hipStream_t st, hipError_t* err) {
+    const int d_rot = 2 * a.half, d = d_rot + a.copy_dims;
+    if (n_outer != 1 || d % kVec != 0 || a.half % 2 != 0) return false;
+    // Angles: always faster than rope_span_kernel, which alone takes them otherwise.  Tables: where the half span
+    // is no multiple of 8 dims the other kernels move 8 or 4 bytes per access; where it is, or where the whole head
+    // rotates, rope_piece_kernel reads nothing twice.  us per launch, fp16, that kernel or rope_span_kernel -> this:
+    // [2048,2,64,96] d_rot 24 angles 27.7 -> 19.0, tables 25.9 -> 19.3; [2048,2,40,80] d_rot 20 angles 28.6 -> 13.1,
+    // tables 24.5 -> 13.1, d_rot 40 angles 15.4 -> 13.2; angles [2048,2,64,128] d_rot 32 24.9 -> 23.4, d_rot = d = 96
+    // 20.5 -> 20.3; against it: tables [2048,2,64,128] d_rot 32 23.3 -> 23.7, d_rot = d = 128 13.3 -> 14.6,
+    // d_rot = d = 40 18.3 -> 19.1 (bf16, q and k).
+    if (!std::is_same<CS, Angles>::value && (a.half % kVec == 0 || a.copy_dims == 0)) return false;
+    RopeRunArgs r{};
+    uint32_t positions = 0;  // that a piece can touch
+    const uint32_t spv = (uint32_t)(d / kVec);
+    uintptr_t in_lo[2], in_hi[2], out_lo[2], out_hi[2];
+    for (int i = 0; i < a.nt; ++i) {
+        const RopeTensor& t = a.t[i];
+        const int64_t per_pos = (int64_t)t.n_inner * d;
+        if (t.in_stride[2] != d || t.out_stride[2] != d || t.in_stride[0] != per_pos || t.out_stride[0] != per_pos) return false;
+        in_lo[i] = reinterpret_cast<uintptr_t>(t.in), out_lo[i] = reinterpret_cast<uintptr_t>(t.out);
+        if (in_lo[i] % 16 != 0 || out_lo[i] % 16 != 0) return false;
+        const int64_t slots = (int64_t)t.n_inner * spv * s;
+        if ((int64_t)t.n_inner * spv > 0x7fffffffLL || slots > 0x7fffffffLL) return false;
+        in_hi[i] = in_lo[i] + (uintptr_t)slots * 16, out_hi[i] = out_lo[i] + (uintptr_t)slots * 16;
+        r.in[i] = t.in, r.out[i] = t.out;
+        r.slots[i] = (uint32_t)slots;
+        r.by_vpp[i] = FastDiv::by((uint32_t)t.n_inner);
+        const uint32_t vecs = (kPieceSlots - 2) / spv + 2;  // head vectors that 256 slots in a row can touch
+        const uint32_t p = (vecs - 2 + (uint32_t)t.n_inner) / (uint32_t)t.n_inner + 1;
+        if (p > positions) positions = p;
+    }
+    // a lane's partner is read from memory, so nothing that is read may be written
+    for (int i = 0; i < a.nt; ++i)
+        for (int o = 0; o < a.nt; ++o)
+            if (in_lo[i] < out_hi[o] && out_lo[o] < in_hi[i]) return false;
+    r.by_spv = FastDiv::by(spv);
+    r.by_rot = FastDiv::by((uint32_t)d_rot);
+    r.cos = a.cos, r.sin = a.sin;
+    r.cs_stride = a.cs_stride;
+    r.pos_offset = a.pos_offset;
+    r.half = a.half;
+    r.row = (uint32_t)(d_rot + kVec - 1) & ~(uint32_t)(kVec - 1);
+    r.wave_floats = positions * 2 * r.row;
+    if (r.wave_floats > 2048) return false;  // 32 KiB a block: heads of few bytes per position touch many positions
+    if constexpr (std::is_same<CS, Angles>::value) {
+        if (a.half % 8 == 0) {
+            *err = launch_rope_run<T, CS, 8, BWD>(r, a.nt, st);
+            return true;
+        }
+    }
+    if (a.half % 4 == 0) *err = launch_rope_run<T, CS, 4, BWD>(r, a.nt, st);
+    else *err = launch_rope_run<T, CS, 2, BWD>(r, a.nt, st);
+    return true;
+}
+
 // the rotated span, with the slots stored as loaded behind it, is at most 64 slots of w >= 2 dims:
 // the contiguous-span kernel applies (a pass-through copy must be covered by those slots)
 static bool span_shape(const RopeArgs& a, int w) {
@@ -139,6 +206,9 @@ static hipError_t launch_rope_w(const RopeArgs& a, int s, int n_outer, int w, hi
 template <typename T, typename CS>
 static hipError_t launch_rope_dir(const RopeArgs& a, int s, int n_outer, int w, bool backward,
                                   hipStream_t st) {
+    hipError_t err = hipSuccess;
+    if (backward ? try_launch_rope_run<T, CS, true>(a, s, n_outer, st, &err)
+                 : try_launch_rope_run<T, CS, false>(a, s, n_outer, st, &err)) return err;
     return backward ? launch_rope_w<T, CS, true>(a, s, n_outer, w, st)
                     : launch_rope_w<T, CS, false>(a, s, n_outer, w, st);
 }

@@ -3,7 +3,8 @@
 // s/b/h strides (the inputs are usually views into a fused QKV buffer).
 //
 // One block serves one sequence position: the position's cos/sin values are loaded
-// once into registers and reused for every head of q and k.  Two kernels:
+// once into registers and reused for every head of q and k.  Two kernels (two more, for dense
+// tensors that are taken as one run of memory, are described where they stand):
 //
 // * rope_span_kernel -- the rotated span splits into at most 64 slots of W = 8, 4 or 2 dims
 //   (the widest the alignment of the layouts and of d_rot/2 allows).  Each lane owns ONE
@@ -508,6 +509,149 @@ __global__ __launch_bounds__(256) void rope_piece_kernel(RopeArgs a) {
             }
             buf_st_words<W>(make_rsrc(a.t[t].out + base[u], (t == 0 || a.nt > 1) ? bytes[u] : 0u), lane_off, ow);
         }
+    }
+}
+
+// ---- dense heads out of place, in 4 KiB pieces ---------------------------------------------
+// Whole heads of dense tensors ([s, b, h, d], in and out), taken as one run of 16-byte slots however the
+// rotated span divides: a wave owns one 4 KiB piece of the run, four accesses of 1 KiB, whatever the head
+// size, so that no lane idles (in rope_span_kernel a head of 24 8-byte slots leaves 16 of 64 lanes without
+// work) and every XCD can keep to its own pieces.  A lane fetches the partners of its 8 dims a second time,
+// from the lines its wave has just asked for (PW dims per access: the widest the half span allows), and
+// pass-through dims fetch no partner.  The cos and the signed sin values of the few positions a piece
+// touches are laid out in LDS by the wave itself while its loads are in flight -- sin already at the dim it
+// multiplies --, so that there is no barrier.  Bound by memory: [2048,2,64,96] fp16, first 24 dims, angles,
+// 27.7 us (3.6 TB/s) in rope_span_kernel, which also evaluated its block's angles before it asked for the first
+// head, -> 19.0 us (5.3 TB/s); the rule with the other shapes is at try_launch_rope_run.
+struct RopeRunArgs {
+    const char* in[2];
+    char* out[2];
+    uint32_t slots[2];     // 16-byte slots of the tensor, below 2^31
+    FastDiv by_vpp[2];     // division by the head vectors of one position
+    FastDiv by_spv;        // division by the slots of one head vector
+    FastDiv by_rot;        // division by d_rot
+    const char* cos;
+    const char* sin;
+    int64_t cs_stride;
+    int32_t pos_offset;
+    int32_t half;
+    uint32_t row;          // LDS floats of one position's cos (or sin) values: d_rot rounded up to 8
+    uint32_t wave_floats;  // LDS floats of one wave
+};
+constexpr uint32_t kPieceSlots = 256;  // 16-byte slots of a 4 KiB piece
+
+template <typename T, typename CS, int PW, bool BWD>
+__global__ __launch_bounds__(256) void rope_run_kernel(RopeRunArgs a) {
+    extern __shared__ float lds_run[];
+    constexpr int ITERS = kPieceSlots / kWave;
+    const int t = blockIdx.y;
+    const int lane = threadIdx.x & (kWave - 1);
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t slots = a.slots[t];
+    const uint32_t pieces = (slots + kPieceSlots - 1) / kPieceSlots;
+    // the whole groups of 8 blocks deal their 32 pieces so that block x gets the pieces x (mod 8)
+    const uint32_t b = blockIdx.x;
+    const uint32_t piece = b < (pieces >> 5 << 3) ? (((b >> 3) * 4 + wave) << 3) + (b & 7u) : b * 4 + wave;
+    if (piece >= pieces) return;
+
+    const int half = a.half, d_rot = 2 * half;
+    const uint32_t spv = a.by_spv.d, vec_bytes = spv * 16;
+    const uint32_t slot0 = piece * kPieceSlots;
+    const uint32_t v0 = a.by_spv.div(slot0);                     // head vector the piece begins in
+    const uint32_t v1 = a.by_spv.div(min(slot0 + kPieceSlots, slots) - 1u);
+    const uint32_t pos0 = a.by_vpp[t].div(v0);
+    const uint32_t pos1 = a.by_vpp[t].div(v1);
+    const uint32_t r0 = v0 - pos0 * a.by_vpp[t].d;               // v0 inside its position
+    const uint32_t s0 = slot0 - v0 * spv;                        // slot0 inside v0
+    // everything is addressed from the start of v0; the resource ends with the tensor or with v1
+    const size_t base = (size_t)v0 * vec_bytes;
+    const uint32_t bytes = (v1 - v0 + 1) * vec_bytes;
+    const rsrc_t rx = make_rsrc(a.in[t] + base, bytes);
+    const rsrc_t ro = make_rsrc(a.out[t] + base, bytes);
+
+    // table values of the first 64 (position, dim) pairs, asked for before anything else
+    const int n = (int)(pos1 - pos0 + 1) * d_rot;
+    float* tab = lds_run + wave * a.wave_floats;
+    const uint32_t row = a.row;
+    float cv = 0.f, sv = 0.f;
+    auto table_load = [&](int idx) {
+        const uint32_t p = a.by_rot.div((uint32_t)idx);
+        const int64_t at = (int64_t)(pos0 + p + (uint32_t)a.pos_offset) * a.cs_stride + (idx - (int)p * d_rot);
+        if constexpr (std::is_same<CS, Angles>::value) {
+            cv = reinterpret_cast<const float*>(a.cos)[at];
+        } else if constexpr (sizeof(CS) == 4) {
+            cv = reinterpret_cast<const float*>(a.cos)[at];
+            sv = reinterpret_cast<const float*>(a.sin)[at];
+        } else {
+            cv = Elem<CS>::load1(a.cos + at * 2);
+            sv = Elem<CS>::load1(a.sin + at * 2);
+        }
+    };
+    if (lane < n) table_load(lane);
+
+    u32x4 x[ITERS];
+    uint32_t xp[ITERS][4];
+    int j[ITERS];  // first dim of the lane's slot
+    uint32_t tv[ITERS];
+#pragma unroll
+    for (int it = 0; it < ITERS; ++it) {
+        const uint32_t rel = s0 + it * kWave + lane;  // slot counted from v0
+        const uint32_t v = min(a.by_spv.div(rel), v1 - v0);  // (behind the tensor's end: any vector of the piece)
+        j[it] = (int)(rel - v * spv) * kVec;
+        tv[it] = a.by_vpp[t].div(r0 + v) * (2 * row);
+        x[it] = buf_ld128<true>(rx, rel * 16, 0);
+#pragma unroll
+        for (int g = 0; g < kVec / PW; ++g) {
+            const int e = j[it] + g * PW;
+            const uint32_t off = e < d_rot ? v * vec_bytes + (uint32_t)(e < half ? e + half : e - half) * 2u : kNoAccess;
+            if constexpr (PW == 8) {
+                const u32x4 w = buf_ld128<false>(rx, off, 0);
+                xp[it][0] = w.x, xp[it][1] = w.y, xp[it][2] = w.z, xp[it][3] = w.w;
+            } else if constexpr (PW == 4) {
+                const u32x2 w = buf_ld64(rx, off, 0);
+                xp[it][2 * g] = w.x, xp[it][2 * g + 1] = w.y;
+            } else {
+                xp[it][g] = buf_ld32(rx, off);
+            }
+        }
+    }
+
+    for (int idx = lane; idx < n; idx += kWave) {
+        if (idx >= kWave) table_load(idx);
+        if constexpr (std::is_same<CS, Angles>::value) sincosf(cv, &sv, &cv);
+        const uint32_t p = a.by_rot.div((uint32_t)idx);
+        const int e = idx - (int)p * d_rot;
+        float* at = tab + p * (2 * row);
+        at[e] = cv;
+        // the sign belongs to the first half of the result forward, to the second half backward
+        if constexpr (!BWD) at[row + e] = e < half ? -sv : sv;
+        else if (e < half) at[row + e + half] = -sv;
+        else at[row + e - half] = sv;
+    }
+    // the wave's own LDS accesses are carried out in order; the compiler must keep them in order too
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+
+#pragma unroll
+    for (int it = 0; it < ITERS; ++it) {
+        const float* at = tab + tv[it] + (j[it] < d_rot ? j[it] : 0);
+        float xf[8], pf[8], c[8], sn[8], o[8];
+        load_table<float, 8>(reinterpret_cast<const char*>(at), 0, c);
+        load_table<float, 8>(reinterpret_cast<const char*>(at), row, sn);
+        unpack8<T>(x[it], xf);
+        unpack8<T>(u32x4{xp[it][0], xp[it][1], xp[it][2], xp[it][3]}, pf);
+        {
+#pragma clang fp contract(off)
+#pragma unroll
+            for (int k = 0; k < 8; ++k) o[k] = xf[k] * c[k] + pf[k] * sn[k];
+        }
+        const u32x4 r = pack8<T>(o);
+        u32x4 w;  // d_rot is even: a dword is rotated or passed through as a whole
+        w.x = j[it] < d_rot ? r.x : x[it].x;
+        w.y = j[it] + 2 < d_rot ? r.y : x[it].y;
+        w.z = j[it] + 4 < d_rot ? r.z : x[it].z;
+        w.w = j[it] + 6 < d_rot ? r.w : x[it].w;
+        buf_st128<true>(ro, w, (s0 + it * kWave + lane) * 16, 0);
     }
 }
 

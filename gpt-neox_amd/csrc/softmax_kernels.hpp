@@ -24,25 +24,6 @@
 
 namespace neox {
 
-// Division by a number the launch fixes: floor(n / d) == (mulhi(2 n, mul) >> shift) for every n below
-// 2^31, with mul = ceil(2^(31 + shift) / d) and shift = ceil(log2 d): the error of mul, below d <= 2^shift,
-// times n < 2^31 stays below 2^(31 + shift).  Three scalar or vector instructions; the compiler's own
-// 32-bit division is a chain of some twenty with a reciprocal in it, which the kernels used to go through
-// once or twice before their first load, and per row where a mask row is looked up: fp16, us per launch before
-// and after, mask-tensor forward [4000,129,129] 67.3 -> 62.3, causal forward [4000,129,129] 54.3 -> 52.3,
-// [500,577,577] 106.7 -> 104.5, [600,512,512] 79.8 -> 78.5, [48,2048,2048] bf16 94.6 -> 93.2; elsewhere within 1 %.
-struct FastDiv {
-    uint32_t d, mul, shift;
-    __host__ static FastDiv by(uint32_t d) {
-        FastDiv f{d, 0, 0};
-        while (f.shift < 31 && (1u << f.shift) < d) ++f.shift;
-        f.mul = (uint32_t)((((uint64_t)1 << (31 + f.shift)) + d - 1) / d);
-        return f;
-    }
-    __device__ __forceinline__ uint32_t div(uint32_t n) const { return __umulhi(n << 1, mul) >> shift; }
-    __device__ __forceinline__ uint32_t mod(uint32_t n) const { return n - div(n) * d; }
-};
-
 struct SoftmaxArgs {
     void* out;            // y (forward) or dx (backward)
     const void* in0;      // x (forward) or dy (backward)

@@ -222,3 +222,37 @@ def test_angles_for_q_and_k_in_one_launch(device, dtype):
     rot = q.float()[..., :d2]
     pair = (rot[..., : d2 // 2] ** 2 + rot[..., d2 // 2 :] ** 2).sqrt()  # a rotation mixes the two dims of a pair
     assert ((q1.float()[..., :d2] - rot).abs() <= 3 * ULP[dtype] * torch.cat((pair, pair), -1) + 1e-6).all()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("shape,d2", [
+    ((300, 1, 1, 16), 4),      # a 4 KiB piece holds 128 positions; partners two dims at a time
+    ((65, 1, 1, 8), 8),        # one slot per head, one position per head; a piece of 65 slots
+    ((33, 2, 5, 64), 16),      # heads that tile a piece; a last piece of 80 slots
+    ((43, 1, 3, 96), 24),      # heads that cross pieces; partners four dims at a time
+    ((128, 2, 8, 96), 24),     # whole groups of 32 pieces and none left over
+    ((129, 2, 8, 96), 48),     # ... and a last group of one piece and a half
+    ((90, 2, 20, 80), 20),     # partners two dims at a time, the last slot half rotated
+    ((31, 1, 9, 24), 12),      # the half span ends inside a slot
+    ((13, 2, 2, 256), 256),    # 512-byte heads, rotated whole
+])
+def test_dense_heads_in_pieces(device, dtype, shape, d2):
+    s, b, h, d = shape
+    check_both_variants(normal(shape, dtype, device, 41), d2, False, device)
+    # q and k of different head counts in one launch, between guard elements, from position 3 on
+    freqs = angles(s + 3, d2, device).view(s + 3, d2)
+    cos, sin = freqs.cos(), freqs.sin()
+    ins = [normal((s, b, n, d), dtype, device, 42 + n) for n in (h, h + 1)]
+    for tables, backward in (((cos, sin), False), ((freqs, None), False), ((cos, sin), True), ((freqs, None), True)):
+        bufs = [torch.full((t.numel() + 64,), 7.0, dtype=dtype, device=device) for t in ins]
+        outs = [buf[32:-32].view(t.shape) for buf, t in zip(bufs, ins)]
+        rope_ext.rope_launch(*outs, *ins, *tables, d2, 3, backward, d=d)
+        for buf, out, t in zip(bufs, outs, ins):
+            f = lambda x: x[3 : 3 + s].view(s, 1, 1, d2)
+            want = expected(t, t, f(cos), f(sin), d2)[1 if backward else 0]
+            if tables[1] is not None:
+                assert torch.equal(out, want)
+            else:
+                assert_within_one_ulp(out, want, dtype)
+            assert torch.equal(out[..., d2:], t[..., d2:])
+            assert (buf[:32] == 7).all() and (buf[-32:] == 7).all()
