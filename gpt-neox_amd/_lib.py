@@ -6,6 +6,8 @@ missing or cannot be loaded, :func:`lib` raises ``ImportError``; if a tensor is
 not on the GPU, the wrappers raise ``RuntimeError``.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import subprocess
 import threading
@@ -14,6 +16,7 @@ import torch
 
 _CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
 LIB_PATH = os.path.join(_CSRC, "libneox_fused.so")
+CALLS_PATH = os.path.join(_CSRC, "neox_torch.so")
 ABI_VERSION = 4
 
 NEOX_F16, NEOX_BF16, NEOX_F32 = 0, 1, 2
@@ -92,10 +95,13 @@ SIGNATURES = {
 
 _lock = threading.Lock()
 _lib = None
+_calls = None
+_PLAIN_TENSORS = (torch.Tensor, torch.nn.Parameter)
 
 
 def build(verbose=False, targets=("all",)):
-    """Compile ``libneox_fused.so`` for gfx950 with hipcc (works without a GPU).  ``targets``:
+    """Compile ``libneox_fused.so`` for gfx950 with hipcc and ``neox_torch.so`` against the installed torch
+    (works without a GPU).  ``targets``:
     make targets; ``"probes"`` is the benchmark's copy kernel, a library of its own."""
     cmd = ["make", "-C", _CSRC, "-j8", "-B", *targets]
     res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
@@ -135,6 +141,35 @@ def lib():
             raise ImportError(f"{LIB_PATH}: ABI version {got}, expected {ABI_VERSION}")
         _lib = handle
     return _lib
+
+
+def load_calls():
+    """Return the module of native calls, loading it on first use; ``ImportError`` if it is missing."""
+    global _calls
+    lib()  # the library behind them, with its checks
+    with _lock:
+        if _calls is None:
+            if not os.path.exists(CALLS_PATH):
+                raise ImportError(f"{CALLS_PATH} not found: run `make -C gpt-neox_amd/csrc` (or __graft_entry__.build()).")
+            loader = importlib.machinery.ExtensionFileLoader("neox_torch", CALLS_PATH)
+            module = importlib.util.module_from_spec(importlib.util.spec_from_loader("neox_torch", loader))
+            loader.exec_module(module)
+            _calls = module
+    return _calls
+
+
+def calls(*tensors):
+    """The native calls of ``csrc/torch_calls.cpp`` if they may serve a call on ``tensors``, else None: tensors
+    that are not on the GPU, tensor subclasses, and whatever records or rewrites Python operations (``torch.compile``, ``torch.jit.trace``),
+    keep the autograd Functions of the modules."""
+    if torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None:
+        return None
+    for t in tensors:
+        if type(t) not in _PLAIN_TENSORS:
+            return None
+    if not tensors[0].is_cuda:
+        return None
+    return _calls if _calls is not None else load_calls()
 
 
 def check(status):

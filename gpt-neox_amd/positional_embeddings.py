@@ -29,6 +29,7 @@ import math
 
 import torch
 
+from . import _lib
 from .fused_kernels import fused_rotary_positional_embedding as _rope_ext
 
 _HALF = (torch.float16, torch.bfloat16)
@@ -218,6 +219,11 @@ def apply_rotary_pos_emb(q, k, cos, sin, offset: int = 0):
     """``(q*cos + rotate_half(q)*sin, k*cos + rotate_half(k)*sin)`` with cos/sin rows
     ``offset .. offset+sq`` (megatron/model/positional_embeddings.py:110-116).
     q, k: ``[sq, b, heads, d_rot]``; cos, sin: ``[seq, 1, 1, d_rot]``."""
+    calls = _lib.calls(q, k, cos, sin)
+    if calls is not None and type(offset) is int and 0 <= offset < 2**31:
+        out = calls.rotary(q, k, cos, sin, offset)
+        if out is not None:
+            return out
     if _fusable(q, k, cos, sin):
         if not _needs_grad(q, k):
             return _rotary_out_of_place(q, k, _on(cos, q.device), _on(sin, q.device), offset)[:2]
