@@ -4,7 +4,8 @@
 // wave that holds 2 chunks (1024 columns) is the sweet spot at every row length -- 4 chunks
 // per wave cost 3-5 % of bandwidth, 1 chunk per wave 10-20 % -- so a row gets
 // ceil(chunks / 2) waves:
-//   chunks == 1    several rows per wave (packed kernels)            (sk <= 512)
+//   chunks == 1    several rows per wave (packed kernels; causal rows that leave much of their lane group
+//                  idle: with as many lanes as the rows see keys)    (sk <= 512)
 //   chunks <= 4    full-row backward only: packed kernel, one wave per row, R x C = 4
 //   chunks == 2    1 wave per row, 4 rows per 256-thread block      (sk <= 1024)
 //   chunks <= 4    2 waves per row, 2 rows per block (4 rows at 4 chunks: 2-3 % faster in an
@@ -100,15 +101,38 @@ static hipError_t launch_packed_shape(const SoftmaxArgs& a0, hipStream_t st) {
     return hipGetLastError();
 }
 
+// causal rows that leave much of their group of GMAX lanes idle: see softmax_fwd_causal_packed_kernel
+template <typename T, bool BWD, int EXTRA, int GMAX>
+static hipError_t launch_causal_packed(const SoftmaxArgs& a0, hipStream_t st) {
+    typedef Packed<GMAX, kPackedPasses> P;
+    const dim3 grid((a0.rows + P::kRowsPerBlock - 1) / P::kRowsPerBlock);
+    const SoftmaxArgs a = with_xcd_mapping(a0, (uint64_t)P::kRowsPerWave * a0.sk * 2, 4, grid.x);
+    constexpr int FLAGS = kDefaultFlags | EXTRA;
+    if constexpr (BWD) hipLaunchKernelGGL((softmax_bwd_causal_packed_kernel<T, GMAX, FLAGS>), grid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((softmax_fwd_causal_packed_kernel<T, GMAX, FLAGS>), grid, dim3(256), 0, st, a);
+    return hipGetLastError();
+}
+
 template <typename T, Mask M, bool BWD, int EXTRA, int G>
 static hipError_t launch_packed(const SoftmaxArgs& a, hipStream_t st) {
+    const int lanes = (a.sk + kVec - 1) / kVec;
+    if constexpr (M == Mask::Causal && G >= 16 && (!BWD || (EXTRA & kDropout) != 0)) {
+        // Causal rows that fill less than three quarters of their lane group: as many lanes as the rows see keys,
+        // results staged.  us per launch, bf16, against the kernels below: [2000,161,161] 36.9 -> 34.3, [2000,177,177]
+        // 42.4 -> 40.4, [800,336,336] 55.6 -> 50.8, [4000,80,80] 19.3 -> 19.0; fuller rows lose: [2000,192,192] 42.2 -> 42.9,
+        // [2000,193,193] 46.0 -> 49.7, [400,511,511] 61 -> 69, and so does the plain backward pass at most lengths ([4000,129,129]
+        // 65.7 -> 66.6, [600,384,384] 66.7 -> 68.0).  With dropout, whose Philox rounds the idle lanes computed too, it pays in
+        // both passes up to seven eighths, and to the end of 128 columns (fp16, forward and backward: [600,385,385]
+        // 128 -> 105 and 112 -> 85, [4000,127,127] 84.5 -> 71.5 and 69.8 -> 65.3; [1000,224,224] 47.3 -> 48.3 and 41.8 -> 43.2).
+        const bool pays = (EXTRA & kDropout) != 0 ? (lanes * 8 < G * 7 || (G == 16 && a.sk != G * kVec)) : lanes * 4 < G * 3;
+        if (pays) return launch_causal_packed<T, BWD, EXTRA, G>(a, st);
+    }
     // passes per wave: 4, except for lane groups of 32 and 64 lanes in the causal kernels and the
     // full-row backward, which run faster with 2 when the rows fill their lane groups (causal forward
     // 15 %, causal backward up to 11 % at 512 columns, full-row backward 0-4 %).  With a quarter or
     // more of the lanes idle (129-192 and 257-384 columns) 4 passes are 4-12 % faster there too.
     constexpr int R = (M != Mask::Bytes && G >= 32) ? 2 : kPackedPasses;
     if constexpr (R != kPackedPasses) {
-        const int lanes = (a.sk + kVec - 1) / kVec;
         if (lanes * 4 <= G * 3) return launch_packed_shape<T, M, BWD, EXTRA, G, kPackedPasses, 1>(a, st);
     }
     return launch_packed_shape<T, M, BWD, EXTRA, G, R, 1>(a, st);

@@ -750,18 +750,59 @@ struct Packed {
     static constexpr int kRowsPerBlock = kRowsPerWave * 4;  // 256-thread blocks
 };
 
-template <typename T, int G, Mask MASK, int FLAGS = kDefaultFlags, int R = kPackedPasses, int C = 1>
-__global__ __launch_bounds__(256) void softmax_fwd_packed_kernel(SoftmaxArgs a) {
+// Where a wave's results go.  Direct: one 128-bit store per lane and pass, to the lane's columns.  Staged: into
+// LDS at the place they have in memory, from where flush_staged stores the wave's rows -- one run of memory --
+// in whole 1 KiB accesses: where a row's columns are stored by several accesses that share cache lines, the memory
+// system takes them at 60-80 % of its rate.
+struct DirectSink {
+    rsrc_t out;
+    template <bool NT>
+    __device__ __forceinline__ void put(const u32x4& v, uint32_t off, bool active) const {
+        packed_st<NT>(out, v, off, active);
+    }
+};
+struct __attribute__((packed, aligned(2))) Slot16 { u32x4 v; };  // 16 bytes at the alignment of an element
+struct StagedSink {
+    char* lds;
+    template <bool NT>
+    __device__ __forceinline__ void put(const u32x4& v, uint32_t off, bool active) const {
+        if (active) reinterpret_cast<Slot16*>(lds + off)->v = v;
+    }
+};
+constexpr int kStageBytes = kPackedPasses * kChunk * 2;  // of one wave: its passes, every lane with 8 columns
+
+__device__ __forceinline__ void clear_stage(char* lds, uint32_t n, int lane) {
+    for (uint32_t e = lane * kVec; e < n; e += kChunk) *reinterpret_cast<u32x4*>(lds + e * 2) = u32x4{0, 0, 0, 0};
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+// the n staged elements of a wave to `out`; only the tensor's last wave can have n % 8 != 0
+template <bool NT>
+__device__ __forceinline__ void flush_staged(rsrc_t out, const char* lds, uint32_t n, int lane) {
+    // a wave's LDS accesses are carried out in order: no barrier, but the compiler must keep that order
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const uint32_t whole = n & ~(uint32_t)(kVec - 1);
+#pragma unroll
+    for (uint32_t e0 = 0; e0 < kStageBytes / 2; e0 += kChunk) {
+        const uint32_t e = e0 + lane * kVec;
+        if (e0 < whole) buf_st128<NT>(out, *reinterpret_cast<const u32x4*>(lds + e * 2), e < whole ? e * 2 : kNoAccess, 0);
+    }
+    if (whole != n) buf_st16(out, *reinterpret_cast<const uint16_t*>(lds + (whole + lane) % (kStageBytes / 2) * 2),
+                             lane < (int)(n - whole) ? (whole + lane) * 2 : kNoAccess);
+}
+
+// The rows row0 .. row0 + rows_here - 1 of one wave.  Causal rows may be given fewer lanes than they have
+// columns for (G * 8 < sk), as long as no row sees a key behind them: see softmax_fwd_causal_packed_kernel.
+// Returns whether every row has a sum (scores that are NaN or infinite leave none, and no probability in the row).
+template <typename T, int G, Mask MASK, int FLAGS, int R, int C, typename Sink>
+__device__ __forceinline__ bool softmax_fwd_rows(const SoftmaxArgs& a, uint32_t row0, uint32_t rows_here, int lane,
+                                                 const Sink& out, const Sink& out2) {
     static_assert(C == 1 || G == kWave, "several chunks per row need a whole wave per row");
-    constexpr int RPP = Packed<G, R>::kRowsPerPass, RPW = Packed<G, R>::kRowsPerWave;
+    constexpr int RPP = Packed<G, R>::kRowsPerPass;
     constexpr bool kLdNt = (FLAGS & kNtLoad) != 0, kStNt = (FLAGS & kNtStore) != 0;
     constexpr bool kRag = (FLAGS & kRagged) != 0;
     static_assert(!kRag || C == 1, "ragged rows: one chunk per lane group");
-    const int lane = threadIdx.x & (kWave - 1);
-    const uint32_t wave = xcd_slot(blockIdx.x, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), 4, a);
-    const uint32_t row0 = wave * RPW;  // first row of this wave
-    if (row0 >= a.rows) return;
-    const uint32_t rows_here = min((uint32_t)RPW, a.rows - row0);
     const int sk = a.sk;
     const int grp = lane / G;
     const int back = ragged_back<kRag>((lane % G) * kVec, sk);  // kRagged: see ragged_back
@@ -771,14 +812,10 @@ __global__ __launch_bounds__(256) void softmax_fwd_packed_kernel(SoftmaxArgs a) 
     const float ninf = -__builtin_inff();
 
     const rsrc_t rx = make_rsrc(static_cast<const char*>(a.in0) + (size_t)row0 * sk * 2, rows_here * sk * 2);
-    const rsrc_t ry = make_rsrc(static_cast<char*>(a.out) + (size_t)row0 * sk * 2, rows_here * sk * 2);
     const rsrc_t rm = make_rsrc(a.mask, a.mask_bytes);
-    rsrc_t ry2 = ry;
-    if constexpr ((FLAGS & kDropout) != 0) {
-        ry2 = make_rsrc(static_cast<char*>(a.out2) + (size_t)row0 * sk * 2, rows_here * sk * 2);
-    }
     const rsrc_t rb = make_rsrc(a.bias, a.bias_bytes);  // kBias: the whole bias tensor
 
+    bool summed = true;
     u32x4 raw[R][C];
     u32x4 rawb[R][C];
     u32x2 mk[R][C];
@@ -882,6 +919,7 @@ __global__ __launch_bounds__(256) void softmax_fwd_packed_kernel(SoftmaxArgs a) 
         sum = group_reduce<OpSum, G>(sum);
         const float inv = 1.0f / sum;
         const uint32_t lr = p * RPP + grp;
+        summed = summed && (lr >= rows_here || sum == sum);
 #pragma unroll
         for (int c = 0; c < C; ++c) {
             const int col = col0 + c * kChunk;
@@ -889,27 +927,102 @@ __global__ __launch_bounds__(256) void softmax_fwd_packed_kernel(SoftmaxArgs a) 
             for (int k = 0; k < 8; ++k) v[c][k] *= inv;  // lanes of absent rows hold NaN and store nothing
             const bool st = lr < rows_here && col < sk;
             const u32x4 o = pack8<T>(v[c]);
-            packed_st<kStNt>(ry, o, (lr * sk + col) * 2u, st);
+            out.template put<kStNt>(o, (lr * sk + col) * 2u, st);
             if constexpr ((FLAGS & kDropout) != 0) {
                 const uint32_t bits = keep_bits_row8<kRag>(drop, row0 + lr, sk, col);
-                packed_st<kStNt>(ry2, dropout8<T>(o, bits, drop.scale), (lr * sk + col) * 2u, st);
+                out2.template put<kStNt>(dropout8<T>(o, bits, drop.scale), (lr * sk + col) * 2u, st);
             }
         }
     }
+    return __builtin_amdgcn_ballot_w64(!summed) == 0;
+}
+
+// The two outputs of a wave's rows, as resources
+template <int FLAGS>
+__device__ __forceinline__ void wave_outputs(const SoftmaxArgs& a, uint32_t row0, uint32_t rows_here, rsrc_t& y, rsrc_t& y2) {
+    const size_t at = (size_t)row0 * a.sk * 2;
+    y = y2 = make_rsrc(static_cast<char*>(a.out) + at, rows_here * a.sk * 2);
+    if constexpr ((FLAGS & kDropout) != 0) y2 = make_rsrc(static_cast<char*>(a.out2) + at, rows_here * a.sk * 2);
 }
 
 template <typename T, int G, Mask MASK, int FLAGS = kDefaultFlags, int R = kPackedPasses, int C = 1>
-__global__ __launch_bounds__(256) void softmax_bwd_packed_kernel(SoftmaxArgs a) {
+__global__ __launch_bounds__(256) void softmax_fwd_packed_kernel(SoftmaxArgs a) {
+    constexpr int RPW = Packed<G, R>::kRowsPerWave;
+    const uint32_t wave = xcd_slot(blockIdx.x, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), 4, a);
+    const uint32_t row0 = wave * RPW;  // first row of this wave
+    if (row0 >= a.rows) return;
+    const uint32_t rows_here = min((uint32_t)RPW, a.rows - row0);
+    rsrc_t ry, ry2;
+    wave_outputs<FLAGS>(a, row0, rows_here, ry, ry2);
+    softmax_fwd_rows<T, G, MASK, FLAGS, R, C>(a, row0, rows_here, threadIdx.x & (kWave - 1), DirectSink{ry}, DirectSink{ry2});
+}
+
+// The number of leading keys that any of the causal rows row0 .. row0 + rows_here - 1 sees.
+__device__ __forceinline__ int keys_seen(uint32_t row0, uint32_t rows_here, const SoftmaxArgs& a) {
+    const uint32_t last = a.by_sq.mod(row0) + rows_here;  // beyond sq: the matrix ends inside the wave's rows
+    return (int)min(min(last, (uint32_t)a.sq), (uint32_t)a.sk);
+}
+
+// fn(lanes per row) for the fewest lanes, of 8, 16, 32 and GMAX, that `seen` keys need
+template <int GMAX, typename Fn>
+__device__ __forceinline__ auto with_lanes_for(int seen, const Fn& fn) {
+    if constexpr (GMAX > 8) {
+        if (seen <= 8 * kVec) return fn(std::integral_constant<int, 8>{});
+    }
+    if constexpr (GMAX > 16) {
+        if (seen <= 16 * kVec) return fn(std::integral_constant<int, 16>{});
+    }
+    if constexpr (GMAX > 32) {
+        if (seen <= 32 * kVec) return fn(std::integral_constant<int, 32>{});
+    }
+    return fn(std::integral_constant<int, GMAX>{});
+}
+
+// Causal rows of 65 .. 512 columns that leave much of their lane group idle: a wave owns the rows of four passes
+// and gives them only as many lanes as the keys they see need, chosen once for the wave, so that it makes one or
+// two passes where it made four; the zeros behind those lanes are there before the results are staged.  The
+// omitted lanes held zeros and -inf only: every sum has the same terms in the same order, the same bits.  Bound
+// by the vector units and by partly written cache lines before, by latency and memory now; us per launch,
+// softmax_fwd_packed_kernel -> this, fp16 [384,129,129] 8.1 -> 6.5, [4000,129,129] 51.9 -> 45.7, with dropout
+// [2000,129,129] 69.2 -> 49.3 and 65.5 -> 38.7 backward; bf16 [1200,257,257] 63.6 -> 51.6, [800,320,320]
+// 51.9 -> 44.9.  Few lanes without the staging lose (129: 51.9 -> 70.6): the zeros and the results of a row are
+// then parts of the same lines stored by different accesses.
+template <typename T, int GMAX, int FLAGS>
+__global__ __launch_bounds__(256) void softmax_fwd_causal_packed_kernel(SoftmaxArgs a) {
+    constexpr uint32_t RW = Packed<GMAX, kPackedPasses>::kRowsPerWave;
+    constexpr bool kStNt = (FLAGS & kNtStore) != 0, kDrp = (FLAGS & kDropout) != 0;
+    __shared__ __attribute__((aligned(16))) char stage[4 * (kDrp ? 2 : 1)][kStageBytes];
+    const int lane = threadIdx.x & (kWave - 1);
+    const uint32_t wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t row0 = xcd_slot(blockIdx.x, wib, 4, a) * RW;
+    if (row0 >= a.rows) return;
+    const uint32_t rows_here = min(RW, a.rows - row0), n = rows_here * a.sk;
+    const StagedSink s1{stage[wib]}, s2{stage[kDrp ? 4 + wib : wib]};
+    auto with_lanes = [&](auto g) {
+        constexpr int G = decltype(g)::value;
+        if constexpr (G < GMAX) {
+            clear_stage(s1.lds, n, lane);
+            if constexpr (kDrp) clear_stage(s2.lds, n, lane);
+        }
+        return softmax_fwd_rows<T, G, Mask::Causal, FLAGS, kPackedPasses * G / GMAX + (G * kPackedPasses < GMAX), 1>(
+            a, row0, rows_here, lane, s1, s2);
+    };
+    // a row without a sum is NaN in its hidden columns too: all lanes, once more (nothing is stored yet)
+    if (!with_lanes_for<GMAX>(keys_seen(row0, rows_here, a), with_lanes)) with_lanes(std::integral_constant<int, GMAX>{});
+    rsrc_t ry, ry2;
+    wave_outputs<FLAGS>(a, row0, rows_here, ry, ry2);
+    flush_staged<kStNt>(ry, s1.lds, n, lane);
+    if constexpr (kDrp) flush_staged<kStNt>(ry2, s2.lds, n, lane);
+}
+
+template <typename T, int G, Mask MASK, int FLAGS, int R, int C, typename Sink>
+__device__ __forceinline__ void softmax_bwd_rows(const SoftmaxArgs& a, uint32_t row0, uint32_t rows_here, int lane,
+                                                 const Sink& out) {
     static_assert(C == 1 || G == kWave, "several chunks per row need a whole wave per row");
-    constexpr int RPP = Packed<G, R>::kRowsPerPass, RPW = Packed<G, R>::kRowsPerWave;
+    constexpr int RPP = Packed<G, R>::kRowsPerPass;
     constexpr bool kLdNt = (FLAGS & kNtLoad) != 0, kStNt = (FLAGS & kNtStore) != 0;
     constexpr bool kRag = (FLAGS & kRagged) != 0;
     static_assert(!kRag || C == 1, "ragged rows: one chunk per lane group");
-    const int lane = threadIdx.x & (kWave - 1);
-    const uint32_t wave = xcd_slot(blockIdx.x, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), 4, a);
-    const uint32_t row0 = wave * RPW;
-    if (row0 >= a.rows) return;
-    const uint32_t rows_here = min((uint32_t)RPW, a.rows - row0);
     const int sk = a.sk;
     const int grp = lane / G;
     const int back = ragged_back<kRag>((lane % G) * kVec, sk);  // kRagged: see ragged_back
@@ -919,7 +1032,6 @@ __global__ __launch_bounds__(256) void softmax_bwd_packed_kernel(SoftmaxArgs a) 
 
     const rsrc_t bg = make_rsrc(static_cast<const char*>(a.in0) + (size_t)row0 * sk * 2, rows_here * sk * 2);
     const rsrc_t by = make_rsrc(static_cast<const char*>(a.in1) + (size_t)row0 * sk * 2, rows_here * sk * 2);
-    const rsrc_t bo = make_rsrc(static_cast<char*>(a.out) + (size_t)row0 * sk * 2, rows_here * sk * 2);
 
     u32x4 rg[R][C], rp[R][C];
     int len[R];
@@ -998,9 +1110,43 @@ __global__ __launch_bounds__(256) void softmax_bwd_packed_kernel(SoftmaxArgs a) 
                 if ((col + k) >= len[p]) gv[k] = 0.f;
             }
             const bool st = lr < rows_here && col < sk;
-            packed_st<kStNt>(bo, pack8<T>(gv), (lr * sk + col) * 2u, st);
+            out.template put<kStNt>(pack8<T>(gv), (lr * sk + col) * 2u, st);
         }
     }
+}
+
+template <typename T, int G, Mask MASK, int FLAGS = kDefaultFlags, int R = kPackedPasses, int C = 1>
+__global__ __launch_bounds__(256) void softmax_bwd_packed_kernel(SoftmaxArgs a) {
+    constexpr int RPW = Packed<G, R>::kRowsPerWave;
+    const uint32_t wave = xcd_slot(blockIdx.x, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), 4, a);
+    const uint32_t row0 = wave * RPW;
+    if (row0 >= a.rows) return;
+    const uint32_t rows_here = min((uint32_t)RPW, a.rows - row0);
+    rsrc_t dx, dx2;
+    wave_outputs<0>(a, row0, rows_here, dx, dx2);
+    softmax_bwd_rows<T, G, MASK, FLAGS, R, C>(a, row0, rows_here, threadIdx.x & (kWave - 1), DirectSink{dx});
+}
+
+// The backward pass of softmax_fwd_causal_packed_kernel, with dropout.  (dx may alias dy: a wave's rows are read before they are stored.)
+template <typename T, int GMAX, int FLAGS>
+__global__ __launch_bounds__(256) void softmax_bwd_causal_packed_kernel(SoftmaxArgs a) {
+    constexpr uint32_t RW = Packed<GMAX, kPackedPasses>::kRowsPerWave;
+    __shared__ __attribute__((aligned(16))) char stage[4][kStageBytes];
+    const int lane = threadIdx.x & (kWave - 1);
+    const uint32_t wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t row0 = xcd_slot(blockIdx.x, wib, 4, a) * RW;
+    if (row0 >= a.rows) return;
+    const uint32_t rows_here = min(RW, a.rows - row0), n = rows_here * a.sk;
+    const StagedSink s{stage[wib]};
+    with_lanes_for<GMAX>(keys_seen(row0, rows_here, a), [&](auto g) {
+        constexpr int G = decltype(g)::value;
+        if constexpr (G < GMAX) clear_stage(s.lds, n, lane);
+        softmax_bwd_rows<T, G, Mask::Causal, FLAGS, kPackedPasses * G / GMAX + (G * kPackedPasses < GMAX), 1>(
+            a, row0, rows_here, lane, s);
+    });
+    rsrc_t dx, dx2;
+    wave_outputs<0>(a, row0, rows_here, dx, dx2);
+    flush_staged<(FLAGS & kNtStore) != 0>(dx, s.lds, n, lane);
 }
 
 // ---------------------------------------------------------------------------------

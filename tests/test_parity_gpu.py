@@ -1532,3 +1532,34 @@ def test_mask_and_bias_tensors_beyond_4_gib(device):
     assert torch.equal(probs[0, 0, rows], y[0, 0, rows])
     keep = rng.keep_mask(probs.numel(), 0.25, 3, 4, device).view(probs.shape)
     assert torch.equal(dropped[0, 0, rows], R.dropout_with_mask(probs[0, 0, rows], keep[0, 0, rows], 0.25))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("s", [65, 88, 96, 127, 129, 136, 191, 193, 223, 257, 264, 300, 383, 385, 447])
+def test_causal_rows_with_as_many_lanes_as_they_see_keys(device, dtype, s):
+    # causal lengths around the limits of the kernel that chooses its lanes by the keys a wave's rows see:
+    # square, wide and tall matrices, waves that hold the end of one and the start of the next, a last wave
+    # of one row.  Outputs pre-filled with 7: every element must have been written, and none around them.
+    lib, code = _lib.lib(), _lib.dtype_code(dtype)
+    stream = torch.cuda.current_stream().cuda_stream
+    for batches, sq in ((5, s), (1, s - 3), (3, s + 9), (67, 3), (1, 1)):
+        x, g = scores((batches, sq, s), dtype, device, s), normal((batches, sq, s), dtype, device, s + 1)
+        hidden = torch.ones(sq, s, dtype=torch.bool, device=device).triu_(1)
+        bufs = [torch.full((x.numel() + 64,), 7.0, dtype=dtype, device=device) for _ in range(4)]
+        y, y1, y2, dx = (t[32:-32].view(x.shape) for t in bufs)
+        _lib.check(lib.neox_causal_softmax_fwd(y.data_ptr(), x.data_ptr(), 0.125, batches, sq, s, code, stream))
+        assert max_err(y, R.softmax_fp32(x, hidden, 0.125)) <= TOL[dtype] and (y[:, hidden] == 0).all()
+        _lib.check(lib.neox_causal_softmax_dropout_fwd(y2.data_ptr(), y1.data_ptr(), x.data_ptr(), None, None, 0, 0.125,
+                                                       0.25, 77, 8, None, batches, 1, sq, s, code, stream))
+        keep = rng_keep(y.numel(), 0.25, 77, 8, device).view(y.shape)
+        assert torch.equal(y1, y) and torch.equal(y2, R.dropout_with_mask(y, keep, 0.25))
+        _lib.check(lib.neox_causal_softmax_dropout_bwd(dx.data_ptr(), g.data_ptr(), y.data_ptr(), 0.125, 0.25, 77, 8, None,
+                                                       batches, sq, s, code, stream))
+        want = R.softmax_backward_fp32(g.float() * keep / 0.75, y, 0.125)
+        assert max_err(dx, want) <= TOL[dtype] * max(1.0, want.float().abs().max().item()) and (dx[:, hidden] == 0).all()
+        assert all((t[:32] == 7).all() and (t[-32:] == 7).all() for t in bufs)
+        # a row with a score that is not a number has no probabilities, and no other row notices
+        x2 = x.clone()
+        x2[0, sq // 2, 0] = float("nan")
+        _lib.check(lib.neox_causal_softmax_fwd(dx.data_ptr(), x2.data_ptr(), 0.125, batches, sq, s, code, stream))
+        assert dx[0, sq // 2].isnan().all() and dx.isnan().sum() == s
