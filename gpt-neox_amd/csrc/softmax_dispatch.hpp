@@ -23,7 +23,8 @@
 //                  blocks per CU (sk <= 40448), or in all of it       (sk <= 81408)
 //   ragged rows    (sk % 8 != 0 or pointers not 16-byte aligned; 8 <= sk < 81408)
 //                  the same packed, one- to sixteen-wave row and LDS-staged kernels with the kRagged flag
-//   sliding window (kBand) the one- to sixteen-wave row kernels, aligned rows of 513-32768 columns
+//   sliding window (kBand) the one- to sixteen-wave row kernels, aligned rows of 513-32768 columns, by the
+//                  chunks the band can touch
 //   anything else  element-wise kernels (rows shorter than 8 columns or beyond 81408)
 #pragma once
 
@@ -41,10 +42,11 @@ namespace neox {
 
 // Switches the XCD-aware block -> unit mapping on (see xcd_slot) when the work units of a block
 // -- `units` of them, `unit_bytes` each, consecutive in memory -- tile 4 KiB pieces exactly and
-// the output starts on a 4 KiB boundary.
+// the output starts on a 4 KiB boundary; and for rows of two pieces, several per block.
 static SoftmaxArgs with_xcd_mapping(const SoftmaxArgs& a, uint64_t unit_bytes, uint32_t units, uint32_t blocks) {
     SoftmaxArgs b = a;
     b.piece_shift = 0;
+    b.group_shift = 3;
     b.affine_blocks = 0;
     const bool aligned = (reinterpret_cast<uintptr_t>(a.out) & 4095u) == 0 &&
                          (a.out2 == nullptr || (reinterpret_cast<uintptr_t>(a.out2) & 4095u) == 0);
@@ -55,6 +57,14 @@ static SoftmaxArgs with_xcd_mapping(const SoftmaxArgs& a, uint64_t unit_bytes, u
             b.affine_blocks = blocks & ~7u;
         }
     }
+    // Units of two pieces, several per block: blocks 4 apart run on XCDs that share two pieces in eight, and a
+    // block takes every fourth unit of its group's run (sliding window over 4096 columns, [32,4096,4096]
+    // window 1024, forward 226 -> 206 us, backward 274 -> 247).  Units of four pieces gain nothing that
+    // way ([8,8192,8192] window 1024: 220 -> 220 and 241 -> 254).
+    if (aligned && unit_bytes == 8192 && units > 1) {
+        b.group_shift = 2;
+        b.affine_blocks = blocks & ~3u;
+    }
     return b;
 }
 
@@ -62,7 +72,9 @@ template <typename T, Mask M, bool BWD, int EXTRA, int NCH, int WPR, int RPB>
 static hipError_t launch_shape(const SoftmaxArgs& a0, hipStream_t st) {
     const dim3 grid((a0.rows + RPB - 1) / RPB);
     const dim3 block(kWave * WPR * RPB);
-    const SoftmaxArgs a = with_xcd_mapping(a0, (uint64_t)a0.sk * 2, RPB, grid.x);
+    // (one wave per row of two pieces: the order costs 2-5 %, sliding window of 256 over 4096 columns)
+    const uint64_t unit_bytes = (uint64_t)a0.sk * 2;
+    const SoftmaxArgs a = with_xcd_mapping(a0, WPR == 1 && unit_bytes > 4096 ? 0 : unit_bytes, RPB, grid.x);
     constexpr int FLAGS = kDefaultFlags | EXTRA;
     if constexpr (BWD) {
         hipLaunchKernelGGL((softmax_bwd_kernel<T, NCH, WPR, RPB, M, FLAGS>), grid, block, 0, st, a);
@@ -265,6 +277,12 @@ static hipError_t dispatch_rows(const SoftmaxArgs& a, bool vec_ok, hipStream_t s
     // (the aligned full-row backward has taken 2 to 4 chunks with its packed kernel above)
     if constexpr (!(BWD && M == Mask::None && (EXTRA & kRagged) == 0)) {
         if (chunks == 2) return launch_shape<T, M, BWD, EXTRA, 2, 1, 4>(a, st);
+        if constexpr ((EXTRA & kBand) != 0) {
+            // rows that are mostly zeros in front of and behind the band: twice the waves, one chunk of the band
+            // each ([8,8192,8192] window 1024: 220 -> 207 us forward, 241 -> 236 backward; [20,5000,5000] window 1250:
+            // 252 -> 236 and 294 -> 274; 3000 columns +2 and -3 %)
+            if (a.sk > 4096 && (chunks == 3 || chunks == 4)) return launch_shape<T, M, BWD, EXTRA, 1, 4, 1>(a, st);
+        }
         if (chunks == 3) return launch_shape<T, M, BWD, EXTRA, 2, 2, 2>(a, st);
         if (chunks == 4) {
             // the causal forward with two output streams (dropout) measured 3 % faster with 2 rows
@@ -289,6 +307,11 @@ static hipError_t dispatch_rows(const SoftmaxArgs& a, bool vec_ok, hipStream_t s
         // which up to half would hold nothing (-13 % at 8200 columns, -8 % at 10240, -4 % at 12288).  The
         // same step at the shorter ranges and for the full-row backward measured -3...+5 %: not taken.
         if (chunks > 16 && chunks <= 24) return launch_shape<T, M, BWD, EXTRA, 3, 8, 1>(a, st);
+    }
+    if constexpr ((EXTRA & kBand) != 0) {
+        // rows of two 4 KiB pieces: two per block, in the order of with_xcd_mapping ([32,4096,4096] window 2048:
+        // 248 -> 234 us forward, 317 -> 311 backward; at 8192 columns, which that order does not serve, 230 -> 254)
+        if (chunks <= 6 && a.sk == 4096) return launch_shape<T, M, BWD, EXTRA, 3, 2, 2>(a, st);
     }
     if (chunks <= 8) return launch_shape<T, M, BWD, EXTRA, 2, 4, 1>(a, st);
     if (chunks <= 16) return launch_shape<T, M, BWD, EXTRA, 2, 8, 1>(a, st);

@@ -47,7 +47,8 @@ struct SoftmaxArgs {
     // Block -> memory mapping that keeps every XCD on its own 4 KiB pieces (see xcd_slot), filled in
     // by the launchers: log2 of the work units (rows, or the rows of a wave) per 4 KiB piece
     uint32_t piece_shift;
-    uint32_t affine_blocks;        // leading blocks that take part: a multiple of 8; 0 = units in order
+    uint32_t group_shift;          // log2 of the blocks that share a run of units: 8, fewer for units of several pieces
+    uint32_t affine_blocks;        // leading blocks that take part: whole groups; 0 = units in order
     int32_t window;                // kBand kernels: row i sees the keys max(0, i - window) .. i
     // Mask-tensor forward and full-row backward, optional: per mask row [mask_b * sq], the number of
     // leading keys that can be visible -- the caller's promise that the mask hides every key from
@@ -228,14 +229,15 @@ __device__ __forceinline__ uint32_t keep_bits_row8(const DropoutArgs& d, uint32_
 // several consecutive pieces or the pieces rotate over the XCDs (loads do not care).  So where the
 // units of a block (U of them: rows, or the row groups of its waves) tile 4 KiB pieces exactly,
 // 2^piece_shift units per piece, the blocks of a group of 8 share the 8 * U units of the group like this:
-// block x of the group takes the pieces x, x + 8, x + 16, ... instead of consecutive ones.
+// block x of the group takes the pieces x, x + 8, x + 16, ... instead of consecutive ones.  Units of two pieces
+// each go the same way in groups of 4 blocks (group_shift 2): an XCD then keeps to two pieces in eight.
 // Returns the unit index for unit l of block b; the identity for the last, incomplete group.
 __device__ __forceinline__ uint32_t xcd_slot(uint32_t b, uint32_t l, uint32_t U, const SoftmaxArgs& a) {
     if (b >= a.affine_blocks) return b * U + l;
-    const uint32_t sh = a.piece_shift;
-    const uint32_t g = b >> 3, x = b & 7u;
+    const uint32_t sh = a.piece_shift, gs = a.group_shift;
+    const uint32_t g = b >> gs, x = b & ((1u << gs) - 1u);
     const uint32_t j = l >> sh, t = l & ((1u << sh) - 1u);  // piece of the block, unit inside the piece
-    return ((((g * (U >> sh)) + j) * 8u + x) << sh) + t;
+    return (((((g * (U >> sh)) + j) << gs) + x) << sh) + t;
 }
 
 // Where a wave works: the row, its position i inside its [sq, sk] matrix, the number of

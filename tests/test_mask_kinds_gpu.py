@@ -131,6 +131,15 @@ def test_sliding_window_sizes(device, s, w, dtype):
     check_window(device, 3 if s <= 2056 else 1, s, w, dtype, 0.125, seed=s + w)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+# rows of two 4 KiB pieces, several per block and out of order, with bands of two to seven chunks; longer rows
+# with a band of three or four chunks, one per wave
+@pytest.mark.parametrize("s,w", [(4096, 300), (4096, 512), (4096, 1023), (4096, 1535), (4096, 2048), (4096, 2600),
+                                 (4104, 600), (5000, 1250), (8192, 512), (8192, 1535), (16384, 1024)])
+def test_sliding_window_order_and_shapes(device, s, w, dtype):
+    check_window(device, 2 if s <= 4104 else 1, s, w, dtype, 0.125, seed=s + w)
+
+
 # (the kernel shape goes by the chunks a band can touch, w / 512 + 2, capped by the row's: narrow windows on long
 # rows take few waves per row, the last three cases the 16-wave shapes with 2, 3 and 4 chunks per wave)
 @pytest.mark.parametrize("s,w", [(10240, 4096), (12288, 511), (13312, 4096), (16384, 8192), (20000, 4096), (28672, 1000), (32768, 4096),
