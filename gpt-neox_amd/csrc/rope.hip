@@ -115,8 +115,8 @@ static bool try_launch_rope_piece(const RopeArgs& a, int s, int n_outer, hipStre
 template <typename T, typename CS, int PW, bool BWD>
 static hipError_t launch_rope_run(const RopeRunArgs& r, int nt, hipStream_t st) {
     const uint32_t slots = nt > 1 && r.slots[1] > r.slots[0] ? r.slots[1] : r.slots[0];
-    const uint32_t pieces = (slots + kPieceSlots - 1) / kPieceSlots;
-    hipLaunchKernelGGL((rope_run_kernel<T, CS, PW, BWD>), dim3((pieces + 3) / 4, nt), dim3(256),
+    const uint32_t units = (slots + kRunSlots - 1) / kRunSlots;
+    hipLaunchKernelGGL((rope_run_kernel<T, CS, PW, BWD>), dim3((units + 3) / 4, nt), dim3(256),
                        4 * r.wave_floats * sizeof(float), st, r);
     return hipGetLastError();
 }
@@ -130,9 +130,9 @@ static bool try_launch_rope_run(const RopeArgs& a, int s, int n_outer, hipStream
     // Angles: always faster than rope_span_kernel, which alone takes them otherwise.  Tables: where the half span
     // is no multiple of 8 dims the other kernels move 8 or 4 bytes per access; where it is, or where the whole head
     // rotates, rope_piece_kernel reads nothing twice.  us per launch, fp16, that kernel or rope_span_kernel -> this:
-    // [2048,2,64,96] d_rot 24 angles 27.7 -> 19.0, tables 25.9 -> 19.3; [2048,2,40,80] d_rot 20 angles 28.6 -> 13.1,
-    // tables 24.5 -> 13.1, d_rot 40 angles 15.4 -> 13.2; angles [2048,2,64,128] d_rot 32 24.9 -> 23.4, d_rot = d = 96
-    // 20.5 -> 20.3; against it: tables [2048,2,64,128] d_rot 32 23.3 -> 23.7, d_rot = d = 128 13.3 -> 14.6,
+    // [2048,2,64,96] d_rot 24 angles 27.7 -> 18.6, tables 25.9 -> 18.9; [2048,2,40,80] d_rot 20 angles 28.6 -> 12.1,
+    // tables 24.5 -> 12.2, d_rot 40 angles 15.4 -> 12.3; angles [2048,2,64,128] d_rot 32 24.9 -> 23.3, d_rot = d = 96
+    // 20.5 -> 20.1; against it: tables [2048,2,64,128] d_rot 32 23.3 -> 23.7, d_rot = d = 128 13.3 -> 14.6,
     // d_rot = d = 40 18.3 -> 19.1 (bf16, q and k).
     if (!std::is_same<CS, Angles>::value && (a.half % kVec == 0 || a.copy_dims == 0)) return false;
     RopeRunArgs r{};
@@ -151,7 +151,7 @@ static bool try_launch_rope_run(const RopeArgs& a, int s, int n_outer, hipStream
         r.in[i] = t.in, r.out[i] = t.out;
         r.slots[i] = (uint32_t)slots;
         r.by_vpp[i] = FastDiv::by((uint32_t)t.n_inner);
-        const uint32_t vecs = (kPieceSlots - 2) / spv + 2;  // head vectors that 256 slots in a row can touch
+        const uint32_t vecs = (kRunSlots - 2) / spv + 2;  // head vectors that the slots of a wave can touch
         const uint32_t p = (vecs - 2 + (uint32_t)t.n_inner) / (uint32_t)t.n_inner + 1;
         if (p > positions) positions = p;
     }

@@ -514,7 +514,7 @@ __global__ __launch_bounds__(256) void rope_piece_kernel(RopeArgs a) {
 
 // ---- dense heads out of place, in 4 KiB pieces ---------------------------------------------
 // Whole heads of dense tensors ([s, b, h, d], in and out), taken as one run of 16-byte slots however the
-// rotated span divides: a wave owns one 4 KiB piece of the run, four accesses of 1 KiB, whatever the head
+// rotated span divides: a wave owns half a 4 KiB piece of the run, two accesses of 1 KiB, whatever the head
 // size, so that no lane idles (in rope_span_kernel a head of 24 8-byte slots leaves 16 of 64 lanes without
 // work) and every XCD can keep to its own pieces.  A lane fetches the partners of its 8 dims a second time,
 // from the lines its wave has just asked for (PW dims per access: the widest the half span allows), and
@@ -522,7 +522,9 @@ __global__ __launch_bounds__(256) void rope_piece_kernel(RopeArgs a) {
 // touches are laid out in LDS by the wave itself while its loads are in flight -- sin already at the dim it
 // multiplies --, so that there is no barrier.  Bound by memory: [2048,2,64,96] fp16, first 24 dims, angles,
 // 27.7 us (3.6 TB/s) in rope_span_kernel, which also evaluated its block's angles before it asked for the first
-// head, -> 19.0 us (5.3 TB/s); the rule with the other shapes is at try_launch_rope_run.
+// head, -> 18.6 us (5.4 TB/s).  A whole piece per wave leaves too few waves for an even last round: 19.0 us, and
+// [4096,1,4,64] first 64 dims 5.5 against 4.0; a quarter 19.7.  Partners fetched with the non-temporal hint come
+// from memory once more where a head spans parts of lines: 19.9.  The rule with the other shapes is at try_launch_rope_run.
 struct RopeRunArgs {
     const char* in[2];
     char* out[2];
@@ -539,26 +541,30 @@ struct RopeRunArgs {
     uint32_t wave_floats;  // LDS floats of one wave
 };
 constexpr uint32_t kPieceSlots = 256;  // 16-byte slots of a 4 KiB piece
+constexpr uint32_t kRunSlots = 128;    // ... of a wave
 
 template <typename T, typename CS, int PW, bool BWD>
 __global__ __launch_bounds__(256) void rope_run_kernel(RopeRunArgs a) {
     extern __shared__ float lds_run[];
-    constexpr int ITERS = kPieceSlots / kWave;
+    constexpr int ITERS = kRunSlots / kWave;
     const int t = blockIdx.y;
     const int lane = threadIdx.x & (kWave - 1);
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t slots = a.slots[t];
-    const uint32_t pieces = (slots + kPieceSlots - 1) / kPieceSlots;
-    // the whole groups of 8 blocks deal their 32 pieces so that block x gets the pieces x (mod 8)
+    const uint32_t units = (slots + kRunSlots - 1) / kRunSlots;
+    // the whole groups of 8 blocks deal their pieces so that block x gets the pieces x (mod 8)
     const uint32_t b = blockIdx.x;
-    const uint32_t piece = b < (pieces >> 5 << 3) ? (((b >> 3) * 4 + wave) << 3) + (b & 7u) : b * 4 + wave;
-    if (piece >= pieces) return;
+    constexpr uint32_t upp = kPieceSlots / kRunSlots;
+    const uint32_t unit = b < (units >> 5 << 3)
+                              ? ((((b >> 3) * (4 / upp) + wave / upp) << 3) + (b & 7u)) * upp + wave % upp
+                              : b * 4 + wave;
+    if (unit >= units) return;
 
     const int half = a.half, d_rot = 2 * half;
     const uint32_t spv = a.by_spv.d, vec_bytes = spv * 16;
-    const uint32_t slot0 = piece * kPieceSlots;
+    const uint32_t slot0 = unit * kRunSlots;
     const uint32_t v0 = a.by_spv.div(slot0);                     // head vector the piece begins in
-    const uint32_t v1 = a.by_spv.div(min(slot0 + kPieceSlots, slots) - 1u);
+    const uint32_t v1 = a.by_spv.div(min(slot0 + kRunSlots, slots) - 1u);
     const uint32_t pos0 = a.by_vpp[t].div(v0);
     const uint32_t pos1 = a.by_vpp[t].div(v1);
     const uint32_t r0 = v0 - pos0 * a.by_vpp[t].d;               // v0 inside its position
