@@ -179,6 +179,41 @@ static bool try_launch_rope_run(const RopeArgs& a, int s, int n_outer, hipStream
     return true;
 }
 
+// q and k in place in a fused projection whose parts tile 4 KiB pieces: the cell kernel (see rope_cell_kernel).
+// Returns false if the call does not qualify.
+template <typename T, typename CS, bool BWD>
+static bool try_launch_rope_cell(const RopeArgs& a, int s, int n_outer, int w, hipStream_t st, hipError_t* err) {
+    if (std::is_same<CS, Angles>::value || n_outer != 1 || a.nt != 2 || w != kVec || a.copy_dims != 0) return false;
+    const RopeTensor &q = a.t[0], &k = a.t[1];
+    const int64_t cell = q.in_stride[2], hn = cell / 3;
+    // Parts of one cache line, or of two that are rotated whole: the lanes of this kernel pass over what does not
+    // move.  us per launch, rope_span_kernel -> this: bf16 [8192,1,32,3*128] d_rot 128 52.5 -> 47.1, [2048,4,32,3*128]
+    // 53.3 -> 45.7, fp16 [2048,4,16,3*64] d_rot 64 14.7 -> 13.5, d_rot 16 12.8 -> 11.9; against it: bf16 [8192,1,32,3*128]
+    // d_rot 64 27.4 -> 35.6, fp16 [2048,2,16,3*256] d_rot 256 25.1 -> 25.7, d_rot 64 9.7 -> 16.9.
+    const bool pays = hn == 64 || (hn == 128 && a.half == 64);
+    if (cell % 3 != 0 || !pays || k.in != q.in + hn * 2 || k.n_inner != q.n_inner) return false;
+    for (const RopeTensor* t : {&q, &k}) {
+        if (t->in != t->out || t->in_stride[2] != cell || t->out_stride[2] != cell) return false;
+        if (t->in_stride[0] != t->n_inner * cell || t->out_stride[0] != t->in_stride[0]) return false;
+    }
+    const int64_t per_pos = q.n_inner * cell / kVec;
+    if (reinterpret_cast<uintptr_t>(q.in) % 4096 != 0 || per_pos % kRunSlots != 0 || per_pos * s > 0x7fffffffLL) return false;
+    if ((a.lpv * 2 + a.pad_slots) * kVec > hn) return false;
+    RopeCellArgs r{};
+    r.mixed = q.out;
+    r.cos = a.cos, r.sin = a.sin;
+    r.cs_stride = a.cs_stride;
+    r.pos_offset = a.pos_offset;
+    r.slots = (uint32_t)(per_pos * s);
+    r.by_pos = FastDiv::by((uint32_t)per_pos);
+    r.by_part = FastDiv::by((uint32_t)(hn / kVec));
+    r.lps = a.lpv * 2;
+    r.moved = a.lpv * 2 + a.pad_slots;
+    hipLaunchKernelGGL((rope_cell_kernel<T, CS, BWD>), dim3((r.slots / kRunSlots + 3) / 4), dim3(256), 0, st, r);
+    *err = hipGetLastError();
+    return true;
+}
+
 // the rotated span, with the slots stored as loaded behind it, is at most 64 slots of w >= 2 dims:
 // the contiguous-span kernel applies (a pass-through copy must be covered by those slots)
 static bool span_shape(const RopeArgs& a, int w) {
@@ -209,6 +244,10 @@ static hipError_t launch_rope_dir(const RopeArgs& a, int s, int n_outer, int w, 
     hipError_t err = hipSuccess;
     if (backward ? try_launch_rope_run<T, CS, true>(a, s, n_outer, st, &err)
                  : try_launch_rope_run<T, CS, false>(a, s, n_outer, st, &err)) return err;
+    if constexpr (!std::is_same<CS, Angles>::value) {
+        if (backward ? try_launch_rope_cell<T, CS, true>(a, s, n_outer, w, st, &err)
+                     : try_launch_rope_cell<T, CS, false>(a, s, n_outer, w, st, &err)) return err;
+    }
     return backward ? launch_rope_w<T, CS, true>(a, s, n_outer, w, st)
                     : launch_rope_w<T, CS, false>(a, s, n_outer, w, st);
 }

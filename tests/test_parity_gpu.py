@@ -1563,3 +1563,41 @@ def test_causal_rows_with_as_many_lanes_as_they_see_keys(device, dtype, s):
         x2[0, sq // 2, 0] = float("nan")
         _lib.check(lib.neox_causal_softmax_fwd(dx.data_ptr(), x2.data_ptr(), 0.125, batches, sq, s, code, stream))
         assert dx[0, sq // 2].isnan().all() and dx.isnan().sum() == s
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("half_tables", [False, True])
+@pytest.mark.parametrize("s,b,h,hn,d_rot", [
+    (1, 1, 16, 128, 128),   # three pieces
+    (11, 1, 16, 128, 128),  # one whole group of 32 half pieces, a last one of two
+    (33, 2, 8, 128, 128),
+    (3, 1, 16, 64, 64),
+    (43, 2, 8, 64, 32),
+    (7, 4, 12, 64, 16),     # 32-byte spans, stored with the rest of their 64 bytes
+    (5, 1, 5, 128, 128),    # positions that are no whole number of half pieces
+    (9, 1, 16, 128, 64),    # half of every part: the general kernel
+])
+def test_rotary_in_place_on_pieces_of_a_fused_projection(device, s, b, h, hn, d_rot, half_tables, dtype):
+    angles = torch.randn(s + 2, 1, 1, d_rot, device=device, generator=gen(device, s))
+    cos, sin = (t.to(dtype) if half_tables else t for t in (angles.cos(), angles.sin()))
+    rows = slice(2, 2 + s)
+    before = normal((s, b, h, 3 * hn), dtype, device, 3 + s)
+    q, k = before[..., :d_rot], before[..., hn : hn + d_rot]
+    fwd = R.partial_rotary(q.float(), k.float(), cos[rows].float(), sin[rows].float(), d_rot)
+    bwd = R.rotary_autograd_fp32(q, k, cos[rows].float(), sin[rows].float(), q, k)
+    for backward, (wq, wk) in ((False, fwd), (True, bwd)):
+        want = before.clone()
+        want[..., :d_rot], want[..., hn : hn + d_rot] = wq.to(dtype), wk.to(dtype)
+        # on a 4 KiB boundary, between guard elements
+        buf = torch.full((before.numel() + 8192,), 7.0, dtype=dtype, device=device)
+        at = 2048 - buf.data_ptr() % 4096 // 2
+        mixed = buf[at : at + before.numel()].view(before.shape)
+        assert mixed.data_ptr() % 4096 == 0
+        mixed.copy_(before)
+        if backward:
+            dq, dk = mixed[..., :hn], mixed[..., hn : 2 * hn]
+            rope_ext.rope_launch(dq, dk, dq, dk, cos.view(s + 2, d_rot), sin.view(s + 2, d_rot), d_rot, 2, True)
+        else:
+            apply_rotary_pos_emb_qkv_(mixed, cos, sin, offset=2, rotary_ndims=d_rot)
+        assert torch.equal(mixed, want)
+        assert (buf[:at] == 7).all() and (buf[at + before.numel() :] == 7).all()
