@@ -142,9 +142,11 @@ static hipError_t launch_packed(const SoftmaxArgs& a, hipStream_t st) {
     // passes per wave: 4, except for lane groups of 32 and 64 lanes in the causal kernels and the
     // full-row backward, which run faster with 2 when the rows fill their lane groups (causal forward
     // 15 %, causal backward up to 11 % at 512 columns, full-row backward 0-4 %).  With a quarter or
-    // more of the lanes idle (129-192 and 257-384 columns) 4 passes are 4-12 % faster there too.
+    // more of the lanes idle 4 passes are faster there too (full-row and causal backward passes at 129-192 and
+    // 257-384 columns; causal forward at the end of those ranges, whose fuller rows are all that is left to it).
     constexpr int R = (M != Mask::Bytes && G >= 32) ? 2 : kPackedPasses;
-    if constexpr (R != kPackedPasses) {
+    // (causal rows with dropout that leave so many idle have gone above)
+    if constexpr (R != kPackedPasses && !(M == Mask::Causal && (EXTRA & kDropout) != 0)) {
         if (lanes * 4 <= G * 3) return launch_packed_shape<T, M, BWD, EXTRA, G, kPackedPasses, 1>(a, st);
     }
     return launch_packed_shape<T, M, BWD, EXTRA, G, R, 1>(a, st);

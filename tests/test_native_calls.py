@@ -176,6 +176,28 @@ def test_saved_tensors_go_through_hooks_and_version_checks(device):
 
 
 @gpu
+def test_native_calls_run_on_the_current_stream(device):
+    x = torch.randn(2, 4, 200, 200, device=device).half()
+    mod, mask, dy = module(torch.float16, SoftmaxFusionTypes.upper_triang), causal_mask(200, device), torch.randn_like(x)
+    leaf = x.clone().requires_grad_(True)
+    want = mod(leaf, mask)
+    want_dx = torch.autograd.grad(want, leaf, dy.clone())[0]
+    late, late_dy = torch.zeros_like(x).requires_grad_(True), torch.zeros_like(dy)
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(20_000_000)  # the inputs arrive late, on this stream
+        with torch.no_grad():
+            late.copy_(x)
+        y = mod(late, mask)
+        torch.cuda._sleep(20_000_000)
+        late_dy.copy_(dy)
+        (dx,) = torch.autograd.grad(y, late, late_dy)
+    side.synchronize()
+    assert torch.equal(y, want) and torch.equal(dx, want_dx)
+
+
+@gpu
 def test_what_the_native_calls_leave_alone(device, monkeypatch):
     q = torch.randn(4, 1, 2, 16, device=device).half()
     cos, sin = torch.randn(2, 8, 1, 1, 16, device=device)

@@ -1601,3 +1601,45 @@ def test_rotary_in_place_on_pieces_of_a_fused_projection(device, s, b, h, hn, d_
             apply_rotary_pos_emb_qkv_(mixed, cos, sin, offset=2, rotary_ndims=d_rot)
         assert torch.equal(mixed, want)
         assert (buf[:at] == 7).all() and (buf[at + before.numel() :] == 7).all()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("slopes,with_bias,p", [(s, b, p) for s in (False, True) for b in (False, True) for p in (0.0, 0.25)])
+@pytest.mark.parametrize("s,shift", [(88, 0), (81, 0), (128, 1), (192, 0), (190, 0), (384, 0), (381, 0)])
+def test_short_causal_rows_on_both_sides_of_the_lane_rule(device, s, shift, slopes, with_bias, p, dtype):
+    # every feature set, at lengths below and above those that get their lanes by the keys they see, aligned
+    # and ragged (128 columns from an odd element on)
+    b, np_ = 2, 2
+    n = b * np_ * s * s
+
+    def place(t):
+        buf = torch.zeros(n + 8, dtype=dtype, device=device)
+        buf[shift : shift + n] = t.reshape(-1)
+        return buf[shift : shift + n].view(b, np_, s, s)
+
+    x = place(scores((b, np_, s, s), dtype, device, s))
+    bias = normal((1, np_, s, s), dtype, device, s + 1) if with_bias else None
+    sl = torch.tensor([0.25, 0.0625], device=device) if slopes else None
+    total = x.float()
+    if with_bias:
+        total = total + bias.float()
+    if slopes:
+        at = torch.arange(s, device=device)
+        total = total + sl.view(1, np_, 1, 1) * (at.view(1, 1, 1, s) - at.view(1, 1, s, 1)).float()
+    hidden = torch.ones(s, s, dtype=torch.bool, device=device).triu_(1)
+    want = R.softmax_fp32(total, hidden, 0.125)
+    if p:
+        y, dropped = causal_ext.forward_dropout(x, 0.125, p, 9, 4, slopes=sl, bias=bias)
+        keep = rng_keep(n, p, 9, 4, device).view(y.shape)
+        assert torch.equal(dropped, R.dropout_with_mask(y, keep, p))
+        g = place(normal((b, np_, s, s), dtype, device, s + 2))
+        want_dx = R.softmax_backward_fp32(g.float() * keep / (1 - p), y, 0.125)
+        dx = causal_ext.backward_dropout(g, y, 0.125, p, 9, 4)
+        assert max_err(dx, want_dx) <= TOL[dtype] * max(1.0, want_dx.float().abs().max().item()) and (dx[..., hidden] == 0).all()
+    elif with_bias:
+        y = causal_ext.forward_bias(x, bias, 0.125, sl)
+    elif slopes:
+        y = causal_ext.forward_alibi(x, sl, 0.125)
+    else:
+        y = causal_ext.forward_nd(x, 0.125)
+    assert max_err(y, want) <= TOL[dtype] and (y[..., hidden] == 0).all()
