@@ -293,17 +293,16 @@ std::optional<Tensor> rope(const Tensor& x, const Tensor& cos, const std::option
 
 }  // namespace
 
-// the interpreter is not held while a launch waits for room in its queue
+// The interpreter is not held while a launch waits for room in its queue.  An exception that a saved-tensor hook
+// raises (activation checkpointing ends its recomputation with one) comes back as what it is.
 PYBIND11_MODULE(neox_torch, m) {
     namespace py = pybind11;
-    m.def("causal_softmax", &causal_softmax, py::arg("x"), py::arg("scale"), py::arg("window") = -1,
-          py::arg("slopes") = std::optional<Tensor>(), py::arg("p") = 0.0, py::arg("seed") = 0, py::arg("offset") = 0,
-          py::call_guard<py::gil_scoped_release>());
-    m.def("causal_takes", &causal_takes, py::arg("x"), py::arg("slopes") = std::optional<Tensor>());
-    m.def("masked_softmax", &masked_softmax, py::arg("x"), py::arg("mask"), py::arg("scale"),
-          py::call_guard<py::gil_scoped_release>());
-    m.def("rotary", &rotary, py::arg("q"), py::arg("k"), py::arg("cos"), py::arg("sin"), py::arg("offset"),
-          py::call_guard<py::gil_scoped_release>());
-    m.def("rope", &rope, py::arg("x"), py::arg("cos"), py::arg("sin"), py::arg("transposed"),
-          py::call_guard<py::gil_scoped_release>());
+    using torch::wrap_pybind_function_no_gil;
+    m.def("causal_softmax", wrap_pybind_function_no_gil(causal_softmax), py::arg("x"), py::arg("scale"), py::arg("window") = -1,
+          py::arg("slopes") = std::optional<Tensor>(), py::arg("p") = 0.0, py::arg("seed") = 0, py::arg("offset") = 0);
+    m.def("causal_takes", wrap_pybind_function_no_gil(causal_takes), py::arg("x"), py::arg("slopes") = std::optional<Tensor>());
+    m.def("masked_softmax", wrap_pybind_function_no_gil(masked_softmax), py::arg("x"), py::arg("mask"), py::arg("scale"));
+    m.def("rotary", wrap_pybind_function_no_gil(rotary), py::arg("q"), py::arg("k"), py::arg("cos"), py::arg("sin"),
+          py::arg("offset"));
+    m.def("rope", wrap_pybind_function_no_gil(rope), py::arg("x"), py::arg("cos"), py::arg("sin"), py::arg("transposed"));
 }

@@ -3,6 +3,7 @@
 every form the native calls take; what they leave alone goes, and fails, the general way."""
 import pytest
 import torch
+import torch.utils.checkpoint
 
 from gpt_neox_amd import _lib, fused_rope
 from gpt_neox_amd.fused_softmax import FusedScaleMaskSoftmax, SoftmaxFusionTypes
@@ -173,6 +174,32 @@ def test_saved_tensors_go_through_hooks_and_version_checks(device):
     torch.autograd.grad(y, x, dy.clone())
     with pytest.raises(RuntimeError, match="second time"):
         torch.autograd.grad(y, x, dy.clone())
+
+
+@gpu
+def test_exceptions_of_saved_tensor_hooks_and_activation_checkpointing(device):
+    x = torch.randn(1, 2, 40, 40, device=device).half().requires_grad_(True)
+    mod, mask = module(torch.float16, SoftmaxFusionTypes.upper_triang), causal_mask(40, device)
+    q = torch.randn(4, 1, 2, 16, device=device).half().requires_grad_(True)
+    cos, sin = torch.randn(2, 8, 1, 1, 16, device=device)
+    freqs = torch.randn(4, 1, 1, 16, device=device)
+
+    class Stop(Exception):
+        pass
+
+    def stop(t):
+        raise Stop
+
+    calls = (lambda: mod(x, mask), lambda: apply_rotary_pos_emb(q, q, cos, sin)[0],
+             lambda: fused_rope.fused_apply_rotary_pos_emb(q, freqs))
+    for call in calls:
+        with pytest.raises(Stop), torch.autograd.graph.saved_tensors_hooks(stop, lambda t: t):
+            call()
+    # recomputed segments stop, by an exception from the pack hook, at the last tensor that is saved: in this call
+    for leaf, call in zip((x, q, q), calls):
+        want = torch.autograd.grad(call().float().pow(2).sum(), leaf)[0]
+        y = torch.utils.checkpoint.checkpoint(lambda _: call(), leaf, use_reentrant=False)
+        assert torch.equal(torch.autograd.grad(y.float().pow(2).sum(), leaf)[0], want)
 
 
 @gpu
