@@ -10,7 +10,7 @@
 //   chunks == 2    1 wave per row, 4 rows per 256-thread block      (sk <= 1024)
 //   chunks <= 4    2 waves per row, 2 rows per block (4 rows at 4 chunks: 2-3 % faster in an
 //                  interleaved comparison; at 3 chunks 2 rows are)   (sk <= 2048)
-//   chunks <= 8    4 waves per row                                   (sk <= 4096)
+//   chunks <= 8    4 waves per row (causal rows of 7 or 8 chunks: 2 rows per block)  (sk <= 4096)
 //   chunks <= 16   8 waves per row, 512-thread block                 (sk <= 8192)
 //   chunks <= 32   16 waves per row, 1024-thread block               (sk <= 16384)
 //                  forward, in the lower 3/4 of each of these three ranges (7/8 of the last):
@@ -314,6 +314,13 @@ static hipError_t dispatch_rows(const SoftmaxArgs& a, bool vec_ok, hipStream_t s
         // rows of two 4 KiB pieces: two per block, in the order of with_xcd_mapping ([32,4096,4096] window 2048:
         // 248 -> 234 us forward, 317 -> 311 backward; at 8192 columns, which that order does not serve, 230 -> 254)
         if (chunks <= 6 && a.sk == 4096) return launch_shape<T, M, BWD, EXTRA, 3, 2, 2>(a, st);
+    }
+    if constexpr (M == Mask::Causal && (EXTRA & kBand) == 0 && !(BWD && (EXTRA & kDropout) != 0)) {
+        // Causal rows of 3585-4096 columns: two per block, at 4096 columns in the order of with_xcd_mapping.  us per launch
+        // forward / backward, one row per block -> two: bf16 [32,4096,4096] 265 -> 254 / 346 -> 340, fp16 [32,4000,4000]
+        // 284 -> 265 / 375 -> 354, bf16 [32,3999,3999] 276 -> 275 / 377 -> 360, with dropout [16,4096,4096] 228 -> 217 /
+        // 174 -> 175, [16,3840,3840] 202 -> 200 / 156 -> 161: the dropout backward stays.  Four chunks per wave: 1-2 % behind.
+        if (chunks == 7 || chunks == 8) return launch_shape<T, M, BWD, EXTRA, 2, 4, 2>(a, st);
     }
     if (chunks <= 8) return launch_shape<T, M, BWD, EXTRA, 2, 4, 1>(a, st);
     if (chunks <= 16) return launch_shape<T, M, BWD, EXTRA, 2, 8, 1>(a, st);

@@ -415,7 +415,8 @@ def test_xcd_aware_block_order_covers_every_row_once(device, sk):
 
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("batches,sq,sk", [(3, 4096, 4096), (2, 8192, 8192), (5, 100, 4096), (2, 5000, 6144),
-                                           (1, 9000, 8192), (3, 2052, 16384), (7, 8, 8192)])
+                                           (1, 9000, 8192), (3, 2052, 16384), (7, 8, 8192),
+                                           (3, 33, 4096), (1, 3601, 3600), (1, 3999, 4001)])  # (an odd last row)
 def test_long_causal_rows_store_every_piece_exactly_once(device, dtype, batches, sq, sk):
     # rows of several KiB, most of them zeros above the diagonal, in matrices that are square, wide
     # and tall.  Outputs pre-filled with NaN: every element must have been written, the zeros
