@@ -315,14 +315,17 @@ static hipError_t dispatch_rows(const SoftmaxArgs& a, bool vec_ok, hipStream_t s
         // 248 -> 234 us forward, 317 -> 311 backward; at 8192 columns, which that order does not serve, 230 -> 254)
         if (chunks <= 6 && a.sk == 4096) return launch_shape<T, M, BWD, EXTRA, 3, 2, 2>(a, st);
     }
-    if constexpr (M == Mask::Causal && (EXTRA & kBand) == 0 && !(BWD && (EXTRA & kDropout) != 0)) {
+    constexpr bool two_rows = M == Mask::Causal && (EXTRA & kBand) == 0 && !(BWD && (EXTRA & kDropout) != 0);
+    if constexpr (two_rows) {
         // Causal rows of 3585-4096 columns: two per block, at 4096 columns in the order of with_xcd_mapping.  us per launch
         // forward / backward, one row per block -> two: bf16 [32,4096,4096] 265 -> 254 / 346 -> 340, fp16 [32,4000,4000]
         // 284 -> 265 / 375 -> 354, bf16 [32,3999,3999] 276 -> 275 / 377 -> 360, with dropout [16,4096,4096] 228 -> 217 /
         // 174 -> 175, [16,3840,3840] 202 -> 200 / 156 -> 161: the dropout backward stays.  Four chunks per wave: 1-2 % behind.
         if (chunks == 7 || chunks == 8) return launch_shape<T, M, BWD, EXTRA, 2, 4, 2>(a, st);
     }
-    if (chunks <= 8) return launch_shape<T, M, BWD, EXTRA, 2, 4, 1>(a, st);
+    if constexpr (!two_rows || BWD) {  // (the causal forward has taken all of them above)
+        if (chunks <= 8) return launch_shape<T, M, BWD, EXTRA, 2, 4, 1>(a, st);
+    }
     if (chunks <= 16) return launch_shape<T, M, BWD, EXTRA, 2, 8, 1>(a, st);
     if (chunks <= 32) return launch_shape<T, M, BWD, EXTRA, 2, 16, 1>(a, st);
     if (chunks <= 48) return launch_shape<T, M, BWD, EXTRA, 3, 16, 1>(a, st);
