@@ -13,6 +13,7 @@ import subprocess
 import threading
 
 import torch
+from torch.autograd import forward_ad
 
 _CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
 LIB_PATH = os.path.join(_CSRC, "libneox_fused.so")
@@ -170,6 +171,12 @@ def calls(*tensors):
     if not tensors[0].is_cuda:
         return None
     return _calls if _calls is not None else load_calls()
+
+
+def carries_tangent(*tensors):
+    """Whether one of ``tensors`` is a dual tensor of forward-mode differentiation.  The kernels compute no
+    tangents, so such a call goes to an autograd Function, which refuses it, and not past it."""
+    return any(forward_ad.unpack_dual(t).tangent is not None for t in tensors)
 
 
 def check(status):

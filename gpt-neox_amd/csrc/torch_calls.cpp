@@ -44,6 +44,9 @@ bool fits_int32(int64_t n) { return n >= 0 && n <= INT32_MAX; }
 bool records(const Tensor& t) { return at::GradMode::is_enabled() && t.requires_grad(); }
 // a tensor whose memory this code may look at
 bool on_gpu(const Tensor& t) { return t.defined() && t.is_cuda() && t.layout() == at::kStrided && !t.is_neg() && !t.is_conj(); }
+// ... and that a call may be served for: one with a forward-mode tangent goes to the Python autograd Functions,
+// which refuse it (a result computed here would have lost the tangent)
+bool plain(const Tensor& t) { return on_gpu(t) && !t._fw_grad(/*level=*/0).defined(); }
 
 // ---- softmax ---------------------------------------------------------------------------------------
 enum Kind : int64_t { kCausal = -1, kMasked = -2 };  // a window width otherwise
@@ -129,7 +132,7 @@ public:
 };
 
 bool plain_scores(const Tensor& x) {
-    return on_gpu(x) && half_type(x) && x.dim() == 4 && x.numel() > 0 && x.is_contiguous() && fits_int32(x.size(0)) &&
+    return plain(x) && half_type(x) && x.dim() == 4 && x.numel() > 0 && x.is_contiguous() && fits_int32(x.size(0)) &&
            fits_int32(x.size(1)) && fits_int32(x.size(2)) && fits_int32(x.size(3));
 }
 
@@ -141,7 +144,7 @@ Tensor run_softmax(const Tensor& x, const SoftmaxCall& c) {
 
 // whether causal_softmax serves these scores (and slopes): asked before random numbers are drawn for it
 bool causal_takes(const Tensor& x, const std::optional<Tensor>& slopes) {
-    return plain_scores(x) && (!slopes || (on_gpu(*slopes) && slopes->device() == x.device() && slopes->scalar_type() == at::kFloat &&
+    return plain_scores(x) && (!slopes || (plain(*slopes) && slopes->device() == x.device() && slopes->scalar_type() == at::kFloat &&
                                            slopes->numel() == x.size(1) && slopes->is_contiguous() && !slopes->requires_grad()));
 }
 
@@ -246,12 +249,12 @@ public:
 
 // strides that count from the tensor's first element upwards, and extents the kernels count in 32 bits
 bool plain_heads(const Tensor& x) {
-    return on_gpu(x) && half_type(x) && x.dim() == 4 && x.numel() > 0 && x.stride(3) == 1 && fits_int32(x.size(0)) &&
+    return plain(x) && half_type(x) && x.dim() == 4 && x.numel() > 0 && x.stride(3) == 1 && fits_int32(x.size(0)) &&
            fits_int32(x.size(1)) && fits_int32(x.size(2)) && fits_int32(x.size(3));
 }
 // a table [n, 1, 1, d_rot] of dense rows in memory order, with the rows offset .. offset + s
 bool plain_table(const Tensor& t, const Tensor& x, int64_t d_rot, int64_t rows) {
-    return on_gpu(t) && t.device() == x.device() && t.dim() == 4 && t.size(1) == 1 && t.size(2) == 1 && t.size(3) == d_rot &&
+    return plain(t) && t.device() == x.device() && t.dim() == 4 && t.size(1) == 1 && t.size(2) == 1 && t.size(3) == d_rot &&
            t.size(0) >= rows && t.is_contiguous() && !t.requires_grad();
 }
 

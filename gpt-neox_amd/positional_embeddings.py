@@ -157,10 +157,12 @@ def _on(t, device):
     return t if t.device == device else t.to(device)
 
 
-def _needs_grad(*tensors):
+def _needs_grad(*tensors, tables=()):
     """Whether autograd has to record the call (else the autograd Function, which costs the host
-    several microseconds per call, is bypassed)."""
-    return torch.is_grad_enabled() and any(t.requires_grad for t in tensors)
+    several microseconds per call, is bypassed), or to refuse it: nothing here has a forward-mode
+    derivative, and a tangent is not to get lost on the way."""
+    return (torch.is_grad_enabled() and any(t.requires_grad for t in tensors)
+            or _lib.carries_tangent(*tensors, *tables))
 
 
 def _rotary_out_of_place(q, k, cos, sin, offset):
@@ -225,7 +227,7 @@ def apply_rotary_pos_emb(q, k, cos, sin, offset: int = 0):
         if out is not None:
             return out
     if _fusable(q, k, cos, sin):
-        if not _needs_grad(q, k):
+        if not _needs_grad(q, k, tables=(cos, sin)):
             return _rotary_out_of_place(q, k, _on(cos, q.device), _on(sin, q.device), offset)[:2]
         return _FusedRotary.apply(q, k, _on(cos, q.device), _on(sin, q.device), offset)
     return _rotary_torch(q, k, cos, sin, offset)
@@ -244,10 +246,10 @@ def apply_rotary_pos_emb_torch(q, k, cos, sin, offset: int = 0):
 _increment_version = getattr(torch.autograd.graph, "increment_version", None)
 
 
-def _may_bypass_autograd(*tensors):
+def _may_bypass_autograd(*tensors, tables):
     """The in-place rotation may skip the autograd Function: nothing needs a gradient and the
     version counters can still be bumped (or no graph is being recorded at all)."""
-    return not _needs_grad(*tensors) and (_increment_version is not None or not torch.is_grad_enabled())
+    return not _needs_grad(*tensors, tables=tables) and (_increment_version is not None or not torch.is_grad_enabled())
 
 
 def _written_in_place(*tensors):
@@ -297,7 +299,7 @@ def apply_rotary_pos_emb_(q, k, cos, sin, offset: int = 0, rotary_ndims=None):
         )
     if d_rot > q.shape[-1] or d_rot % 2:
         raise RuntimeError(f"rotary_ndims={d_rot} must be even and <= head size {q.shape[-1]}")
-    if _may_bypass_autograd(q, k):
+    if _may_bypass_autograd(q, k, tables=(cos, sin)):
         _rotary_in_place(q, k, _on(cos, q.device), _on(sin, q.device), offset, d_rot)
         _written_in_place(q, k)
         return q, k
@@ -356,7 +358,7 @@ def apply_rotary_pos_emb_qkv_(mixed_x_layer, cos, sin, offset: int = 0, rotary_n
             "cos/sin in fp32 or its dtype"
         )
     dev = mixed_x_layer.device
-    if _may_bypass_autograd(mixed_x_layer):
+    if _may_bypass_autograd(mixed_x_layer, tables=(cos, sin)):
         mixed = mixed_x_layer
         if mixed.numel():
             _rotary_in_place(mixed[..., :hn], mixed[..., hn : 2 * hn], _on(cos, dev), _on(sin, dev), offset, d_rot)

@@ -4,10 +4,12 @@ every form the native calls take; what they leave alone goes, and fails, the gen
 import pytest
 import torch
 import torch.utils.checkpoint
+from torch.autograd import forward_ad
 
 from gpt_neox_amd import _lib, fused_rope
 from gpt_neox_amd.fused_softmax import FusedScaleMaskSoftmax, SoftmaxFusionTypes
-from gpt_neox_amd.positional_embeddings import AliBi, apply_rotary_pos_emb
+from gpt_neox_amd.positional_embeddings import (AliBi, apply_rotary_pos_emb, apply_rotary_pos_emb_,
+                                                apply_rotary_pos_emb_qkv_)
 
 gpu = pytest.mark.gpu
 DTYPES = [torch.float16, torch.bfloat16]
@@ -200,6 +202,49 @@ def test_exceptions_of_saved_tensor_hooks_and_activation_checkpointing(device):
         want = torch.autograd.grad(call().float().pow(2).sum(), leaf)[0]
         y = torch.utils.checkpoint.checkpoint(lambda _: call(), leaf, use_reentrant=False)
         assert torch.equal(torch.autograd.grad(y.float().pow(2).sum(), leaf)[0], want)
+
+
+@gpu
+def test_forward_mode_derivatives_are_refused(device):
+    # no kernel computes a tangent: an error, and not a result whose derivative has become zero
+    t = torch.randn(4, 1, 2, 16, device=device).half()
+    cos, sin = torch.randn(2, 4, 1, 1, 16, device=device)
+    x = torch.randn(2, 4, 40, 40, device=device).half()
+    wide = torch.randn(1, 2, 648, 648, device=device).half()
+    causal, window = causal_mask(40, device), causal_mask(648, device, 100)
+    some = torch.rand(1, 1, 40, 40, device=device) < 0.4
+    padding = (torch.arange(40, device=device) >= 20).view(1, 1, 1, 40).expand(1, 1, 40, 40).contiguous()
+    slopes = AliBi(4, mp_size=1, mp_rank=0).slopes.to(device)
+    upper, general = (module(torch.float16, f) for f in (SoftmaxFusionTypes.upper_triang, SoftmaxFusionTypes.general))
+    ends = FusedScaleMaskSoftmax(True, False, SoftmaxFusionTypes.general, None, True, 0.125, causal_mask_check="verify")
+    calls = {  # name: (call, the arguments that may be dual)
+        "rope": (fused_rope.fused_apply_rotary_pos_emb, (t, cos)),
+        "rope cached": (fused_rope.fused_apply_rotary_pos_emb_cached, (t, cos, sin)),
+        "rotary": (apply_rotary_pos_emb, (t, t.clone(), cos, sin)),
+        "rotary in place": (apply_rotary_pos_emb_, (t.clone(), t.clone(), cos, sin)),
+        "rotary of a projection": (apply_rotary_pos_emb_qkv_, (torch.randn(4, 1, 2, 48, device=device).half(), cos, sin)),
+        "causal": (lambda x: upper(x, causal), (x,)),
+        "window": (lambda x: upper(x, window), (wide,)),
+        "mask": (lambda x: general(x, some), (x,)),
+        "mask with row ends": (lambda x: ends(x, padding), (x,)),
+        "alibi": (lambda x, s: upper(x, causal, alibi_slopes=s), (x, slopes)),
+        "dropout": (lambda x: upper(x, causal, dropout_p=0.25), (x,)),
+        "alibi dropout": (lambda x, s: upper(x, causal, alibi_slopes=s, dropout_p=0.25), (x, slopes)),
+    }
+    passed = []
+    for name, (call, args) in calls.items():
+        for i, a in enumerate(args):
+            with forward_ad.dual_level():
+                dual = [forward_ad.make_dual(b, torch.ones_like(b)) if j == i else b for j, b in enumerate(args)]
+                for grad in (True, False):
+                    try:
+                        with torch.set_grad_enabled(grad):
+                            call(*dual)
+                        passed.append((name, i, grad))
+                    except NotImplementedError as e:
+                        assert "jvp" in str(e)
+        call(*args)  # and outside of the level as ever
+    assert not passed
 
 
 @gpu
