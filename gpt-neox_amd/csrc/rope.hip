@@ -112,6 +112,40 @@ static bool try_launch_rope_piece(const RopeArgs& a, int s, int n_outer, hipStre
     return true;
 }
 
+// the rotated span, with the slots stored as loaded behind it, is at most 64 slots of w >= 2 dims:
+// the contiguous-span kernel applies (a pass-through copy must be covered by those slots)
+static bool span_shape(const RopeArgs& a, int w) {
+    return w >= 2 && a.lpv * 2 + a.pad_slots <= kWave && (a.copy_dims == 0 || a.pad_slots * w == a.copy_dims);
+}
+
+// Whether dense heads with angles go to the run kernel rather than to launch_rope_w's: `rounds` sine and cosine
+// evaluations per lane, at most, in a wave of the run kernel, whose 1024 dims no other wave shares them with.
+// A block of rope_span_kernel evaluates a position's angles once for up to 4096 dims, on the other hand with as many
+// of its lanes idle as its head vectors leave.  us per launch, that kernel -> the run kernel:
+//   up to two rounds, any fill: [2048,2,64,96] d_rot 24 27.7 -> 18.6, [2048,1,32,128] d_rot 128 9.1 -> 8.6, [2048,2,64,96]
+//     d_rot 96 20.4 -> 20.0, [2048,2,32,256] d_rot 64 25.1 -> 23.1; the one behind: [2048,2,64,112] d_rot 112 22.7 -> 23.1
+//   more, at most 5/8 of the lanes at work, and that share times the rounds at most 3: [32768,1,2,256] d_rot 256
+//     78 -> 23, [8192,1,8,256] 22.6 -> 17.0, [8192,1,20,256] 43 -> 36, [8192,1,2,512] d_rot 512 23.3 -> 14.3; beyond 3, behind:
+//     [8192,1,4,512] (8 rounds, half the lanes) 24.1 -> 26.2, [8192,1,16,160] (5 rounds, 5/8) 19.9 -> 20.7
+//   more, fuller blocks, all behind: [2048,2,16,256] d_rot 256 14.8 -> 17.0, [2048,2,8,512] d_rot 512 15.8 -> 26.1, [4096,1,32,112]
+//     d_rot 112 13.3 -> 14.4, [2048,1,40,96] d_rot 96 8.8 -> 9.1, [2048,2,32,160] d_rot 160 17.9 -> 19.4
+//   8- and 4-byte slots, which rope_span_kernel moves one by one: [2048,1,40,88] d_rot 88 12.0 -> 8.9, [2048,2,24,168] 22.3 -> 17.9,
+//     [8192,1,8,168] 15.3 -> 14.6; beyond 192 dims where few waves straddle positions, [2048,2,32,200] 29.4 -> 25.9, or the
+//     blocks are as empty as above, [8192,1,4,200] 13.8 -> 11.2; behind: [8192,1,8,200] 15.9 -> 16.6
+//   heads of more than 64 slots, element by element there: [2048,2,16,520] d_rot 256 61 -> 30, [2048,2,8,1024] d_rot 512 57 -> 49;
+//     with nothing to pass through rope_kernel is as wide: [2048,2,16,264] d_rot 264 17.9 -> 21.1
+static bool angles_in_runs(const RopeArgs& a, int w, int rounds) {
+    if (!span_shape(a, w)) return a.copy_dims > 0;
+    if (rounds <= 2) return true;
+    const int lph = a.lpv * 2 + a.pad_slots;
+    const int64_t per_block = (int64_t)(256 / kWave) * (kWave / lph) * kSpanIters;  // head vectors, as in launch_rope_span
+    const int64_t n = a.nt > 1 && a.t[1].n_inner > a.t[0].n_inner ? a.t[1].n_inner : a.t[0].n_inner;
+    const int64_t used = n * lph, lanes = (n + per_block - 1) / per_block * (256 * kSpanIters);
+    const bool idle = used * 8 <= lanes * 5;
+    if (w < kVec) return a.half <= 96 || idle || n * (2 * a.half + a.copy_dims) >= 8 * kRunSlots * kVec;
+    return idle && used * rounds <= lanes * 3;
+}
+
 template <typename T, typename CS, int PW, bool BWD>
 static hipError_t launch_rope_run(const RopeRunArgs& r, int nt, hipStream_t st) {
     const uint32_t slots = nt > 1 && r.slots[1] > r.slots[0] ? r.slots[1] : r.slots[0];
@@ -124,16 +158,14 @@ static hipError_t launch_rope_run(const RopeRunArgs& r, int nt, hipStream_t st) 
 // Whole heads of dense tensors, out of place: the run kernel (see rope_run_kernel).  Returns false if the
 // call does not qualify.
 template <typename T, typename CS, bool BWD>
-static bool try_launch_rope_run(const RopeArgs& a, int s, int n_outer, hipStream_t st, hipError_t* err) {
+static bool try_launch_rope_run(const RopeArgs& a, int s, int n_outer, int w, hipStream_t st, hipError_t* err) {
     const int d_rot = 2 * a.half, d = d_rot + a.copy_dims;
     if (n_outer != 1 || d % kVec != 0 || a.half % 2 != 0) return false;
-    // Angles: always faster than rope_span_kernel, which alone takes them otherwise.  Tables: where the half span
-    // is no multiple of 8 dims the other kernels move 8 or 4 bytes per access; where it is, or where the whole head
-    // rotates, rope_piece_kernel reads nothing twice.  us per launch, fp16, that kernel or rope_span_kernel -> this:
-    // [2048,2,64,96] d_rot 24 angles 27.7 -> 18.6, tables 25.9 -> 18.9; [2048,2,40,80] d_rot 20 angles 28.6 -> 12.1,
-    // tables 24.5 -> 12.2, d_rot 40 angles 15.4 -> 12.3; angles [2048,2,64,128] d_rot 32 24.9 -> 23.3, d_rot = d = 96
-    // 20.5 -> 20.1; against it: tables [2048,2,64,128] d_rot 32 23.3 -> 23.7, d_rot = d = 128 13.3 -> 14.6,
-    // d_rot = d = 40 18.3 -> 19.1 (bf16, q and k).
+    // Tables: where the half span is no multiple of 8 dims the other kernels move 8 or 4 bytes per access; where it is,
+    // or where the whole head rotates, rope_piece_kernel reads nothing twice.  us per launch, fp16, that kernel or
+    // rope_span_kernel -> this: [2048,2,64,96] d_rot 24 25.7 -> 18.8, [2048,2,40,80] d_rot 20 24.5 -> 12.2, [2048,2,8,256]
+    // d_rot 24 9.0 -> 7.8; against it: [2048,2,64,128] d_rot 32 23.3 -> 23.7, d_rot = d = 128 13.3 -> 14.6, d_rot = d = 40
+    // 18.3 -> 19.1 (bf16, q and k).  Angles: angles_in_runs.
     if (!std::is_same<CS, Angles>::value && (a.half % kVec == 0 || a.copy_dims == 0)) return false;
     RopeRunArgs r{};
     uint32_t positions = 0;  // that a piece can touch
@@ -168,6 +200,15 @@ static bool try_launch_rope_run(const RopeArgs& a, int s, int n_outer, hipStream
     r.row = (uint32_t)(d_rot + kVec - 1) & ~(uint32_t)(kVec - 1);
     r.wave_floats = positions * 2 * r.row;
     if (r.wave_floats > 2048) return false;  // 32 KiB a block: heads of few bytes per position touch many positions
+    if constexpr (std::is_same<CS, Angles>::value) {
+        uint32_t evaluated = 0;  // positions whose angles a wave evaluates: one where every position is whole waves
+        for (int i = 0; i < a.nt; ++i) {
+            const uint32_t per_pos = (uint32_t)a.t[i].n_inner * spv;
+            const uint32_t p = per_pos % kRunSlots == 0 ? 1u : kRunSlots % per_pos == 0 ? kRunSlots / per_pos : positions;
+            if (p > evaluated) evaluated = p;
+        }
+        if (!angles_in_runs(a, w, (int)((evaluated * (uint32_t)d_rot + kWave - 1) / kWave))) return false;
+    }
     if constexpr (std::is_same<CS, Angles>::value) {
         if (a.half % 8 == 0) {
             *err = launch_rope_run<T, CS, 8, BWD>(r, a.nt, st);
@@ -214,12 +255,6 @@ static bool try_launch_rope_cell(const RopeArgs& a, int s, int n_outer, int w, h
     return true;
 }
 
-// the rotated span, with the slots stored as loaded behind it, is at most 64 slots of w >= 2 dims:
-// the contiguous-span kernel applies (a pass-through copy must be covered by those slots)
-static bool span_shape(const RopeArgs& a, int w) {
-    return w >= 2 && a.lpv * 2 + a.pad_slots <= kWave && (a.copy_dims == 0 || a.pad_slots * w == a.copy_dims);
-}
-
 template <typename T, typename CS, bool BWD>
 static hipError_t launch_rope_w(const RopeArgs& a, int s, int n_outer, int w, hipStream_t st) {
     if (span_shape(a, w)) {
@@ -242,8 +277,8 @@ template <typename T, typename CS>
 static hipError_t launch_rope_dir(const RopeArgs& a, int s, int n_outer, int w, bool backward,
                                   hipStream_t st) {
     hipError_t err = hipSuccess;
-    if (backward ? try_launch_rope_run<T, CS, true>(a, s, n_outer, st, &err)
-                 : try_launch_rope_run<T, CS, false>(a, s, n_outer, st, &err)) return err;
+    if (backward ? try_launch_rope_run<T, CS, true>(a, s, n_outer, w, st, &err)
+                 : try_launch_rope_run<T, CS, false>(a, s, n_outer, w, st, &err)) return err;
     if constexpr (!std::is_same<CS, Angles>::value) {
         if (backward ? try_launch_rope_cell<T, CS, true>(a, s, n_outer, w, st, &err)
                      : try_launch_rope_cell<T, CS, false>(a, s, n_outer, w, st, &err)) return err;

@@ -256,3 +256,19 @@ def test_dense_heads_in_pieces(device, dtype, shape, d2):
                 assert_within_one_ulp(out, want, dtype)
             assert torch.equal(out[..., d2:], t[..., d2:])
             assert (buf[:32] == 7).all() and (buf[-32:] == 7).all()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("shape,d2", [
+    ((20, 2, 16, 256), 256),   # dense heads whose angles take four rounds of a wave's lanes, blocks of span heads filled
+    ((20, 1, 8, 256), 256),    # ... half filled
+    ((20, 1, 4, 512), 512),    # ... half filled, eight rounds
+    ((9, 1, 32, 112), 112),    # positions that are no whole number of waves
+    ((9, 1, 128, 112), 112),   # ... and that are
+    ((9, 1, 16, 168), 168),    # 8-byte slots, up to and behind 192 rotated dims
+    ((9, 1, 16, 200), 200),
+    ((5, 1, 6, 520), 256),     # more than 64 slots, with and without something to pass through
+    ((5, 1, 6, 264), 264),
+])
+def test_angles_on_both_sides_of_the_rule(device, dtype, shape, d2):
+    check_both_variants(normal(shape, dtype, device, 43), d2, False, device)
