@@ -40,6 +40,13 @@ namespace neox {
 // every kernel of the unit is compiled for exactly that set: the caller picks the unit by what the
 // call brings along (slopes, a bias tensor, a dropout probability, unaligned rows).
 
+// the output starts on a 4 KiB boundary (both outputs, with dropout)
+static bool on_pieces(const SoftmaxArgs& a) {
+    return (reinterpret_cast<uintptr_t>(a.out) & 4095u) == 0 && (a.out2 == nullptr || (reinterpret_cast<uintptr_t>(a.out2) & 4095u) == 0);
+}
+// rows of two 4 KiB pieces each, which several rows per block store in the order of with_xcd_mapping
+static bool two_piece_rows(const SoftmaxArgs& a) { return a.sk * 2 == 8192 && on_pieces(a); }
+
 // Switches the XCD-aware block -> unit mapping on (see xcd_slot) when the work units of a block
 // -- `units` of them, `unit_bytes` each, consecutive in memory -- tile 4 KiB pieces exactly and
 // the output starts on a 4 KiB boundary; and for rows of two pieces, several per block.
@@ -48,8 +55,7 @@ static SoftmaxArgs with_xcd_mapping(const SoftmaxArgs& a, uint64_t unit_bytes, u
     b.piece_shift = 0;
     b.group_shift = 3;
     b.affine_blocks = 0;
-    const bool aligned = (reinterpret_cast<uintptr_t>(a.out) & 4095u) == 0 &&
-                         (a.out2 == nullptr || (reinterpret_cast<uintptr_t>(a.out2) & 4095u) == 0);
+    const bool aligned = on_pieces(a);
     if (aligned && unit_bytes > 0 && unit_bytes <= 4096 && 4096 % unit_bytes == 0 && blocks >= 8) {
         const uint32_t upp = (uint32_t)(4096 / unit_bytes);
         if (units % upp == 0 && units / upp >= 1) {
@@ -312,8 +318,9 @@ static hipError_t dispatch_rows(const SoftmaxArgs& a, bool vec_ok, hipStream_t s
     }
     if constexpr ((EXTRA & kBand) != 0) {
         // rows of two 4 KiB pieces: two per block, in the order of with_xcd_mapping ([32,4096,4096] window 2048:
-        // 248 -> 234 us forward, 317 -> 311 backward; at 8192 columns, which that order does not serve, 230 -> 254)
-        if (chunks <= 6 && a.sk == 4096) return launch_shape<T, M, BWD, EXTRA, 3, 2, 2>(a, st);
+        // 248 -> 232 us forward, 315 -> 306 backward; window 1600 239 -> 222 and 298 -> 281).  Without that order the shape
+        // loses: on an output off the 4 KiB boundary 263 -> 284 and 341 -> 354, 3600 columns 219 -> 226 and 284 -> 297.
+        if (chunks <= 6 && two_piece_rows(a)) return launch_shape<T, M, BWD, EXTRA, 3, 2, 2>(a, st);
     }
     constexpr bool two_rows = M == Mask::Causal && (EXTRA & kBand) == 0 && !(BWD && (EXTRA & kDropout) != 0);
     if constexpr (two_rows) {

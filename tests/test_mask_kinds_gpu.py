@@ -8,7 +8,7 @@ bars of fp32 autograd from x, hidden positions exactly 0 in both.
 import pytest
 import torch
 
-from gpt_neox_amd import fused_softmax as fs
+from gpt_neox_amd import _lib, fused_softmax as fs
 from gpt_neox_amd.fused_kernels import scaled_masked_softmax_cuda as masked_ext
 from gpt_neox_amd.fused_kernels import scaled_upper_triang_masked_softmax_cuda as causal_ext
 from gpt_neox_amd.fused_softmax import FusedScaleMaskSoftmax, ScaledSlidingWindowSoftmax, SoftmaxFusionTypes
@@ -138,6 +138,25 @@ def test_sliding_window_sizes(device, s, w, dtype):
                                  (4104, 600), (5000, 1250), (8192, 512), (8192, 1535), (16384, 1024)])
 def test_sliding_window_order_and_shapes(device, s, w, dtype):
     check_window(device, 2 if s <= 4104 else 1, s, w, dtype, 0.125, seed=s + w)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("w", [1600, 2048])
+def test_sliding_window_off_the_piece_boundary(device, w, dtype):
+    # rows of two 4 KiB pieces whose outputs start 16 bytes behind a piece: another kernel shape, in plain order
+    s, batches = 4096, 2
+    lib, code, stream = _lib.lib(), _lib.dtype_code(dtype), torch.cuda.current_stream().cuda_stream
+    x, g = scores((batches, s, s), dtype, device, w), normal((batches, s, s), dtype, device, w + 1)
+    bufs = [torch.full((x.numel() + 4096,), 7.0, dtype=dtype, device=device) for _ in range(2)]
+    at = [(4096 - t.data_ptr() % 4096) // 2 % 2048 + 8 for t in bufs]
+    y, dx = (t[a : a + x.numel()].view(x.shape) for t, a in zip(bufs, at))
+    assert y.data_ptr() % 4096 == dx.data_ptr() % 4096 == 16
+    _lib.check(lib.neox_sliding_window_softmax_fwd(y.data_ptr(), x.data_ptr(), 0.125, batches, s, s, w, code, stream))
+    _lib.check(lib.neox_sliding_window_softmax_bwd(dx.data_ptr(), g.data_ptr(), y.data_ptr(), 0.125, batches, s, s, w, code, stream))
+    hidden = R.get_attn_mask(s, device, sliding_window_width=w)[0].expand_as(y)
+    assert max_err(y, R.softmax_fp32(x, hidden, 0.125)) <= TOL[dtype] and (y[hidden] == 0).all()
+    assert max_err(dx, R.softmax_backward_fp32(g, y, 0.125)) <= TOL[dtype] and (dx[hidden] == 0).all()
+    assert all((t[:a] == 7).all() and (t[a + x.numel() :] == 7).all() for t, a in zip(bufs, at))
 
 
 # (the kernel shape goes by the chunks a band can touch, w / 512 + 2, capped by the row's: narrow windows on long
