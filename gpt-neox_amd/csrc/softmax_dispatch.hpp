@@ -286,10 +286,12 @@ static hipError_t dispatch_rows(const SoftmaxArgs& a, bool vec_ok, hipStream_t s
     if constexpr (!(BWD && M == Mask::None && (EXTRA & kRagged) == 0)) {
         if (chunks == 2) return launch_shape<T, M, BWD, EXTRA, 2, 1, 4>(a, st);
         if constexpr ((EXTRA & kBand) != 0) {
-            // rows that are mostly zeros in front of and behind the band: twice the waves, one chunk of the band
-            // each ([8,8192,8192] window 1024: 220 -> 207 us forward, 241 -> 236 backward; [20,5000,5000] window 1250:
-            // 252 -> 236 and 294 -> 274; 3000 columns +2 and -3 %)
-            if (a.sk > 4096 && (chunks == 3 || chunks == 4)) return launch_shape<T, M, BWD, EXTRA, 1, 4, 1>(a, st);
+            // rows that are mostly zeros in front of and behind the band: twice the waves, one chunk of the band each.
+            // us per launch forward / backward, two chunks per wave -> one: [8,8192,8192] window 1024 220 -> 207 / 241 -> 236,
+            // [20,5000,5000] window 1250 252 -> 236 / 294 -> 274, [4,12288,12288] 1500 272 -> 243 / 280 -> 270, [3,14336,14336] 1024
+            // 273 -> 260 / 268 -> 254; behind at 3000 columns (+2 / -3 %) and beyond 28 chunks: [2,15360,15360] 1024 200 -> 204 /
+            // 207 -> 203, [2,16384,16384] 1500 210 -> 232 / 223 -> 232, [1,32768,32768] 1024 408 -> 446 / 431 -> 460
+            if (a.sk > 4096 && a.sk <= 28 * kChunk && (chunks == 3 || chunks == 4)) return launch_shape<T, M, BWD, EXTRA, 1, 4, 1>(a, st);
         }
         if (chunks == 3) return launch_shape<T, M, BWD, EXTRA, 2, 2, 2>(a, st);
         if (chunks == 4) {

@@ -133,9 +133,10 @@ def test_sliding_window_sizes(device, s, w, dtype):
 
 @pytest.mark.parametrize("dtype", DTYPES)
 # rows of two 4 KiB pieces, several per block and out of order, with bands of two to seven chunks; longer rows
-# with a band of three or four chunks, one per wave
+# with a band of three or four chunks, one per wave up to 14336 columns
 @pytest.mark.parametrize("s,w", [(4096, 300), (4096, 512), (4096, 1023), (4096, 1535), (4096, 2048), (4096, 2600),
-                                 (4104, 600), (5000, 1250), (8192, 512), (8192, 1535), (16384, 1024)])
+                                 (4104, 600), (5000, 1250), (8192, 512), (8192, 1535), (14336, 1024), (14344, 1024),
+                                 (14344, 1100), (16384, 1024)])
 def test_sliding_window_order_and_shapes(device, s, w, dtype):
     check_window(device, 2 if s <= 4104 else 1, s, w, dtype, 0.125, seed=s + w)
 
