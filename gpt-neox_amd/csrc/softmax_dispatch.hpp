@@ -10,7 +10,7 @@
 //   chunks == 2    1 wave per row, 4 rows per 256-thread block      (sk <= 1024)
 //   chunks <= 4    2 waves per row, 2 rows per block (4 rows at 4 chunks: 2-3 % faster in an
 //                  interleaved comparison; at 3 chunks 2 rows are)   (sk <= 2048)
-//   chunks <= 8    4 waves per row (causal rows of 7 or 8 chunks: 2 rows per block)  (sk <= 4096)
+//   chunks <= 8    4 waves per row (2 rows per block: two_causal_rows)  (sk <= 4096)
 //   chunks <= 16   8 waves per row, 512-thread block                 (sk <= 8192)
 //   chunks <= 32   16 waves per row, 1024-thread block               (sk <= 16384)
 //                  forward, in the lower 3/4 of each of these three ranges (7/8 of the last):
@@ -259,6 +259,30 @@ static std::optional<hipError_t> dispatch_aligned(const SoftmaxArgs& a, bool vec
     return std::nullopt;
 }
 
+// Whether causal rows of 7 or 8 chunks go two to a block (not the dropout backward: [16,4096,4096] 174 -> 175 us, [16,3840,3840]
+// 156 -> 161).  It pays where neighbouring rows share a cache line, which one block then stores as a whole, and at 4096
+// columns in the order of with_xcd_mapping.  us per launch forward / backward / forward with dropout (16 matrices), one row per
+// block -> two, 32 matrices; alignment of the rows:
+//   32 or 64 bytes   3248 186 -> 177 / 245 -> 233 / 159 -> 152, 3616 227 -> 215 / 307 -> 286 / 193 -> 183, 4000 279 -> 263 / 375 -> 351 /
+//                    223 -> 213, 3088 158 -> 159 / 218 -> 218 / 139 -> 139
+//   128 bytes        3200 165 -> 169 / 215 -> 222 / 140 -> 141, 3712 221 -> 221 / 292 -> 291 / 183 -> 182, 3968 245 -> 251 / 330 -> 332;
+//                    4096 265 -> 254 / 346 -> 340 / 227 -> 217, but off the 4 KiB boundary 279 -> 275 / 373 -> 373
+//   16 bytes         3080 159 -> 161 / 211 -> 219 / 139 -> 141, 3592 219 -> 219 / 292 -> 299, 4088 279 -> 287 / 376 -> 390 / 248 -> 257
+//   8 bytes          3076 162 -> 172 / 220 -> 214, 3500 207 -> 213 / 283 -> 274 / 194 -> 184, 4004 269 -> 273 / 372 -> 361 / 251 -> 237
+//   4 bytes          3130 168 -> 175 / 224 -> 218 / 153 -> 164, 3998 260 -> 268 / 361 -> 354 / 241 -> 256
+//   2 bytes          3201 184 -> 187 / 245 -> 234, 3333 197 -> 198 / 265 -> 254 / 182 -> 182, 3689 237 -> 235 / 320 -> 306 / 220 -> 216,
+//                    3999 277 -> 275 / 373 -> 358 / 254 -> 251
+// (rows of 16 bytes and more on tensors off a 16-byte boundary were not measured: one row).  One or two matrices leave too few blocks
+// for either: [1,3616,3616] forward 9.5 -> 9.9, [2,4096,4096] 18.8 -> 19.1, [4,3616,3616] 29.7 -> 29.5.
+template <bool BWD, int EXTRA>
+static bool two_causal_rows(const SoftmaxArgs& a, int chunks) {
+    if (a.rows < 12288) return false;
+    if constexpr ((EXTRA & kRagged) == 0) return (a.sk % 16 == 0 && a.sk % 64 != 0) || two_piece_rows(a);
+    else if (BWD) return a.sk % 8 != 0;
+    else if (a.sk % 2 != 0) return chunks == 8;
+    else return (EXTRA & kDropout) != 0 && a.sk % 8 == 4;
+}
+
 template <typename T, Mask M, bool BWD, int EXTRA>
 static hipError_t dispatch_rows(const SoftmaxArgs& a, bool vec_ok, hipStream_t st) {
     int chunks = (a.sk + kChunk - 1) / kChunk;
@@ -324,17 +348,10 @@ static hipError_t dispatch_rows(const SoftmaxArgs& a, bool vec_ok, hipStream_t s
         // loses: on an output off the 4 KiB boundary 263 -> 284 and 341 -> 354, 3600 columns 219 -> 226 and 284 -> 297.
         if (chunks <= 6 && two_piece_rows(a)) return launch_shape<T, M, BWD, EXTRA, 3, 2, 2>(a, st);
     }
-    constexpr bool two_rows = M == Mask::Causal && (EXTRA & kBand) == 0 && !(BWD && (EXTRA & kDropout) != 0);
-    if constexpr (two_rows) {
-        // Causal rows of 3585-4096 columns: two per block, at 4096 columns in the order of with_xcd_mapping.  us per launch
-        // forward / backward, one row per block -> two: bf16 [32,4096,4096] 265 -> 254 / 346 -> 340, fp16 [32,4000,4000]
-        // 284 -> 265 / 375 -> 354, bf16 [32,3999,3999] 276 -> 275 / 377 -> 360, with dropout [16,4096,4096] 228 -> 217 /
-        // 174 -> 175, [16,3840,3840] 202 -> 200 / 156 -> 161: the dropout backward stays.  Four chunks per wave: 1-2 % behind.
-        if (chunks == 7 || chunks == 8) return launch_shape<T, M, BWD, EXTRA, 2, 4, 2>(a, st);
+    if constexpr (M == Mask::Causal && (EXTRA & kBand) == 0 && !(BWD && (EXTRA & kDropout) != 0)) {
+        if (chunks >= 7 && chunks <= 8 && two_causal_rows<BWD, EXTRA>(a, chunks)) return launch_shape<T, M, BWD, EXTRA, 2, 4, 2>(a, st);
     }
-    if constexpr (!two_rows || BWD) {  // (the causal forward has taken all of them above)
-        if (chunks <= 8) return launch_shape<T, M, BWD, EXTRA, 2, 4, 1>(a, st);
-    }
+    if (chunks <= 8) return launch_shape<T, M, BWD, EXTRA, 2, 4, 1>(a, st);
     if (chunks <= 16) return launch_shape<T, M, BWD, EXTRA, 2, 8, 1>(a, st);
     if (chunks <= 32) return launch_shape<T, M, BWD, EXTRA, 2, 16, 1>(a, st);
     if (chunks <= 48) return launch_shape<T, M, BWD, EXTRA, 3, 16, 1>(a, st);

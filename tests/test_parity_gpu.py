@@ -1644,3 +1644,46 @@ def test_short_causal_rows_on_both_sides_of_the_lane_rule(device, s, shift, slop
     else:
         y = causal_ext.forward_nd(x, 0.125)
     assert max_err(y, want) <= TOL[dtype] and (y[..., hidden] == 0).all()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("slopes,with_bias,p", [(s, b, p) for s in (False, True) for b in (False, True) for p in (0.0, 0.25)])
+@pytest.mark.parametrize("np_,sq,sk", [
+    (4, 3616, 3616),  # rows of whole 64 bytes: two per block in every pass
+    (4, 3111, 3592),  # rows of whole 16 bytes: one
+    (5, 2502, 3589),  # odd rows: two (an even number a matrix: the sums' order goes by the parity of a row's start)
+    (5, 2501, 3500),  # rows of whole 8 bytes, an odd number: two in the dropout forward and in the backward pass
+    (4, 3100, 3130),  # rows of whole 4 bytes: two in the backward pass
+])
+def test_two_causal_rows_per_block(device, np_, sq, sk, slopes, with_bias, p, dtype):
+    # enough rows for two per block, against the same matrices one by one, which are too few for it: the same sums
+    # in the same order, the same bits; one matrix against the fp32 expression
+    x, g = scores((1, np_, sq, sk), dtype, device, sk), normal((1, np_, sq, sk), dtype, device, sk + 1)
+    bias = normal((1, np_, sq, sk), dtype, device, sk + 2) if with_bias else None
+    sl = torch.tensor([2.0 ** -i for i in range(1, np_ + 1)], device=device) if slopes else None
+
+    def probs(x, sl, bias):
+        if bias is not None:
+            return causal_ext.forward_bias(x, bias, 0.125, sl)
+        return causal_ext.forward_nd(x, 0.125) if sl is None else causal_ext.forward_alibi(x, sl, 0.125)
+
+    each = [slice(m, m + 1) for m in range(np_)]
+    alone = torch.cat([probs(x[:, m], None if sl is None else sl[m], None if bias is None else bias[:, m]) for m in each], 1)
+    if p:
+        y, dropped = causal_ext.forward_dropout(x, 0.125, p, 9, 4, slopes=sl, bias=bias)
+        keep = rng_keep(y.numel(), p, 9, 4, device).view(y.shape)
+        assert torch.equal(dropped, R.dropout_with_mask(y, keep, p))
+    else:
+        y = probs(x, sl, bias)
+        dx = causal_ext.backward_nd(g.clone(), y, 0.125)
+        assert torch.equal(dx, torch.cat([causal_ext.backward_nd(g[:, m].clone(), y[:, m].contiguous(), 0.125) for m in each], 1))
+    assert torch.equal(y, alone)
+    hidden = torch.ones(sq, sk, dtype=torch.bool, device=device).triu_(1)
+    total = x[0, 1].float()
+    if with_bias:
+        total += bias[0, 1].float()
+    if slopes:
+        total += sl[1] * (torch.arange(sk, device=device) - torch.arange(sq, device=device).view(-1, 1)).float()
+    assert max_err(y[0, 1], R.softmax_fp32(total, hidden, 0.125)) <= TOL[dtype] and (y[..., hidden] == 0).all()
+    if not p:
+        assert max_err(dx[0, 1], R.softmax_backward_fp32(g[0, 1], y[0, 1], 0.125)) <= TOL[dtype] and (dx[..., hidden] == 0).all()
