@@ -754,10 +754,11 @@ struct Packed {
 
 // Where a wave's results go.  Direct: one 128-bit store per lane and pass, to the lane's columns.  Staged: into
 // LDS at the place they have in memory, from where flush_staged stores the wave's rows -- one run of memory --
-// in whole 1 KiB accesses: where a row's columns are stored by several accesses that share cache lines, the memory
-// system takes them at 60-80 % of its rate.
+// in 1 KiB accesses (a remainder of a few elements aside): where a row's columns are stored by several accesses that
+// share cache lines, the memory system takes them at 60-80 % of its rate.
 struct DirectSink {
     rsrc_t out;
+    __device__ __forceinline__ DirectSink(void* y, size_t at, uint32_t bytes, char*) : out(make_rsrc(static_cast<char*>(y) + at, bytes)) {}
     template <bool NT>
     __device__ __forceinline__ void put(const u32x4& v, uint32_t off, bool active) const {
         packed_st<NT>(out, v, off, active);
@@ -766,6 +767,7 @@ struct DirectSink {
 struct __attribute__((packed, aligned(2))) Slot16 { u32x4 v; };  // 16 bytes at the alignment of an element
 struct StagedSink {
     char* lds;
+    __device__ __forceinline__ StagedSink(void*, size_t, uint32_t, char* stage) : lds(stage) {}
     template <bool NT>
     __device__ __forceinline__ void put(const u32x4& v, uint32_t off, bool active) const {
         if (active) reinterpret_cast<Slot16*>(lds + off)->v = v;
@@ -778,7 +780,8 @@ __device__ __forceinline__ void clear_stage(char* lds, uint32_t n, int lane) {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
 }
-// the n staged elements of a wave to `out`; only the tensor's last wave can have n % 8 != 0
+// the n staged elements of a wave to `out`.  n % 8 is 0 or, where a wave owns four rows of an odd length, 4; the
+// tensor's last wave can leave any remainder.
 template <bool NT>
 __device__ __forceinline__ void flush_staged(rsrc_t out, const char* lds, uint32_t n, int lane) {
     // a wave's LDS accesses are carried out in order: no barrier, but the compiler must keep that order
@@ -799,143 +802,8 @@ __device__ __forceinline__ void flush_staged(rsrc_t out, const char* lds, uint32
 // Returns whether every row has a sum (scores that are NaN or infinite leave none, and no probability in the row).
 template <typename T, int G, Mask MASK, int FLAGS, int R, int C, typename Sink>
 __device__ __forceinline__ bool softmax_fwd_rows(const SoftmaxArgs& a, uint32_t row0, uint32_t rows_here, int lane,
-                                                 const Sink& out, const Sink& out2) {
-    static_assert(C == 1 || G == kWave, "several chunks per row need a whole wave per row");
-    constexpr int RPP = Packed<G, R>::kRowsPerPass;
-    constexpr bool kLdNt = (FLAGS & kNtLoad) != 0, kStNt = (FLAGS & kNtStore) != 0;
-    constexpr bool kRag = (FLAGS & kRagged) != 0;
-    static_assert(!kRag || C == 1, "ragged rows: one chunk per lane group");
-    const int sk = a.sk;
-    const int grp = lane / G;
-    const int back = ragged_back<kRag>((lane % G) * kVec, sk);  // kRagged: see ragged_back
-    const int col0 = (lane % G) * kVec - back;                  // first column of the lane's accesses
-    DropoutArgs drop = a.drop;
-    if constexpr ((FLAGS & kDropout) != 0) drop = resolve(drop);
-    const float ninf = -__builtin_inff();
-
-    const rsrc_t rx = make_rsrc(static_cast<const char*>(a.in0) + (size_t)row0 * sk * 2, rows_here * sk * 2);
-    const rsrc_t rm = make_rsrc(a.mask, a.mask_bytes);
-    const rsrc_t rb = make_rsrc(a.bias, a.bias_bytes);  // kBias: the whole bias tensor
-
-    bool summed = true;
-    u32x4 raw[R][C];
-    u32x4 rawb[R][C];
-    u32x2 mk[R][C];
-    int len[R];
-    int ipos[R];       // row position inside its matrix (ALiBi)
-    float slope2[R];   // slope[head] * scale of the lane's row (ALiBi)
-    const uint32_t i0 = a.by_sq.mod(row0);  // wave-uniform
-#pragma unroll
-    for (int p = 0; p < R; ++p) {
-        const uint32_t lr = p * RPP + grp;  // row of this lane group inside the wave
-        const uint32_t row = row0 + lr;
-        const uint32_t i = wrap_row(i0 + lr, a.by_sq);
-        len[p] = (MASK == Mask::Causal) ? min((int)i + 1, sk) : sk;
-        if (lr >= rows_here) len[p] = 0;
-        ipos[p] = alibi_row_position<MASK>(i, a);
-        slope2[p] = 0.f;
-        if constexpr ((FLAGS & kAlibi) != 0) {
-            const uint32_t safe_row = lr < rows_here ? row : row0;
-            slope2[p] = a.slopes[a.by_np.mod(a.by_sq.div(safe_row))] * a.scale;
-        }
-        if constexpr (MASK == Mask::Bytes) {
-#pragma unroll
-            for (int c = 0; c < C; ++c) {
-                const int col = col0 + c * kChunk;
-                const uint32_t mb = a.mask_bcast ? 0u : a.by_mask_batch.div(row);
-                const uint32_t moff = (mb * (uint32_t)a.sq + i) * sk + col;
-                mk[p][c] = packed_ld_mask(rm, moff, col < len[p]);
-            }
-        }
-    }
-    // the scores (and the bias) after the mask bytes: a lane whose 8 keys are all hidden fetches neither
-#pragma unroll
-    for (int p = 0; p < R; ++p) {
-        const uint32_t lr = p * RPP + grp;
-#pragma unroll
-        for (int c = 0; c < C; ++c) {
-            const int col = col0 + c * kChunk;
-            bool active = col < len[p];
-            // (SoftmaxArgs::row_end is not looked at here: it spared nothing more and cost a load per row)
-            if constexpr (MASK == Mask::Bytes && kSkipHidden && !kRag) active = active && !all_hidden(mk[p][c]);
-            raw[p][c] = packed_ld<kLdNt>(rx, (lr * sk + col) * 2u, active);
-            if constexpr ((FLAGS & kBias) != 0) {
-                const uint32_t boff = (bias_row(row0 + lr, a) * (uint32_t)sk + col) * 2u;
-                rawb[p][c] = packed_ld<false>(rb, boff, active);
-            }
-        }
-    }
-
-#pragma unroll
-    for (int p = 0; p < R; ++p) {
-        float v[C][8];
-        float mx = ninf;
-#pragma unroll
-        for (int c = 0; c < C; ++c) {
-            const int col = col0 + c * kChunk;
-            unpack8<T>(raw[p][c], v[c]);
-            if constexpr ((FLAGS & kBias) != 0) {
-                float bv[8];
-                unpack8<T>(rawb[p][c], bv);
-#pragma unroll
-                for (int k = 0; k < 8; ++k) v[c][k] += bv[k];
-            }
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                bool keep = (col + k) < len[p];
-                if constexpr (MASK == Mask::Bytes) {
-                    const uint32_t w = (k < 4) ? mk[p][c].x : mk[p][c].y;
-                    keep = keep && (((w >> (8 * (k & 3))) & 0xffu) == 0);
-                }
-                float bias = 0.f;
-                if constexpr ((FLAGS & kAlibi) != 0) bias = slope2[p] * alibi_distance<MASK>(col + k, ipos[p]);
-                v[c][k] = keep ? fmaf(v[c][k], a.scale, bias) : ninf;
-                mx = fmaxf(mx, v[c][k]);
-            }
-        }
-        mx = group_reduce<OpMax, G>(mx);
-        float sum = 0.f;
-#pragma unroll
-        for (int c = 0; c < C; ++c)
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                v[c][k] = fast_exp2(v[c][k] - mx);
-                sum += (kRag && k < back) ? 0.f : v[c][k];  // columns the lane before counts
-            }
-        if constexpr (MASK == Mask::Bytes) {
-            // rows with every key hidden (rare): uniform over the sk columns
-            const bool all_masked = (mx == ninf) && len[p] > 0;
-            if (__builtin_amdgcn_ballot_w64(all_masked) != 0) {
-                if (all_masked) {
-                    sum = 0.f;
-#pragma unroll
-                    for (int c = 0; c < C; ++c)
-#pragma unroll
-                        for (int k = 0; k < 8; ++k) {
-                            v[c][k] = ((col0 + c * kChunk + k) < len[p]) ? 1.f : 0.f;
-                            sum += (kRag && k < back) ? 0.f : v[c][k];
-                        }
-                }
-            }
-        }
-        sum = group_reduce<OpSum, G>(sum);
-        const float inv = 1.0f / sum;
-        const uint32_t lr = p * RPP + grp;
-        summed = summed && (lr >= rows_here || sum == sum);
-#pragma unroll
-        for (int c = 0; c < C; ++c) {
-            const int col = col0 + c * kChunk;
-#pragma unroll
-            for (int k = 0; k < 8; ++k) v[c][k] *= inv;  // lanes of absent rows hold NaN and store nothing
-            const bool st = lr < rows_here && col < sk;
-            const u32x4 o = pack8<T>(v[c]);
-            out.template put<kStNt>(o, (lr * sk + col) * 2u, st);
-            if constexpr ((FLAGS & kDropout) != 0) {
-                const uint32_t bits = keep_bits_row8<kRag>(drop, row0 + lr, sk, col);
-                out2.template put<kStNt>(dropout8<T>(o, bits, drop.scale), (lr * sk + col) * 2u, st);
-            }
-        }
-    }
+                                                 char* stage, char* stage2) {
+#include "softmax_fwd_rows.inl"
     return __builtin_amdgcn_ballot_w64(!summed) == 0;
 }
 
@@ -950,13 +818,18 @@ __device__ __forceinline__ void wave_outputs(const SoftmaxArgs& a, uint32_t row0
 template <typename T, int G, Mask MASK, int FLAGS = kDefaultFlags, int R = kPackedPasses, int C = 1>
 __global__ __launch_bounds__(256) void softmax_fwd_packed_kernel(SoftmaxArgs a) {
     constexpr int RPW = Packed<G, R>::kRowsPerWave;
+    const int lane = threadIdx.x & (kWave - 1);
     const uint32_t wave = xcd_slot(blockIdx.x, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), 4, a);
     const uint32_t row0 = wave * RPW;  // first row of this wave
     if (row0 >= a.rows) return;
     const uint32_t rows_here = min((uint32_t)RPW, a.rows - row0);
-    rsrc_t ry, ry2;
-    wave_outputs<FLAGS>(a, row0, rows_here, ry, ry2);
-    softmax_fwd_rows<T, G, MASK, FLAGS, R, C>(a, row0, rows_here, threadIdx.x & (kWave - 1), DirectSink{ry}, DirectSink{ry2});
+    if constexpr (MASK == Mask::Bytes && (FLAGS & kAlibi) == 0) {
+        softmax_fwd_rows<T, G, MASK, FLAGS, R, C, DirectSink>(a, row0, rows_here, lane, nullptr, nullptr);
+    } else {
+        typedef DirectSink Sink;
+        char *const stage = nullptr, *const stage2 = nullptr;
+#include "softmax_fwd_rows.inl"
+    }
 }
 
 // The number of leading keys that any of the causal rows row0 .. row0 + rows_here - 1 sees.
@@ -999,27 +872,27 @@ __global__ __launch_bounds__(256) void softmax_fwd_causal_packed_kernel(SoftmaxA
     const uint32_t row0 = xcd_slot(blockIdx.x, wib, 4, a) * RW;
     if (row0 >= a.rows) return;
     const uint32_t rows_here = min(RW, a.rows - row0), n = rows_here * a.sk;
-    const StagedSink s1{stage[wib]}, s2{stage[kDrp ? 4 + wib : wib]};
+    char *const s1 = stage[wib], *const s2 = stage[kDrp ? 4 + wib : wib];
     auto with_lanes = [&](auto g) {
         constexpr int G = decltype(g)::value;
         if constexpr (G < GMAX) {
-            clear_stage(s1.lds, n, lane);
-            if constexpr (kDrp) clear_stage(s2.lds, n, lane);
+            clear_stage(s1, n, lane);
+            if constexpr (kDrp) clear_stage(s2, n, lane);
         }
-        return softmax_fwd_rows<T, G, Mask::Causal, FLAGS, kPackedPasses * G / GMAX + (G * kPackedPasses < GMAX), 1>(
+        return softmax_fwd_rows<T, G, Mask::Causal, FLAGS, kPackedPasses * G / GMAX + (G * kPackedPasses < GMAX), 1, StagedSink>(
             a, row0, rows_here, lane, s1, s2);
     };
     // a row without a sum is NaN in its hidden columns too: all lanes, once more (nothing is stored yet)
     if (!with_lanes_for<GMAX>(keys_seen(row0, rows_here, a), with_lanes)) with_lanes(std::integral_constant<int, GMAX>{});
     rsrc_t ry, ry2;
     wave_outputs<FLAGS>(a, row0, rows_here, ry, ry2);
-    flush_staged<kStNt>(ry, s1.lds, n, lane);
-    if constexpr (kDrp) flush_staged<kStNt>(ry2, s2.lds, n, lane);
+    flush_staged<kStNt>(ry, s1, n, lane);
+    if constexpr (kDrp) flush_staged<kStNt>(ry2, s2, n, lane);
 }
 
 template <typename T, int G, Mask MASK, int FLAGS, int R, int C, typename Sink>
 __device__ __forceinline__ void softmax_bwd_rows(const SoftmaxArgs& a, uint32_t row0, uint32_t rows_here, int lane,
-                                                 const Sink& out) {
+                                                 char* stage) {
     static_assert(C == 1 || G == kWave, "several chunks per row need a whole wave per row");
     constexpr int RPP = Packed<G, R>::kRowsPerPass;
     constexpr bool kLdNt = (FLAGS & kNtLoad) != 0, kStNt = (FLAGS & kNtStore) != 0;
@@ -1034,6 +907,7 @@ __device__ __forceinline__ void softmax_bwd_rows(const SoftmaxArgs& a, uint32_t 
 
     const rsrc_t bg = make_rsrc(static_cast<const char*>(a.in0) + (size_t)row0 * sk * 2, rows_here * sk * 2);
     const rsrc_t by = make_rsrc(static_cast<const char*>(a.in1) + (size_t)row0 * sk * 2, rows_here * sk * 2);
+    const Sink out(a.out, (size_t)row0 * sk * 2, rows_here * sk * 2, stage);
 
     u32x4 rg[R][C], rp[R][C];
     int len[R];
@@ -1124,9 +998,7 @@ __global__ __launch_bounds__(256) void softmax_bwd_packed_kernel(SoftmaxArgs a) 
     const uint32_t row0 = wave * RPW;
     if (row0 >= a.rows) return;
     const uint32_t rows_here = min((uint32_t)RPW, a.rows - row0);
-    rsrc_t dx, dx2;
-    wave_outputs<0>(a, row0, rows_here, dx, dx2);
-    softmax_bwd_rows<T, G, MASK, FLAGS, R, C>(a, row0, rows_here, threadIdx.x & (kWave - 1), DirectSink{dx});
+    softmax_bwd_rows<T, G, MASK, FLAGS, R, C, DirectSink>(a, row0, rows_here, threadIdx.x & (kWave - 1), nullptr);
 }
 
 // The backward pass of softmax_fwd_causal_packed_kernel, with dropout.  (dx may alias dy: a wave's rows are read before they are stored.)
@@ -1139,16 +1011,16 @@ __global__ __launch_bounds__(256) void softmax_bwd_causal_packed_kernel(SoftmaxA
     const uint32_t row0 = xcd_slot(blockIdx.x, wib, 4, a) * RW;
     if (row0 >= a.rows) return;
     const uint32_t rows_here = min(RW, a.rows - row0), n = rows_here * a.sk;
-    const StagedSink s{stage[wib]};
+    char* const s = stage[wib];
     with_lanes_for<GMAX>(keys_seen(row0, rows_here, a), [&](auto g) {
         constexpr int G = decltype(g)::value;
-        if constexpr (G < GMAX) clear_stage(s.lds, n, lane);
-        softmax_bwd_rows<T, G, Mask::Causal, FLAGS, kPackedPasses * G / GMAX + (G * kPackedPasses < GMAX), 1>(
+        if constexpr (G < GMAX) clear_stage(s, n, lane);
+        softmax_bwd_rows<T, G, Mask::Causal, FLAGS, kPackedPasses * G / GMAX + (G * kPackedPasses < GMAX), 1, StagedSink>(
             a, row0, rows_here, lane, s);
     });
     rsrc_t dx, dx2;
     wave_outputs<0>(a, row0, rows_here, dx, dx2);
-    flush_staged<(FLAGS & kNtStore) != 0>(dx, s.lds, n, lane);
+    flush_staged<(FLAGS & kNtStore) != 0>(dx, s, n, lane);
 }
 
 // ---------------------------------------------------------------------------------
