@@ -131,28 +131,53 @@ static hipError_t launch_causal_packed(const SoftmaxArgs& a0, hipStream_t st) {
     return hipGetLastError();
 }
 
+// Whether causal rows of 65 to 447 columns go that way: those that fill less than three quarters of their lane group, with
+// dropout, whose Philox rounds the idle lanes compute too, up to seven eighths and in both passes, and enough rows of them.
+// The kernel's chain is longer by the zeroing, the staging and its bigger code, half a microsecond, which few rows do
+// not win back.  us per launch, fp16, softmax_*_packed_kernel -> softmax_*_causal_packed_kernel, timed from 2^11 to 2^18 rows:
+//   forward, 65-88 columns    aligned rows -6...+2 % throughout: never; ragged [504,65,65] 4.3 -> 4.4, [1008,65,65] 5.8 -> 5.5
+//     129-184                 [64,129,129] 4.0 -> 4.1, [127,129,129] 4.7 -> 4.6, [254,129,129] 6.5 -> 5.3, [46,177,177] 4.1 -> 4.2, [93,177,177] 5.4 -> 5.1
+//     257-376                 [7,281,281] 3.7 -> 4.0, [29,281,281] 4.7 -> 4.6, [58,281,281] 6.3 -> 5.6, [1020,257,257] 54 -> 44
+//   with dropout, 65-127      aligned [2731,96,96] 28.1 -> 27.0, -5...-15 % with fewer rows; ragged [504,65,65] 7.7 -> 7.9, [1008,65,65] 11.6 -> 10.1
+//     129-192                 [64,129,129] 7.4 -> 6.2, [57,144,144] 5.4 -> 5.4; ragged [46,177,177] 5.9 -> 6.4, [93,177,177] 9.5 -> 8.8; aligned
+//                             [341,192,192] 14.1 -> 16.2, [683,192,192] 26.9 -> 26.6
+//     193-216                 aligned -28...+3 % throughout: never; ragged [78,209,209] 7.7 -> 8.7, [157,209,209] 12.7 -> 12.2
+//     257-384                 [28,296,296] 7.2 -> 5.7, [11,376,376] 5.7 -> 5.3, ragged [7,281,281] 5.6 -> 6.1, [14,281,281] +16 %
+//     385-440                 aligned [20,400,400] 6.0 -> 6.6, [82,400,400] 16.3 -> 15.9; ragged [20,401,401] 7.8 -> 8.9, [41,401,401] 13.1 -> 12.4
+//   backward, with dropout    up to 192 and 384 columns -5...+92 % ([1020,257,257] 127 -> 66, [504,65,65] 8.0 -> 7.4); beyond, [78,209,209]
+//                             7.4 -> 8.0, [157,209,209] 11.7 -> 11.2, [20,401,401] 7.4 -> 8.0, [41,401,401] 12.0 -> 10.3, [20,400,400] 5.7 -> 5.7
+template <bool BWD, int EXTRA, int G>
+static bool causal_lanes_pay(const SoftmaxArgs& a, int lanes) {
+    constexpr bool rag = (EXTRA & kRagged) != 0;
+    if constexpr ((EXTRA & kDropout) == 0) {
+        if (lanes * 4 >= G * 3) return false;
+        if (G == 16) return rag && a.rows >= 1u << 16;
+        return a.rows >= (G == 32 ? 1u << 14 : 1u << 13);
+    }
+    if (G == 16) return a.sk != G * kVec && (BWD || a.rows >= (rag ? 1u << 16 : 3u << 16));
+    if (lanes * 8 >= G * 7) return false;
+    if (lanes * 4 > G * 3) {
+        if (G == 32) return rag && a.rows >= 1u << 15;
+        return a.rows >= (rag ? 1u << 14 : BWD ? 1u << 13 : 1u << 15);
+    }
+    if (BWD) return true;
+    if (G == 64) return a.rows >= (rag ? 1u << 12 : 1u << 13);
+    if (lanes * 8 <= G * 5) return a.rows >= (rag ? 1u << 13 : 1u << 14);
+    return a.rows >= (rag ? 1u << 14 : 1u << 17);
+}
+
 template <typename T, Mask M, bool BWD, int EXTRA, int G>
 static hipError_t launch_packed(const SoftmaxArgs& a, hipStream_t st) {
     const int lanes = (a.sk + kVec - 1) / kVec;
     if constexpr (M == Mask::Causal && G >= 16 && (!BWD || (EXTRA & kDropout) != 0)) {
-        // Causal rows that fill less than three quarters of their lane group: as many lanes as the rows see keys,
-        // results staged.  us per launch, bf16, against the kernels below: [2000,161,161] 36.9 -> 34.3, [2000,177,177]
-        // 42.4 -> 40.4, [800,336,336] 55.6 -> 50.8, [4000,80,80] 19.3 -> 19.0; fuller rows lose: [2000,192,192] 42.2 -> 42.9,
-        // [2000,193,193] 46.0 -> 49.7, [400,511,511] 61 -> 69, and so does the plain backward pass at most lengths ([4000,129,129]
-        // 65.7 -> 66.6, [600,384,384] 66.7 -> 68.0).  With dropout, whose Philox rounds the idle lanes computed too, it pays in
-        // both passes up to seven eighths, and to the end of 128 columns (fp16, forward and backward: [600,385,385]
-        // 128 -> 105 and 112 -> 85, [4000,127,127] 84.5 -> 71.5 and 69.8 -> 65.3; [1000,224,224] 47.3 -> 48.3 and 41.8 -> 43.2).
-        const bool pays = (EXTRA & kDropout) != 0 ? (lanes * 8 < G * 7 || (G == 16 && a.sk != G * kVec)) : lanes * 4 < G * 3;
-        if (pays) return launch_causal_packed<T, BWD, EXTRA, G>(a, st);
+        if (causal_lanes_pay<BWD, EXTRA, G>(a, lanes)) return launch_causal_packed<T, BWD, EXTRA, G>(a, st);
     }
     // passes per wave: 4, except for lane groups of 32 and 64 lanes in the causal kernels and the
     // full-row backward, which run faster with 2 when the rows fill their lane groups (causal forward
     // 15 %, causal backward up to 11 % at 512 columns, full-row backward 0-4 %).  With a quarter or
-    // more of the lanes idle 4 passes are faster there too (full-row and causal backward passes at 129-192 and
-    // 257-384 columns; causal forward at the end of those ranges, whose fuller rows are all that is left to it).
+    // more of the lanes idle (129-192 and 257-384 columns) 4 passes are 4-12 % faster there too.
     constexpr int R = (M != Mask::Bytes && G >= 32) ? 2 : kPackedPasses;
-    // (causal rows with dropout that leave so many idle have gone above)
-    if constexpr (R != kPackedPasses && !(M == Mask::Causal && (EXTRA & kDropout) != 0)) {
+    if constexpr (R != kPackedPasses) {
         if (lanes * 4 <= G * 3) return launch_packed_shape<T, M, BWD, EXTRA, G, kPackedPasses, 1>(a, st);
     }
     return launch_packed_shape<T, M, BWD, EXTRA, G, R, 1>(a, st);

@@ -1687,3 +1687,56 @@ def test_two_causal_rows_per_block(device, np_, sq, sk, slopes, with_bias, p, dt
     assert max_err(y[0, 1], R.softmax_fp32(total, hidden, 0.125)) <= TOL[dtype] and (y[..., hidden] == 0).all()
     if not p:
         assert max_err(dx[0, 1], R.softmax_backward_fp32(g[0, 1], y[0, 1], 0.125)) <= TOL[dtype] and (dx[..., hidden] == 0).all()
+
+
+def same(a, b):
+    """Equal bit for bit, NaN for NaN."""
+    return torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(0.0, posinf=9.0, neginf=-9.0), b.nan_to_num(0.0, posinf=9.0, neginf=-9.0))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("slopes,with_bias,p", [(s, b, p) for s in (False, True) for b in (False, True) for p in (0.0, 0.25)])
+@pytest.mark.parametrize("np_,s", [
+    (1010, 65), (760, 87),                       # lane groups of 16 lanes
+    (2050, 96), (1640, 120), (520, 127),         # ... with dropout only
+    (130, 129), (122, 136), (95, 175),           # 32 lanes, up to three quarters of them
+    (685, 192), (160, 209),                      # ... beyond that, with dropout only
+    (40, 257), (32, 264), (22, 376),             # 64 lanes
+    (42, 401), (76, 440),                        # ... with dropout only
+])
+def test_many_short_causal_rows_against_few(device, np_, s, slopes, with_bias, p, dtype):
+    # enough rows for as many lanes as they see keys, against the same matrices a few at a time, which keep whole
+    # lane groups: the same sums, the same bits -- also of rows without a sum (a score that is NaN or +inf, no score above -inf)
+    x = scores((1, np_, s, s), dtype, device, s)
+    g = torch.Generator(device=device).manual_seed(s)
+    for value in (float("nan"), float("inf")):
+        rows = torch.randint(0, np_ * s, (5,), device=device, generator=g)
+        x.view(-1, s)[rows, (rows % s) // 2] = value
+    rows = torch.randint(0, np_ * s, (5,), device=device, generator=g)
+    x.view(-1, s)[rows] = float("-inf")
+    x[0, 0, 0, 0] = x[0, -1, -1, -1] = float("inf")  # the tensor's first and last row
+    bias = normal((1, np_, s, s), dtype, device, s + 2) if with_bias else None
+    sl = torch.linspace(1.0, 0.1, np_, device=device) if slopes else None
+
+    def probs(x, sl, bias):
+        if bias is not None:
+            return causal_ext.forward_bias(x, bias, 0.125, sl)
+        return causal_ext.forward_nd(x, 0.125) if sl is None else causal_ext.forward_alibi(x, sl, 0.125)
+
+    step = max(1, 2000 // s)
+    parts = [slice(m, m + step) for m in range(0, np_, step)]
+    few = torch.cat([probs(x[:, m], None if sl is None else sl[m], None if bias is None else bias[:, m]) for m in parts], 1)
+    if p:
+        y, dropped = causal_ext.forward_dropout(x, 0.125, p, 9, 4, slopes=sl, bias=bias)
+        keep = rng_keep(y.numel(), p, 9, 4, device).view(y.shape)
+        assert same(dropped, R.dropout_with_mask(y, keep, p))
+        clean = y.nan_to_num(0.0)
+        dy = normal((1, np_, s, s), dtype, device, s + 3)
+        dx = causal_ext.backward_dropout(dy.clone(), clean, 0.125, p, 9, 4)
+        want = R.softmax_backward_fp32(dy.float() * keep / (1 - p), clean, 0.125)
+        assert max_err(dx, want) <= TOL[dtype] * max(1.0, want.abs().max().item())
+        assert (dx[..., torch.ones(s, s, dtype=torch.bool, device=device).triu_(1)] == 0).all()
+    else:
+        y = probs(x, sl, bias)
+    assert same(y, few)
+    assert y.isnan().view(-1, s).any(-1).sum() >= 10 and (y.isnan().view(-1, s).all(-1) == y.isnan().view(-1, s).any(-1)).all()
