@@ -200,9 +200,22 @@ void save_tables(AutogradContext* ctx, const Tables& t) {
     ctx->saved_data["d_rot"] = t.d_rot;
     ctx->saved_data["offset"] = t.offset;
 }
-Tables saved_tables(AutogradContext* ctx) {
+// The saved tables, for a gradient g [s, ..]: a saved-tensor hook may have given back another tensor than the forward
+// pass left with it, so everything the kernel takes for granted is looked at again.
+Tables saved_tables(AutogradContext* ctx, const Tensor& g) {
     variable_list v = ctx->get_saved_variables();
-    return {v[0], v.size() > 1 ? v[1] : Tensor(), ctx->saved_data["d_rot"].toInt(), ctx->saved_data["offset"].toInt()};
+    const int64_t d_rot = ctx->saved_data["d_rot"].toInt(), offset = ctx->saved_data["offset"].toInt();
+    for (Tensor& t : v) {
+        if (!on_gpu(t) || t.device() != g.device())
+            throw std::runtime_error("the saved cos/sin tables or angles must be on the device of the gradient");
+        if (t.dim() != 4 || t.size(1) != 1 || t.size(2) != 1 || t.size(3) != d_rot || t.size(0) < offset + g.size(0))
+            throw std::runtime_error("the saved cos/sin tables or angles have another shape than in the forward pass");
+        if (t.scalar_type() != v[0].scalar_type() ||
+            (t.scalar_type() != at::kFloat && (v.size() == 1 || t.scalar_type() != g.scalar_type())))
+            throw std::runtime_error("the saved cos/sin tables must be float32 or have the dtype of the gradient, angles float32");
+        t = t.contiguous();
+    }
+    return {v[0], v.size() > 1 ? v[1] : Tensor(), d_rot, offset};
 }
 Tensor dense_last(const Tensor& t) { return t.stride(-1) == 1 ? t : t.contiguous(); }
 
@@ -221,7 +234,7 @@ public:
         return {oq, ok};
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
-        auto [dq, dk] = rotary_pair(dense_last(grads[0]), dense_last(grads[1]), saved_tables(ctx), true);
+        auto [dq, dk] = rotary_pair(dense_last(grads[0]), dense_last(grads[1]), saved_tables(ctx, grads[0]), true);
         return {dq, dk, Tensor()};
     }
 };
@@ -242,7 +255,7 @@ public:
         return rope_whole(x, t, transposed, false);
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
-        return {rope_whole(dense_last(grads[0]), saved_tables(ctx), ctx->saved_data["transposed"].toBool(), true), Tensor(),
+        return {rope_whole(dense_last(grads[0]), saved_tables(ctx, grads[0]), ctx->saved_data["transposed"].toBool(), true), Tensor(),
                 Tensor()};
     }
 };

@@ -147,6 +147,18 @@ def _as_table(t, d_rot, need_rows):
     return t2
 
 
+def _saved_tables(ctx, grad, d_rot):
+    """The tables that an autograd Function saved, for the gradient ``grad``: a saved-tensor hook may have given back
+    other tensors than it was given, so what the kernel takes for granted is looked at again."""
+    cos, sin = ctx.saved_tensors
+    if cos.device != grad.device or sin.device != grad.device:
+        raise RuntimeError("the saved cos/sin tables must be on the device of the gradient")
+    if cos.dtype != sin.dtype or cos.dtype not in (torch.float32, grad.dtype):
+        raise RuntimeError("the saved cos/sin tables must be float32 or have the dtype of the gradient")
+    rows = ctx.offset + grad.shape[0]
+    return _as_table(cos, d_rot, rows), _as_table(sin, d_rot, rows)
+
+
 def _dense_last(t):
     return t if t.stride(-1) == 1 else t.contiguous()
 
@@ -190,7 +202,7 @@ class _FusedRotary(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_q, grad_k):
-        cos2, sin2 = ctx.saved_tensors
+        cos2, sin2 = _saved_tables(ctx, grad_q, grad_q.shape[-1])
         grad_q, grad_k = _dense_last(grad_q), _dense_last(grad_k)
         dq = torch.empty(grad_q.shape, dtype=grad_q.dtype, device=grad_q.device)
         dk = torch.empty(grad_k.shape, dtype=grad_k.dtype, device=grad_k.device)
@@ -276,7 +288,7 @@ class _FusedRotaryInplace(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_q, grad_k):
-        cos2, sin2 = ctx.saved_tensors
+        cos2, sin2 = _saved_tables(ctx, grad_q, ctx.d_rot)
         dq, dk = grad_q.clone(), grad_k.clone()
         dq, dk = _dense_last(dq), _dense_last(dk)
         if dq.numel() or dk.numel():
@@ -322,7 +334,7 @@ class _FusedQKVRotary(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_mixed):
-        cos2, sin2 = ctx.saved_tensors
+        cos2, sin2 = _saved_tables(ctx, grad_mixed, ctx.d_rot)
         dm = grad_mixed.clone(memory_format=torch.contiguous_format)  # v and pass-through dims: identity
         if dm.numel():
             dq, dk = dm[..., : ctx.hn], dm[..., ctx.hn : 2 * ctx.hn]

@@ -205,6 +205,39 @@ def test_exceptions_of_saved_tensor_hooks_and_activation_checkpointing(device):
 
 
 @gpu
+@pytest.mark.parametrize("native", [True, False])
+def test_tables_that_a_saved_tensor_hook_gives_back(device, monkeypatch, native):
+    # whatever the hook returns is checked on the host again before a kernel reads it
+    if not native:
+        monkeypatch.setattr(_lib, "calls", lambda *tensors: None)
+    q = torch.randn(4, 1, 2, 16, device=device).half().requires_grad_(True)
+    mixed = torch.randn(4, 1, 2, 48, device=device).half().requires_grad_(True)
+    cos, sin = torch.randn(2, 6, 1, 1, 16, device=device)
+    forward = [
+        lambda: apply_rotary_pos_emb(q, q, cos, sin, 2)[0],
+        lambda: apply_rotary_pos_emb_(q * 1, q * 1, cos, sin, 2)[0],
+        lambda: apply_rotary_pos_emb_qkv_(mixed * 1, cos, sin, 2)[0],
+        lambda: fused_rope.fused_apply_rotary_pos_emb(q, cos[:4]),
+        lambda: fused_rope.fused_apply_rotary_pos_emb_cached(q, cos[:4], sin[:4]),
+    ]
+
+    def gradient(call, unpack):
+        leaf = mixed if call is forward[2] else q
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: unpack(t) if t.dtype == torch.float32 else t):
+            y = call()
+        g = torch.ones_like(y)
+        return torch.autograd.grad(y, leaf, g)[0]
+
+    for call in forward:
+        want = gradient(call, lambda t: t)
+        # the same values in another layout
+        assert torch.equal(gradient(call, lambda t: t.transpose(0, -1).contiguous().transpose(0, -1)), want)
+        for unpack in (lambda t: t.cpu(), lambda t: t.double(), lambda t: t[:-1], lambda t: t.flatten()):
+            with pytest.raises(RuntimeError):
+                gradient(call, unpack)
+
+
+@gpu
 def test_forward_mode_derivatives_are_refused(device):
     # no kernel computes a tangent: an error, and not a result whose derivative has become zero
     t = torch.randn(4, 1, 2, 16, device=device).half()
