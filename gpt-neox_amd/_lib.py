@@ -9,8 +9,10 @@ import ctypes
 import importlib.machinery
 import importlib.util
 import os
+import re
 import subprocess
 import threading
+import warnings
 
 import torch
 from torch.autograd import forward_ad
@@ -97,6 +99,7 @@ SIGNATURES = {
 _lock = threading.Lock()
 _lib = None
 _calls = None
+_calls_missing = False  # neox_torch.so was looked for and cannot be used
 _PLAIN_TENSORS = (torch.Tensor, torch.nn.Parameter)
 
 
@@ -145,7 +148,8 @@ def lib():
 
 
 def load_calls():
-    """Return the module of native calls, loading it on first use; ``ImportError`` if it is missing."""
+    """Return the module of native calls, loading it on first use; ``ImportError`` if it is missing or was built
+    against another library or another torch than those it is loaded into."""
     global _calls
     lib()  # the library behind them, with its checks
     with _lock:
@@ -155,6 +159,9 @@ def load_calls():
             loader = importlib.machinery.ExtensionFileLoader("neox_torch", CALLS_PATH)
             module = importlib.util.module_from_spec(importlib.util.spec_from_loader("neox_torch", loader))
             loader.exec_module(module)
+            got, want = (module.abi_version, module.torch_version), (ABI_VERSION, re.match(r"[\d.]*\d", torch.__version__)[0])
+            if got != want:
+                raise ImportError(f"{CALLS_PATH}: built for ABI version and torch {got}, expected {want}: build it again")
             _calls = module
     return _calls
 
@@ -162,7 +169,7 @@ def load_calls():
 def calls(*tensors):
     """The native calls of ``csrc/torch_calls.cpp`` if they may serve a call on ``tensors``, else None: tensors
     that are not on the GPU, tensor subclasses, and whatever records or rewrites Python operations (``torch.compile``, ``torch.jit.trace``),
-    keep the autograd Functions of the modules."""
+    keep the autograd Functions of the modules.  So does everything where ``neox_torch.so`` cannot be loaded."""
     if torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None:
         return None
     for t in tensors:
@@ -170,7 +177,22 @@ def calls(*tensors):
             return None
     if not tensors[0].is_cuda:
         return None
-    return _calls if _calls is not None else load_calls()
+    return _calls if _calls is not None else find_calls()
+
+
+def find_calls():
+    """:func:`load_calls`, or None where the module cannot be loaded: the general path serves every call then, with the
+    same kernels through ctypes and more time on the host, which a warning says once."""
+    global _calls_missing
+    lib()
+    if _calls_missing:
+        return None
+    try:
+        return load_calls()
+    except ImportError as exc:
+        _calls_missing = True
+        warnings.warn(f"the native calls cannot be used, calls go through ctypes: {exc}", RuntimeWarning, stacklevel=3)
+        return None
 
 
 def carries_tangent(*tensors):

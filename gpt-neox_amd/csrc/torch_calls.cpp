@@ -7,6 +7,7 @@
 // checks and messages.  The kernels are those of include/neox_fused.h.  Nothing is kept between calls: what a
 // backward pass needs is saved through autograd, under its version checks and saved-tensor hooks.
 #include <torch/extension.h>
+#include <torch/version.h>
 
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
@@ -314,6 +315,8 @@ std::optional<Tensor> rope(const Tensor& x, const Tensor& cos, const std::option
 PYBIND11_MODULE(neox_torch, m) {
     namespace py = pybind11;
     using torch::wrap_pybind_function_no_gil;
+    m.attr("abi_version") = NEOX_FUSED_ABI_VERSION;  // what this was compiled against, for the loader to compare
+    m.attr("torch_version") = TORCH_VERSION;
     m.def("causal_softmax", wrap_pybind_function_no_gil(causal_softmax), py::arg("x"), py::arg("scale"), py::arg("window") = -1,
           py::arg("slopes") = std::optional<Tensor>(), py::arg("p") = 0.0, py::arg("seed") = 0, py::arg("offset") = 0);
     m.def("causal_takes", wrap_pybind_function_no_gil(causal_takes), py::arg("x"), py::arg("slopes") = std::optional<Tensor>());

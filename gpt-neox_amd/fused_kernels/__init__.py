@@ -30,7 +30,7 @@ def load(neox_args=None):
     ``neox_args`` is accepted for signature compatibility; its
     ``fused_kernels_build_path`` is not used because the library lives next to its sources.
     """
-    if not (os.path.exists(_lib.LIB_PATH) and os.path.exists(_lib.CALLS_PATH)):
+    if not os.path.exists(_lib.LIB_PATH):
         rank = getattr(neox_args, "rank", 0) if neox_args is not None else 0
         if rank == 0:
             _lib.build()
@@ -42,7 +42,8 @@ def load(neox_args=None):
 
 def load_fused_kernels():
     """Check that the kernels are usable; register the extension-named modules."""
-    _lib.load_calls()  # ImportError if the library or the module of native calls is absent or broken
+    _lib.lib()  # ImportError if the library is absent or broken
+    _lib.find_calls()  # (and a warning if the module of native calls is)
     from . import fused_rotary_positional_embedding as rope
     from . import scaled_masked_softmax_cuda as masked
     from . import scaled_upper_triang_masked_softmax_cuda as causal

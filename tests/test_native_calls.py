@@ -7,6 +7,7 @@ import torch.utils.checkpoint
 from torch.autograd import forward_ad
 
 from gpt_neox_amd import _lib, fused_rope
+from gpt_neox_amd.fused_kernels import load, load_fused_kernels
 from gpt_neox_amd.fused_softmax import FusedScaleMaskSoftmax, SoftmaxFusionTypes
 from gpt_neox_amd.positional_embeddings import (AliBi, apply_rotary_pos_emb, apply_rotary_pos_emb_,
                                                 apply_rotary_pos_emb_qkv_)
@@ -355,4 +356,53 @@ def test_missing_native_calls_raise_import_error(monkeypatch):
     monkeypatch.setattr(_lib, "_calls", None)
     monkeypatch.setattr(_lib, "CALLS_PATH", "/nonexistent/neox_torch.so")
     with pytest.raises(ImportError, match="neox_torch.so"):
+        _lib.load_calls()
+
+
+@pytest.fixture
+def without_native_calls(monkeypatch):
+    """A tree in which only libneox_fused.so was built."""
+    monkeypatch.setattr(_lib, "_calls", None)
+    monkeypatch.setattr(_lib, "_calls_missing", False)
+    monkeypatch.setattr(_lib, "CALLS_PATH", "/nonexistent/neox_torch.so")
+
+
+def test_the_library_alone_is_enough_to_load(without_native_calls, monkeypatch):
+    with pytest.warns(RuntimeWarning, match="neox_torch.so"):
+        load_fused_kernels()
+    load_fused_kernels()  # (said once)
+    built = []
+    monkeypatch.setattr(_lib, "build", lambda *args, **kwargs: built.append(args))
+    load()
+    assert _lib.find_calls() is None and not built
+
+
+@gpu
+def test_the_library_alone_serves_every_call(device, without_native_calls):
+    x = torch.randn(2, 2, 40, 40, device=device).half().requires_grad_(True)
+    with pytest.warns(RuntimeWarning, match="neox_torch.so"):
+        mod = module(torch.float16, SoftmaxFusionTypes.upper_triang)
+    mask = causal_mask(40, device)
+    y = mod(x, mask)
+    assert type(y.grad_fn).__name__ == "_CausalSoftmax4DBackward"
+    want = torch.softmax((x.detach().float() * 0.125).masked_fill(mask, float("-inf")), -1)
+    assert (y.float() - want).abs().max() <= 1e-3
+    q, freqs = torch.randn(4, 1, 2, 16, device=device).half(), torch.randn(4, 1, 1, 16, device=device)
+    assert torch.equal(apply_rotary_pos_emb(q, q, freqs.cos(), freqs.sin())[1],
+                       fused_rope.fused_apply_rotary_pos_emb_cached(q, freqs.cos(), freqs.sin()))
+
+
+@pytest.mark.parametrize("attr,value", [("abi_version", 3), ("torch_version", "1.0.0")])
+def test_native_calls_of_another_build_are_not_used(monkeypatch, attr, value):
+    real = _lib.importlib.util.module_from_spec
+
+    def other(spec):
+        module = real(spec)
+        exec_module = spec.loader.exec_module
+        monkeypatch.setattr(spec.loader, "exec_module", lambda m: (exec_module(m), setattr(m, attr, value)), raising=False)
+        return module
+
+    monkeypatch.setattr(_lib, "_calls", None)
+    monkeypatch.setattr(_lib.importlib.util, "module_from_spec", other)
+    with pytest.raises(ImportError, match="build it again"):
         _lib.load_calls()
