@@ -2,9 +2,10 @@
 // out of place, over the first d_rot dims of [s, b, h, d] tensors with arbitrary
 // s/b/h strides (the inputs are usually views into a fused QKV buffer).
 //
-// One block serves one sequence position: the position's cos/sin values are loaded
-// once into registers and reused for every head of q and k.  Two kernels (two more, for dense
-// tensors that are taken as one run of memory, are described where they stand):
+// Five kernels.  In the first two one block serves one sequence position: the position's cos/sin
+// values are loaded once into registers and reused for every head of q and k.  rope_piece_kernel,
+// rope_run_kernel and rope_cell_kernel take dense tensors as one run of memory, in 4 KiB pieces; they are
+// described where they stand.
 //
 // * rope_span_kernel -- the rotated span splits into at most 64 slots of W = 8, 4 or 2 dims
 //   (the widest the alignment of the layouts and of d_rot/2 allows).  Each lane owns ONE
@@ -17,7 +18,7 @@
 //   rotated span; the thread also owns the matching W dims of the second half, so no data
 //   crosses lanes (W = 8, 4, 2, 1).
 //
-// In both, a lane reads everything it needs before it writes, and a pair
+// In these two, a lane reads everything it needs before it writes, and a pair
 // (j, j + d_rot/2) is written by the lane(s) that read it, so in-place operation is
 // race-free.  q/k accesses carry the non-temporal hint (each byte is touched once).
 //
@@ -609,7 +610,7 @@ __global__ __launch_bounds__(256) void rope_run_kernel(RopeRunArgs a) {
 #pragma unroll
         for (int g = 0; g < kVec / PW; ++g) {
             const int e = j[it] + g * PW;
-            const uint32_t off = e < d_rot ? v * vec_bytes + (uint32_t)(e < half ? e + half : e - half) * 2u : kNoAccess;
+            const uint32_t off = e < d_rot ? v * vec_bytes + (uint32_t)(e < half ? e + half : e - half) * 2u : kOutOfRange;
             if constexpr (PW == 8) {
                 const u32x4 w = buf_ld128<false>(rx, off, 0);
                 xp[it][0] = w.x, xp[it][1] = w.y, xp[it][2] = w.z, xp[it][3] = w.w;
@@ -703,7 +704,7 @@ __global__ __launch_bounds__(256) void rope_cell_kernel(RopeCellArgs a) {
     for (int it = 0; it < ITERS; ++it) {
         const uint32_t part = a.by_part.div(slot0 + it * kWave + lane);
         const uint32_t kind = part % 3u;  // q, k or v
-        off[it] = (kind < 2 && slot < a.moved) ? (uint32_t)(it * kWave + lane) * 16 : kNoAccess;
+        off[it] = (kind < 2 && slot < a.moved) ? (uint32_t)(it * kWave + lane) * 16 : kOutOfRange;
         x[it] = buf_ld128<true>(r, off[it], 0);
     }
     const bool rotated = slot < a.lps, second = slot >= hl;

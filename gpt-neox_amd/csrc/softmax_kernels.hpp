@@ -97,7 +97,6 @@ constexpr int kRagged = 32;
 // computed (wave-uniform branch), like those above the diagonal; their zeros are still stored.
 constexpr int kBand = 64;
 constexpr int kDefaultFlags = kNtLoad | kNtStore;
-constexpr uint32_t kOutOfRange = 0xFFFFFFFFu;  // a byte offset no buffer contains
 
 // kRagged: 1 if the row starts on an odd element (2 mod 4 bytes) of the tensor at `base` and sk is
 // odd, so that rows alternate between the two alignments.  (With an even sk every row has the
@@ -791,10 +790,10 @@ __device__ __forceinline__ void flush_staged(rsrc_t out, const char* lds, uint32
 #pragma unroll
     for (uint32_t e0 = 0; e0 < kStageBytes / 2; e0 += kChunk) {
         const uint32_t e = e0 + lane * kVec;
-        if (e0 < whole) buf_st128<NT>(out, *reinterpret_cast<const u32x4*>(lds + e * 2), e < whole ? e * 2 : kNoAccess, 0);
+        if (e0 < whole) buf_st128<NT>(out, *reinterpret_cast<const u32x4*>(lds + e * 2), e < whole ? e * 2 : kOutOfRange, 0);
     }
     if (whole != n) buf_st16(out, *reinterpret_cast<const uint16_t*>(lds + (whole + lane) % (kStageBytes / 2) * 2),
-                             lane < (int)(n - whole) ? (whole + lane) * 2 : kNoAccess);
+                             lane < (int)(n - whole) ? (whole + lane) * 2 : kOutOfRange);
 }
 
 // The rows row0 .. row0 + rows_here - 1 of one wave.  Causal rows may be given fewer lanes than they have

@@ -130,7 +130,7 @@ struct FastDiv {
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 constexpr int kRsrcFlags = 0x00020000;  // raw buffer, 32-bit data format (gfx9 family)
 constexpr int kAuxNt = 2;               // non-temporal hint
-constexpr uint32_t kNoAccess = 0xFFFFFFFFu;  // a byte offset no buffer contains
+constexpr uint32_t kOutOfRange = 0xFFFFFFFFu;  // a byte offset no buffer contains
 
 __device__ __forceinline__ rsrc_t make_rsrc(const void* base, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)bytes, kRsrcFlags);
