@@ -16,10 +16,10 @@
     const float ninf = -__builtin_inff();
 
     const rsrc_t rx = make_rsrc(static_cast<const char*>(a.in0) + (size_t)row0 * sk * 2, rows_here * sk * 2);
-    const Sink out(a.out, (size_t)row0 * sk * 2, rows_here * sk * 2, stage);
+    const Sink out = Sink::at(a.out, (size_t)row0 * sk * 2, rows_here * sk * 2, stage);
     const rsrc_t rm = make_rsrc(a.mask, a.mask_bytes);
     Sink out2 = out;
-    if constexpr ((FLAGS & kDropout) != 0) out2 = Sink(a.out2, (size_t)row0 * sk * 2, rows_here * sk * 2, stage2);
+    if constexpr ((FLAGS & kDropout) != 0) out2 = Sink::at(a.out2, (size_t)row0 * sk * 2, rows_here * sk * 2, stage2);
     const rsrc_t rb = make_rsrc(a.bias, a.bias_bytes);  // kBias: the whole bias tensor
 
     bool summed = true;
