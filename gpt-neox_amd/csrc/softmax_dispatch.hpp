@@ -135,9 +135,11 @@ static hipError_t launch_causal_packed(const SoftmaxArgs& a0, hipStream_t st) {
 // dropout, whose Philox rounds the idle lanes compute too, up to seven eighths and in both passes, and enough rows of them.
 // The kernel's chain is longer by the zeroing, the staging and its bigger code, half a microsecond, which few rows do
 // not win back.  us per launch, fp16, softmax_*_packed_kernel -> softmax_*_causal_packed_kernel, timed from 2^11 to 2^18 rows:
-//   forward, 65-88 columns    aligned rows -6...+2 % throughout: never; ragged [504,65,65] 4.3 -> 4.4, [1008,65,65] 5.8 -> 5.5
+//   forward, 65-88 columns    aligned rows -6...+2 % up to 2^17, [3640,72,72] level, with ALiBi 16.8 -> 15.4; ragged [504,65,65] 4.3 -> 4.4,
+//                             [1008,65,65] 5.8 -> 5.5
 //     129-184                 [64,129,129] 4.0 -> 4.1, [127,129,129] 4.7 -> 4.6, [254,129,129] 6.5 -> 5.3, [46,177,177] 4.1 -> 4.2, [93,177,177] 5.4 -> 5.1
-//     257-376                 [7,281,281] 3.7 -> 4.0, [29,281,281] 4.7 -> 4.6, [58,281,281] 6.3 -> 5.6, [1020,257,257] 54 -> 44
+//     257-376                 [7,281,281] 3.7 -> 4.0, [29,281,281] 4.7 -> 4.6, [58,281,281] 6.3 -> 5.6, [1020,257,257] 54 -> 44; aligned
+//                             [28,296,296] 4.8 -> 4.1, [14,296,296] +2 %, [14,304,304] -3 %
 //   with dropout, 65-127      aligned [2731,96,96] 28.1 -> 27.0, -5...-15 % with fewer rows; ragged [504,65,65] 7.7 -> 7.9, [1008,65,65] 11.6 -> 10.1
 //     129-192                 [64,129,129] 7.4 -> 6.2, [57,144,144] 5.4 -> 5.4; ragged [46,177,177] 5.9 -> 6.4, [93,177,177] 9.5 -> 8.8; aligned
 //                             [341,192,192] 14.1 -> 16.2, [683,192,192] 26.9 -> 26.6
@@ -151,8 +153,9 @@ static bool causal_lanes_pay(const SoftmaxArgs& a, int lanes) {
     constexpr bool rag = (EXTRA & kRagged) != 0;
     if constexpr ((EXTRA & kDropout) == 0) {
         if (lanes * 4 >= G * 3) return false;
-        if (G == 16) return rag && a.rows >= 1u << 16;
-        return a.rows >= (G == 32 ? 1u << 14 : 1u << 13);
+        if (G == 16) return a.rows >= (rag ? 1u << 16 : 3u << 16);
+        if (G == 32) return a.rows >= 1u << 14;
+        return a.rows >= (rag ? 1u << 12 : lanes * 8 <= G * 5 ? 3u << 11 : 1u << 13);
     }
     if (G == 16) return a.sk != G * kVec && (BWD || a.rows >= (rag ? 1u << 16 : 3u << 16));
     if (lanes * 8 >= G * 7) return false;

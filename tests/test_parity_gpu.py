@@ -1697,7 +1697,7 @@ def same(a, b):
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("slopes,with_bias,p", [(s, b, p) for s in (False, True) for b in (False, True) for p in (0.0, 0.25)])
 @pytest.mark.parametrize("np_,s", [
-    (1010, 65), (760, 87),                       # lane groups of 16 lanes
+    (1010, 65), (760, 87), (2740, 72),           # lane groups of 16 lanes
     (2050, 96), (1640, 120), (520, 127),         # ... with dropout only
     (130, 129), (122, 136), (95, 175),           # 32 lanes, up to three quarters of them
     (685, 192), (160, 209),                      # ... beyond that, with dropout only
