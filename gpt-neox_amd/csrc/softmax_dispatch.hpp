@@ -180,7 +180,8 @@ static hipError_t launch_packed(const SoftmaxArgs& a, hipStream_t st) {
     // 15 %, causal backward up to 11 % at 512 columns, full-row backward 0-4 %).  With a quarter or
     // more of the lanes idle (129-192 and 257-384 columns) 4 passes are 4-12 % faster there too.
     constexpr int R = (M != Mask::Bytes && G >= 32) ? 2 : kPackedPasses;
-    if constexpr (R != kPackedPasses) {
+    // (the dropout backward of causal rows that leave so many idle has gone above, see causal_lanes_pay)
+    if constexpr (R != kPackedPasses && !(BWD && M == Mask::Causal && (EXTRA & kDropout) != 0)) {
         if (lanes * 4 <= G * 3) return launch_packed_shape<T, M, BWD, EXTRA, G, kPackedPasses, 1>(a, st);
     }
     return launch_packed_shape<T, M, BWD, EXTRA, G, R, 1>(a, st);
