@@ -521,7 +521,8 @@ __global__ __launch_bounds__(256) void rope_piece_kernel(RopeArgs a) {
 // from the lines its wave has just asked for (PW dims per access: the widest the half span allows), and
 // pass-through dims fetch no partner.  The cos and the signed sin values of the few positions a piece
 // touches are laid out in LDS by the wave itself while its loads are in flight -- sin already at the dim it
-// multiplies --, so that there is no barrier.  Bound by memory: [2048,2,64,96] fp16, first 24 dims, angles,
+// multiplies --, so that there is no barrier.  Bound by memory (counters at [2048,2,64,96] fp16,
+// 50.3 MB in and out: 53.1 fetched, the partners come from L2, 50.3 written): with angles of 24 dims,
 // 27.7 us (3.6 TB/s) in rope_span_kernel, which also evaluated its block's angles before it asked for the first
 // head, -> 18.6 us (5.4 TB/s).  A whole piece per wave leaves too few waves for an even last round: 19.0 us, and
 // [4096,1,4,64] first 64 dims 5.5 against 4.0; a quarter 19.7.  Partners fetched with the non-temporal hint come
@@ -668,7 +669,7 @@ __global__ __launch_bounds__(256) void rope_run_kernel(RopeRunArgs a) {
 // nothing, and every XCD keeps to its own pieces.  A part lies within one access, so a lane's partner dims come
 // through a wave shuffle, and a lane has the same dims of a part in both accesses: its cos and sin values are
 // loaded once.  Bound by memory: [8192,1,32,3*128] bf16, 52.5 us (5.1 TB/s) in rope_span_kernel, whose block
-// stores the six pieces of a position, -> 47.1 us (5.7 TB/s).
+// stores the six pieces of a position, -> 47.1 us (5.7 TB/s; 6.8 by the counters, 50 MB of it the tables, read once per XCD).
 struct RopeCellArgs {
     char* mixed;
     const char* cos;

@@ -861,8 +861,9 @@ __device__ __forceinline__ auto with_lanes_for(int seen, const Fn& fn) {
 // and gives them only as many lanes as the keys they see need, chosen once for the wave, so that it makes one or
 // two passes where it made four; the zeros behind those lanes are there before the results are staged.  The
 // omitted lanes held zeros and -inf only: every sum has the same terms in the same order, the same bits.  Bound
-// by the vector units and by partly written cache lines before, by latency and memory now; us per launch,
-// softmax_fwd_packed_kernel -> this, fp16 [384,129,129] 8.1 -> 6.5, [4000,129,129] 51.9 -> 45.7, with dropout
+// by the vector units and by partly written cache lines before; by memory now where there are many rows ([4000,129,129]: 118 MB
+// fetched, the lines of 67 MB of visible scores, and 137 written in 45.7 us, 5.6 TB/s), else by the chain of one round of
+// waves.  us per launch, softmax_fwd_packed_kernel -> this, fp16 [384,129,129] 8.1 -> 6.5, [4000,129,129] 51.9 -> 45.7, with dropout
 // [2000,129,129] 69.2 -> 49.3 and 65.5 -> 38.7 backward; bf16 [1200,257,257] 63.6 -> 51.6, [800,320,320]
 // 51.9 -> 44.9.  Few lanes without the staging lose (129: 51.9 -> 70.6): the zeros and the results of a row are
 // then parts of the same lines stored by different accesses.
