@@ -124,9 +124,10 @@ static bool span_shape(const RopeArgs& a, int w) {
 // of its lanes idle as its head vectors leave.  us per launch, that kernel -> the run kernel:
 //   up to two rounds, any fill: [2048,2,64,96] d_rot 24 27.7 -> 18.6, [2048,1,32,128] d_rot 128 9.1 -> 8.6, [2048,2,64,96]
 //     d_rot 96 20.4 -> 20.0, [2048,2,32,256] d_rot 64 25.1 -> 23.1; the one behind: [2048,2,64,112] d_rot 112 22.7 -> 23.1
-//   more, at most 5/8 of the lanes at work, and that share times the rounds at most 3: [32768,1,2,256] d_rot 256
-//     78 -> 23, [8192,1,8,256] 22.6 -> 17.0, [8192,1,20,256] 43 -> 36, [8192,1,2,512] d_rot 512 23.3 -> 14.3; beyond 3, behind:
-//     [8192,1,4,512] (8 rounds, half the lanes) 24.1 -> 26.2, [8192,1,16,160] (5 rounds, 5/8) 19.9 -> 20.7
+//   more, blocks at most 3/4 filled with head vectors, and the share of lanes at work times the rounds at most 3:
+//     [32768,1,2,256] d_rot 256 78 -> 23, [8192,1,8,256] 22.6 -> 17.0, [8192,1,20,256] 43 -> 36, [8192,1,24,256] 44.0 -> 41.8,
+//     [8192,1,2,512] d_rot 512 23.3 -> 14.3; beyond 3, behind: [8192,1,4,512] (8 rounds, half the lanes) 24.1 -> 26.2,
+//     [8192,1,16,160] (5 rounds, 5/8) 19.9 -> 20.7
 //   more, fuller blocks, all behind: [2048,2,16,256] d_rot 256 14.8 -> 17.0, [2048,2,8,512] d_rot 512 15.8 -> 26.1, [4096,1,32,112]
 //     d_rot 112 13.3 -> 14.4, [2048,1,40,96] d_rot 96 8.8 -> 9.1, [2048,2,32,160] d_rot 160 17.9 -> 19.4
 //   8- and 4-byte slots, which rope_span_kernel moves one by one: [2048,1,40,88] d_rot 88 12.0 -> 8.9, [2048,2,24,168] 22.3 -> 17.9,
@@ -140,8 +141,8 @@ static bool angles_in_runs(const RopeArgs& a, int w, int rounds) {
     const int lph = a.lpv * 2 + a.pad_slots;
     const int64_t per_block = (int64_t)(256 / kWave) * (kWave / lph) * kSpanIters;  // head vectors, as in launch_rope_span
     const int64_t n = a.nt > 1 && a.t[1].n_inner > a.t[0].n_inner ? a.t[1].n_inner : a.t[0].n_inner;
-    const int64_t used = n * lph, lanes = (n + per_block - 1) / per_block * (256 * kSpanIters);
-    const bool idle = used * 8 <= lanes * 5;
+    const int64_t blocks = (n + per_block - 1) / per_block, used = n * lph, lanes = blocks * (256 * kSpanIters);
+    const bool idle = n * 4 <= blocks * per_block * 3;
     if (w < kVec) return a.half <= 96 || idle || n * (2 * a.half + a.copy_dims) >= 8 * kRunSlots * kVec;
     return idle && used * rounds <= lanes * 3;
 }
