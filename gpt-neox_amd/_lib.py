@@ -198,10 +198,12 @@ def find_calls():
 def carries_tangent(*tensors):
     """Whether one of ``tensors`` is a dual tensor of forward-mode differentiation.  The kernels compute no
     tangents, so such a call goes to an autograd Function, which refuses it, and not past it."""
-    # outside of every dual level there are none (asking each tensor costs half a microsecond)
-    if getattr(forward_ad, "_current_level", 0) < 0:
-        return False
     return any(forward_ad.unpack_dual(t).tangent is not None for t in tensors)
+
+
+def in_dual_level():
+    """Whether there can be dual tensors at all (asking each tensor costs half a microsecond)."""
+    return getattr(forward_ad, "_current_level", 0) >= 0
 
 
 def check(status):

@@ -173,8 +173,11 @@ def _needs_grad(*tensors, tables=()):
     """Whether autograd has to record the call (else the autograd Function, which costs the host
     several microseconds per call, is bypassed), or to refuse it: nothing here has a forward-mode
     derivative, and a tangent is not to get lost on the way."""
-    return (torch.is_grad_enabled() and any(t.requires_grad for t in tensors)
-            or _lib.carries_tangent(*tensors, *tables))
+    if torch.is_grad_enabled():
+        for t in tensors:
+            if t.requires_grad:
+                return True
+    return _lib.in_dual_level() and _lib.carries_tangent(*tensors, *tables)
 
 
 def _rotary_out_of_place(q, k, cos, sin, offset):
