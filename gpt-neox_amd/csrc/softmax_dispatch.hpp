@@ -22,7 +22,9 @@
 //   longer rows    staged in LDS, one 1024-thread block per row: in half of a CU's LDS, two
 //                  blocks per CU (sk <= 40448), or in all of it       (sk <= 81408)
 //   ragged rows    (sk % 8 != 0 or pointers not 16-byte aligned; 8 <= sk < 81408)
-//                  the same packed, one- to sixteen-wave row and LDS-staged kernels with the kRagged flag
+//                  the same packed, one- to sixteen-wave row and LDS-staged kernels with the kRagged flag; three and
+//                  four chunks (causal forward: up to 1856 columns) in one wave, results of one-wave rows staged
+//                  in LDS (kStaged)
 //   sliding window (kBand) the one- to sixteen-wave row kernels, aligned rows of 513-32768 columns, by the
 //                  chunks the band can touch
 //   anything else  element-wise kernels (rows shorter than 8 columns or beyond 81408)
@@ -45,7 +47,7 @@ static bool on_pieces(const SoftmaxArgs& a) {
     return (reinterpret_cast<uintptr_t>(a.out) & 4095u) == 0 && (a.out2 == nullptr || (reinterpret_cast<uintptr_t>(a.out2) & 4095u) == 0);
 }
 // rows of two 4 KiB pieces each, which several rows per block store in the order of with_xcd_mapping
-static bool two_piece_rows(const SoftmaxArgs& a) { return a.sk * 2 == 8192 && on_pieces(a); }
+[[maybe_unused]] static bool two_piece_rows(const SoftmaxArgs& a) { return a.sk * 2 == 8192 && on_pieces(a); }
 
 // Switches the XCD-aware block -> unit mapping on (see xcd_slot) when the work units of a block
 // -- `units` of them, `unit_bytes` each, consecutive in memory -- tile 4 KiB pieces exactly and
@@ -80,12 +82,14 @@ static hipError_t launch_shape(const SoftmaxArgs& a0, hipStream_t st) {
     const dim3 block(kWave * WPR * RPB);
     // (one wave per row of two pieces: the order costs 2-5 %, sliding window of 256 over 4096 columns)
     const uint64_t unit_bytes = (uint64_t)a0.sk * 2;
-    const SoftmaxArgs a = with_xcd_mapping(a0, WPR == 1 && unit_bytes > 4096 ? 0 : unit_bytes, RPB, grid.x);
     constexpr int FLAGS = kDefaultFlags | EXTRA;
+    constexpr bool staged = (EXTRA & kStaged) != 0;  // a block's rows then are one run: rows in order
+    const SoftmaxArgs a = with_xcd_mapping(a0, staged || (WPR == 1 && unit_bytes > 4096) ? 0 : unit_bytes, RPB, grid.x);
+    const uint32_t lds = staged ? stage_bytes(RPB, (uint32_t)a0.sk) * (!BWD && (EXTRA & kDropout) != 0 ? 2 : 1) : 0;
     if constexpr (BWD) {
-        hipLaunchKernelGGL((softmax_bwd_kernel<T, NCH, WPR, RPB, M, FLAGS>), grid, block, 0, st, a);
+        hipLaunchKernelGGL((softmax_bwd_kernel<T, NCH, WPR, RPB, M, FLAGS>), grid, block, lds, st, a);
     } else {
-        hipLaunchKernelGGL((softmax_fwd_kernel<T, NCH, WPR, RPB, M, FLAGS>), grid, block, 0, st, a);
+        hipLaunchKernelGGL((softmax_fwd_kernel<T, NCH, WPR, RPB, M, FLAGS>), grid, block, lds, st, a);
     }
     return hipGetLastError();
 }
@@ -312,6 +316,19 @@ static bool two_causal_rows(const SoftmaxArgs& a, int chunks) {
     else return (EXTRA & kDropout) != 0 && a.sk % 8 == 4;
 }
 
+// Ragged rows of three or four chunks: one wave per row instead of two, four rows per block, the results through LDS.
+// (Two waves leave a quarter of their slots empty at three chunks and meet at barriers; staged on top, they lose 5-13 %.)  us per
+// launch, fp16, 2^27 elements, two waves -> one, forward / backward / mask-tensor forward with padding / its backward:
+//   [127,1025,1025] 87.1 -> 70.4 / 95.2 -> 93.3 / 99.1 -> 80.9 / 102.1 -> 99.4, [93,1201,1201] 79.0 -> 69.6 / 95.4 -> 92.6 / 84.6 -> 74.4 /
+//   114.4 -> 112.8, [56,1535,1535] 70.6 -> 68.6 / 91.7 -> 91.1 / 79.8 -> 77.5 / 110.9 -> 112.2, [52,1601,1601] 72.3 -> 69.8 / 94.5 -> 91.2 /
+//   80.2 -> 78.9 / 96.8 -> 94.8, [41,1801,1801] 70.7 -> 70.3 / 93.2 -> 90.6 / 81.2 -> 80.0 / 101.2 -> 99.2; causal forward [37,1901,1901]
+//   70.3 -> 70.9, [33,2001,2001] 69.3 -> 74.7, the others there 0...-4 %
+// with ALiBi [60,1049,1049] 44.8 -> 36.3, [20,1801,1801] 36.4 -> 36.1, with a bias 47.7 -> 41.2 and 41.2 -> 40.6, with dropout 76.9 ->
+// 67.0 and 64.3 -> 64.7, its backward 65.4 -> 58.7 and 56.1 -> 53.9.  All feature sets take the same shape: the same sums.
+// (two_waves_ragged: what keeps two waves for the longest of them.)
+template <Mask M, bool BWD>
+constexpr bool two_waves_ragged = !BWD && M == Mask::Causal;
+
 template <typename T, Mask M, bool BWD, int EXTRA>
 static hipError_t dispatch_rows(const SoftmaxArgs& a, bool vec_ok, hipStream_t st) {
     int chunks = (a.sk + kChunk - 1) / kChunk;
@@ -337,7 +354,16 @@ static hipError_t dispatch_rows(const SoftmaxArgs& a, bool vec_ok, hipStream_t s
     }
     // (the aligned full-row backward has taken 2 to 4 chunks with its packed kernel above)
     if constexpr (!(BWD && M == Mask::None && (EXTRA & kRagged) == 0)) {
-        if (chunks == 2) return launch_shape<T, M, BWD, EXTRA, 2, 1, 4>(a, st);
+        if (chunks == 2) {
+            if constexpr (EXTRA == kRagged) {
+                // the block's results through LDS where the rows fill most of their two chunks (see Rows); us per launch, fp16, 2^26
+                // elements, direct -> staged: forward [92,851,851] 36.9 -> 37.5, [82,901,901] 36.9 -> 36.8, [74,951,951] 36.6 -> 36.2,
+                // [64,1022,1022] 36.7 -> 36.1, backward [185,601,601] 50.0 both, [136,701,701] 49.6 -> 48.8, [65,1009,1009] 48.4 -> 47.1;
+                // with dropout behind throughout ([96,1001,1001] 94.2 -> 96.1 and 86.6 -> 90.0)
+                if (a.sk >= (BWD ? 672 : 944)) return launch_shape<T, M, BWD, EXTRA | kStaged, 2, 1, 4>(a, st);
+            }
+            return launch_shape<T, M, BWD, EXTRA, 2, 1, 4>(a, st);
+        }
         if constexpr ((EXTRA & kBand) != 0) {
             // rows that are mostly zeros in front of and behind the band: twice the waves, one chunk of the band each.
             // us per launch forward / backward, two chunks per wave -> one: [8,8192,8192] window 1024 220 -> 207 / 241 -> 236,
@@ -346,12 +372,24 @@ static hipError_t dispatch_rows(const SoftmaxArgs& a, bool vec_ok, hipStream_t s
             // 207 -> 203, [2,16384,16384] 1500 210 -> 232 / 223 -> 232, [1,32768,32768] 1024 408 -> 446 / 431 -> 460
             if (a.sk > 4096 && a.sk <= 28 * kChunk && (chunks == 3 || chunks == 4)) return launch_shape<T, M, BWD, EXTRA, 1, 4, 1>(a, st);
         }
-        if (chunks == 3) return launch_shape<T, M, BWD, EXTRA, 2, 2, 2>(a, st);
-        if (chunks == 4) {
-            // the causal forward with two output streams (dropout) measured 3 % faster with 2 rows
-            if constexpr (!BWD && M == Mask::Causal && (EXTRA & kDropout) != 0)
-                return launch_shape<T, M, BWD, EXTRA, 2, 2, 2>(a, st);
-            return launch_shape<T, M, BWD, EXTRA, 2, 2, 4>(a, st);
+        constexpr bool ragged = (EXTRA & kRagged) != 0;
+        if constexpr (ragged) {
+            // not staged: the backward pass with dropout, [60,1049,1049] 58.7 us against 61.5, [26,1601,1601] 55.9 and 56.4, and the
+            // mask-tensor forward with dropout, [8,7,1049,1049] 95.4 and 99.3, [8,3,1601,1601] 84.2 and 88.0
+            constexpr bool staged = (EXTRA & kDropout) == 0 || (!BWD && M == Mask::Causal);
+            constexpr int FL = EXTRA | (staged ? kStaged : 0);
+            if (chunks == 3) return launch_shape<T, M, BWD, FL, 3, 1, 4>(a, st);
+            if (chunks == 4 && (!two_waves_ragged<M, BWD> || a.sk <= 1856)) return launch_shape<T, M, BWD, FL, 4, 1, 4>(a, st);
+        } else {
+            if (chunks == 3) return launch_shape<T, M, BWD, EXTRA, 2, 2, 2>(a, st);
+        }
+        if constexpr (!ragged || two_waves_ragged<M, BWD>) {
+            if (chunks == 4) {
+                // the causal forward with two output streams (dropout) measured 3 % faster with 2 rows
+                if constexpr (!BWD && M == Mask::Causal && (EXTRA & kDropout) != 0)
+                    return launch_shape<T, M, BWD, EXTRA, 2, 2, 2>(a, st);
+                return launch_shape<T, M, BWD, EXTRA, 2, 2, 4>(a, st);
+            }
         }
     }
     if constexpr (!BWD && (EXTRA & kBand) == 0) {

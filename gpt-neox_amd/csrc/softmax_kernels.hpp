@@ -78,17 +78,17 @@ constexpr int kDropout = 8;
 constexpr int kBias = 16;
 // Ragged rows: the tensors start at any 2-byte boundary and sk is any number >= 8, so a row
 // starts wherever the previous one ends.  128-bit buffer accesses work at any alignment on
-// gfx950 and their range check acts per dword: against a buffer of exactly the row's bytes,
-// every dword inside the row is transferred and only a dword that crosses the row end is
-// dropped.  For 16-bit data that is one element, which these kernels move by a 16-bit access of
-// its own; for the mask bytes it is up to three, fetched again by a dword load that ends with the
-// row.  Accesses that are not even dword-aligned cost 10-20 % of the bandwidth, though, so a row
+// gfx950, but accesses that are not even dword-aligned cost 10-20 % of the bandwidth, so a row
 // that starts on an odd element is laid over the lanes one element later (sh = 1): lane l of a
-// chunk then holds the columns 8l - 1 .. 8l + 6 and all its accesses are dword-aligned; only the
-// first lane of the row, whose access would begin in front of the row, takes its seven columns by
-// a 16-bit and a 96-bit access.  "Positions" below are columns + sh: the row occupies the
-// positions [sh, len + sh).  With kDropout a lane's 8 columns straddle two Philox groups (the
-// pattern is a function of the row-major element index).
+// chunk then holds the columns 8l - 1 .. 8l + 6 and its accesses are dword-aligned.  The lanes at the
+// two ends of a row: RaggedRow for the row kernels, ragged_back for the packed ones.  The LDS-staged
+// kernels end a row by the range check instead, which acts per dword: against a buffer of exactly the
+// row's bytes every dword inside the row is transferred and only one that crosses the row end is
+// dropped -- for 16-bit data one element, which they move by a 16-bit access of its own; for the mask
+// bytes up to three, fetched again by a dword load that ends with the row --, and the first lane of a
+// shifted row takes its seven columns by a 16-bit and a 96-bit access.  "Positions" there are columns + sh:
+// the row occupies the positions [sh, len + sh).  With kDropout a lane's 8 columns straddle two Philox
+// groups (the pattern is a function of the row-major element index).
 constexpr int kRagged = 32;
 // Sliding-window causal rows (Mask::Causal row kernels only): row i sees the keys lo .. i with
 // lo = max(0, i - window) -- the mask megatron/utils.py:67-80 builds for sliding_window_width.  The
@@ -96,6 +96,8 @@ constexpr int kRagged = 32;
 // out-of-range offset, and chunks that lie wholly in front of the band are neither read nor
 // computed (wave-uniform branch), like those above the diagonal; their zeros are still stored.
 constexpr int kBand = 64;
+// Ragged row kernels only: the block's results go through LDS (see Rows).
+constexpr int kStaged = 128;
 constexpr int kDefaultFlags = kNtLoad | kNtStore;
 
 // kRagged: 1 if the row starts on an odd element (2 mod 4 bytes) of the tensor at `base` and sk is
@@ -232,8 +234,8 @@ __device__ __forceinline__ uint32_t keep_bits_row8(const DropoutArgs& d, uint32_
 // each go the same way in groups of 4 blocks (group_shift 2): an XCD then keeps to two pieces in eight.
 // Returns the unit index for unit l of block b; the identity for the last, incomplete group.
 __device__ __forceinline__ uint32_t xcd_slot(uint32_t b, uint32_t l, uint32_t U, const SoftmaxArgs& a) {
-    if (b >= a.affine_blocks) return b * U + l;
-    const uint32_t sh = a.piece_shift, gs = a.group_shift;
+    // (no branch: the kernel's arguments behind one would be fetched a round trip later)
+    const uint32_t sh = a.piece_shift, gs = b < a.affine_blocks ? a.group_shift : 0u;  // groups of one block: in order
     const uint32_t g = b >> gs, x = b & ((1u << gs) - 1u);
     const uint32_t j = l >> sh, t = l & ((1u << sh) - 1u);  // piece of the block, unit inside the piece
     return (((((g * (U >> sh)) + j) << gs) + x) << sh) + t;
@@ -270,6 +272,13 @@ __device__ __forceinline__ RowPos locate(uint32_t row, const SoftmaxArgs& a) {
     return p;
 }
 
+// Loads in front of this point are asked for before anything behind it.  The compiler otherwise moves a chunk's load into
+// the branch that uses it, or the loads of later rows behind the first row's arithmetic: a second round trip to memory.
+__device__ __forceinline__ void loads_first() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
+
 // Combine a per-wave partial across the WPR waves of a row.
 template <typename Op, int WPR, int RPB>
 __device__ __forceinline__ float row_combine(float v, float* red, int wib, int rib, int lane) {
@@ -284,6 +293,138 @@ __device__ __forceinline__ float row_combine(float v, float* red, int wib, int r
         return Op::dec(r);
     }
 }
+
+// How the row kernels lay a row over their lanes.  Aligned rows: lane l of the chunk at position c0 holds the columns
+// c0 + 8l .. c0 + 8l + 7.  kRagged: a row that starts on an odd element lies one position later (sh = 1), so that its
+// accesses are dword-aligned, the lane that would begin in front of the row is moved forward by that position, and the one
+// that would reach behind it is moved back to end with the row.  Such a lane shares columns with its neighbour: both
+// compute and store the same bits for them, and only one counts them in the row's sums.  Every lane so makes one 128-bit
+// access per tensor, inside the row.
+template <bool RAG>
+struct RaggedRow {  // aligned rows
+    static constexpr int sh = 0;
+    int lane;
+    __device__ __forceinline__ RaggedRow(const void*, uint32_t, int, int lane_, bool) : lane(lane_) {}
+    __device__ __forceinline__ int col(int c0) const { return c0 + lane * kVec; }
+    __device__ __forceinline__ int chunk_col(int c0) const { return c0; }
+    __device__ __forceinline__ float add(float sum, const float (&v)[8], int) const {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) sum += v[k];
+        return sum;
+    }
+    __device__ __forceinline__ void own(float (&)[8], int) const {}
+    __device__ __forceinline__ uint32_t store_off(int) const { return 0; }
+};
+template <>
+struct RaggedRow<true> {
+    int sh, sk, lane;
+    bool first;  // the wave holds the row's first chunk, moved by sh
+    __device__ __forceinline__ RaggedRow(const void* base, uint32_t row, int sk_, int lane_, bool first_wave)
+        : sh(ragged_shift(base, row, sk_)), sk(sk_), lane(lane_), first(sh != 0 && first_wave) {}
+    // first column of the lane's access; a lane behind the row: one that no row has
+    __device__ __forceinline__ int col(int c0) const {
+        const int own = c0 + lane * kVec - sh;
+        return own < sk ? min(max(own, 0), sk - kVec) : 0x3fffffff;
+    }
+    // the first column that any lane of the chunk holds (wave-uniform)
+    __device__ __forceinline__ int chunk_col(int c0) const { return c0 - sh < sk ? min(c0 - sh, sk - kVec) : sk; }
+    // the lane moved back is in this chunk (wave-uniform)
+    __device__ __forceinline__ bool moved_back(int c0) const { return c0 + kChunk - sh > sk && ((sk + sh) & (kVec - 1)) != 0; }
+    // columns of the lane that the lane before it counts
+    __device__ __forceinline__ int back(int c0) const {
+        const int own = c0 + lane * kVec - sh;
+        return own < sk ? own + kVec - sk : 0;
+    }
+    __device__ __forceinline__ float add(float sum, const float (&v)[8], int c0) const {
+        if (moved_back(c0)) {
+            const int b = back(c0);
+#pragma unroll
+            for (int k = 0; k < 7; ++k) sum += k < b ? 0.f : v[k];
+        } else {
+#pragma unroll
+            for (int k = 0; k < 7; ++k) sum += v[k];
+        }
+        return sum + ((first && c0 == 0 && lane == 0) ? 0.f : v[7]);  // column 7 is the second lane's
+    }
+    // zero in the columns that another lane counts
+    __device__ __forceinline__ void own(float (&v)[8], int c0) const {
+        if (moved_back(c0)) {
+            const int b = back(c0);
+#pragma unroll
+            for (int k = 0; k < 7; ++k) v[k] = k < b ? 0.f : v[k];
+        }
+        if (first && c0 == 0) v[7] = lane == 0 ? 0.f : v[7];
+    }
+    __device__ __forceinline__ uint32_t store_off(int c0) const {
+        const int at = col(c0);
+        return at < sk ? (uint32_t)at * 2 : kOutOfRange;
+    }
+};
+
+// Where the row kernels put their results: straight into the row (ST false), or, ragged rows, into LDS at the place they
+// have in the block's run of rows, from where the whole block stores the run in accesses that are aligned to cache lines.
+// A wave that stores a ragged row itself writes parts of lines at both ends of every access; the pattern alone, without
+// arithmetic, causal rows of 1001 columns, runs at 5.2 TB/s that way and at 5.6 staged, full rows at 5.9 and 6.2.
+struct __attribute__((packed, aligned(2))) Slot16 { u32x4 v; };  // 16 bytes at the alignment of an element
+constexpr int kLine = 128;
+// LDS of one output of a block of `rows` rows
+__host__ __device__ constexpr uint32_t stage_bytes(uint32_t rows, uint32_t sk) { return (rows * sk * 2 + kLine + 31) & ~15u; }
+extern __shared__ __attribute__((aligned(16))) char lds_stage[];
+
+template <bool ST, int RPB>
+struct Rows {
+    rsrc_t row;
+    __device__ __forceinline__ Rows(const SoftmaxArgs& a, void* out, const RowPos& pos, int, int) {
+        row = make_rsrc(static_cast<char*>(out) + (size_t)pos.row * a.sk * 2, pos.store ? (uint32_t)a.sk * 2u : 0u);
+    }
+    template <bool NT>
+    __device__ __forceinline__ void put(const u32x4& v, uint32_t off) const { buf_st128<NT>(row, v, off, 0); }
+};
+template <int RPB>
+struct Rows<true, RPB> {
+    char* stage;     // the block's rows in LDS, at the place in a line that they have in memory
+    char* mem;       // the line in memory that the run begins in
+    uint32_t head;   // bytes of that line in front of the run
+    uint32_t end;    // of the run, counted from that line
+    char* row;       // the wave's row in LDS (a surplus row: behind the run, where nothing is taken from)
+    uint32_t spare;  // 16 bytes for the lanes behind the row, counted from `row`
+    __device__ __forceinline__ Rows(const SoftmaxArgs& a, void* out, const RowPos&, int rib, int which) {
+        const uint32_t row0 = blockIdx.x * RPB, size = stage_bytes(RPB, a.sk);
+        mem = static_cast<char*>(out) + (size_t)row0 * a.sk * 2;
+        head = (uint32_t)(reinterpret_cast<uintptr_t>(mem) & (kLine - 1));
+        mem -= head;
+        end = head + min((uint32_t)RPB, a.rows - row0) * a.sk * 2;
+        stage = lds_stage + which * size;
+        row = stage + head + rib * a.sk * 2;
+        spare = size - 16 - (uint32_t)(row - stage);
+    }
+    template <bool>
+    __device__ __forceinline__ void put(const u32x4& v, uint32_t off) const {
+        reinterpret_cast<Slot16*>(row + (off != kOutOfRange ? off : spare))->v = v;
+    }
+    // after a barrier
+    template <bool NT, int THREADS, int N>
+    __device__ __forceinline__ void flush() const {
+        const rsrc_t r = make_rsrc(mem, end);  // stores every whole dword in front of the run's end
+        const uint32_t at = threadIdx.x * 16;
+        // N accesses of a thread hold the rows, one more the part of a line in front of them
+#pragma unroll
+        for (int i = 0; i <= N; ++i) {
+            if (i < N || (uint32_t)(N * THREADS * 16) < end) {
+                const u32x4 v = *reinterpret_cast<const u32x4*>(stage + min(at + i * THREADS * 16, end & ~15u));
+                buf_st128<NT>(r, v, (i > 0 || at >= head) ? at + i * THREADS * 16 : kOutOfRange, 0);
+            }
+        }
+        // the elements of the run's first 16 bytes that the block in front has the rest of, and the last one if its dword
+        // is the next block's too
+        if (((head | end) & 15) != 0 && threadIdx.x < 8) {
+            const bool last = threadIdx.x == 7;
+            const uint32_t off = last ? end - 2 : head + threadIdx.x * 2;
+            const bool alone = last ? (end & 3) != 0 : off < ((head + 15) & ~15u);
+            buf_st16(r, *reinterpret_cast<const uint16_t*>(stage + off), alone ? off : kOutOfRange);
+        }
+    }
+};
 
 // kBand: the waves of a row hold the NCH * WPR chunks from the band's first chunk on; the chunks of
 // the row in front of those and behind them hold nothing but zeros, which the waves store here,
@@ -312,7 +453,7 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void softmax_fwd_kernel(SoftmaxArg
     __shared__ float red_sum[WPR * RPB];
     constexpr bool kLdNt = (FLAGS & kNtLoad) != 0, kStNt = (FLAGS & kNtStore) != 0;
     constexpr bool kRag = (FLAGS & kRagged) != 0;
-    constexpr bool kBnd = (FLAGS & kBand) != 0;
+    constexpr bool kBnd = (FLAGS & kBand) != 0, kStage = (FLAGS & kStaged) != 0;
     static_assert(!kBnd || (MASK == Mask::Causal && (FLAGS & (kRagged | kAlibi | kBias | kDropout)) == 0),
                   "the sliding window comes with the plain causal row kernels only");
 
@@ -325,9 +466,7 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void softmax_fwd_kernel(SoftmaxArg
     // byte offset of the lane inside the row, first chunk of its wave.  Everything goes into
     // the per-lane offset: the hardware's range check does not see the scalar offset operand.
     const RowPos pos = locate<MASK>(xcd_slot(blockIdx.x, rib, RPB, a), a);
-    // kRagged: the row lies one position later on the lanes when it starts on an odd element
-    int sh = 0;
-    if constexpr (kRag) sh = ragged_shift(a.in0, pos.row, sk);
+    const RaggedRow<kRag> rag(a.in0, pos.row, sk, lane, wir == 0);
     // kBand: first visible key of the row, and the start of the 128-bit access that holds it.  The
     // waves' chunks are counted from the chunk that holds that key (wch instead of wir), so that a
     // row needs only as many chunk slots as its band is long; see band_zero_fill for the rest.
@@ -335,9 +474,13 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void softmax_fwd_kernel(SoftmaxArg
     if constexpr (kBnd) lo = max((int)pos.i - a.window, 0);
     const int lo8 = lo & ~(kVec - 1);
     const int wch = wir + lo / kChunk;  // the wave's first chunk of the row (wir without a window)
-    const int voff = lane * 16 + wch * kChunk * 2 - 2 * sh;
-    const bool head = kRag && sh != 0 && wir == 0;  // wave-uniform: this wave holds the row start
-    const bool first_lane = head && lane == 0;      // its first access would begin in front of the row
+    const int voff = lane * 16 + wch * kChunk * 2;
+    // byte offset of the lane's access to a tensor of `e`-byte elements, none behind the keys that take part
+    auto lane_off = [&](int c, int e) -> uint32_t {
+        if constexpr (!kRag) return (uint32_t)(voff + c * WPR * kChunk * 2) * e / 2;
+        const int col = rag.col((wch + c * WPR) * kChunk);
+        return col < pos.len ? (uint32_t)col * e : kOutOfRange;
+    };
     DropoutArgs drop = a.drop;
     if constexpr ((FLAGS & kDropout) != 0) drop = resolve(drop);
     // ALiBi: scale*(x + slope*(j - i')) = x*scale + slope2*(j - i'), slope2 wave-uniform
@@ -347,53 +490,33 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void softmax_fwd_kernel(SoftmaxArg
     u32x4 raw[NCH];
     u32x4 rawb[NCH];  // kBias
     u32x2 mk[NCH];
-    uint32_t tail_x = 0, tail_b = 0, tail_m = 0;  // kRagged: what the range check drops at the row end
     {
         // ---- issue every load of the row before the first use
         const char* x = static_cast<const char*>(a.in0) + (size_t)pos.row * sk * 2;
-        // whole 128-bit accesses up to the valid length; a ragged row ends where the next one begins
-        const uint32_t row_bytes = (uint32_t)(kRag ? pos.len : (pos.len + kVec - 1) & ~(kVec - 1)) * 2u;
+        // whole 128-bit accesses up to the valid length
+        const uint32_t row_keys = (uint32_t)(kRag ? sk : (pos.len + kVec - 1) & ~(kVec - 1));
+        const uint32_t row_bytes = row_keys * 2u;
         const rsrc_t rx = make_rsrc(x, row_bytes);
         if constexpr (MASK == Mask::Bytes) {
             const uint32_t mb = a.mask_bcast ? 0u : a.by_mask_batch.div(pos.row);
             // (whole 64-bit accesses up to a row end that a hint has moved in front of sk, like the scores)
-            const rsrc_t rm = make_rsrc(a.mask + ((size_t)mb * a.sq + pos.i) * sk,
-                                        (uint32_t)(kRag ? pos.len : (pos.len + kVec - 1) & ~(kVec - 1)));
+            const rsrc_t rm = make_rsrc(a.mask + ((size_t)mb * a.sq + pos.i) * sk, row_keys);
 #pragma unroll
-            for (int c = 0; c < NCH; ++c)
-                mk[c] = buf_ld64(rm, (c == 0 && first_lane) ? kOutOfRange : lane * 8 + (wir + c * WPR) * kChunk - sh, 0);
-            if constexpr (kRag) {
-                tail_m = ragged_tail_mask(rm, pos.len, sh);
-                if (head) {
-                    const u32x2 hm = ragged_head_mask(rm, first_lane);
-                    mk[0].x |= hm.x;
-                    mk[0].y |= hm.y;
-                }
-            }
+            for (int c = 0; c < NCH; ++c) mk[c] = buf_ld64(rm, lane_off(c, 1), 0);
         }
 #pragma unroll
         for (int c = 0; c < NCH; ++c) {
-            uint32_t off = (c == 0 && first_lane) ? kOutOfRange : voff + c * WPR * kChunk * 2;
+            uint32_t off = lane_off(c, 2);
             if constexpr (kBnd) off = ((int)off < lo8 * 2) ? kOutOfRange : off;  // in front of the band: nothing fetched
             raw[c] = buf_ld128<kLdNt>(rx, off, 0);
-        }
-        if constexpr (kRag) {
-            tail_x = ragged_tail16(rx, pos.len, sh);
-            if (head) raw[0] |= ragged_head_load(rx, first_lane);
         }
         if constexpr ((FLAGS & kBias) != 0) {
             const rsrc_t rb = make_rsrc(static_cast<const char*>(a.bias) + (size_t)bias_row(pos.row, a) * sk * 2, row_bytes);
 #pragma unroll
-            for (int c = 0; c < NCH; ++c) {
-                const uint32_t off = (c == 0 && first_lane) ? kOutOfRange : voff + c * WPR * kChunk * 2;
-                rawb[c] = buf_ld128<false>(rb, off, 0);
-            }
-            if constexpr (kRag) {
-                tail_b = ragged_tail16(rb, pos.len, sh);
-                if (head) rawb[0] |= ragged_head_load(rb, first_lane);
-            }
+            for (int c = 0; c < NCH; ++c) rawb[c] = buf_ld128<false>(rb, lane_off(c, 2), 0);
         }
     }
+    if constexpr (kRag) loads_first();
     if constexpr (kBnd) {
         // while the loads are in flight: the zeros of the chunks that no wave holds
         const rsrc_t rz = make_rsrc(static_cast<char*>(a.out) + (size_t)pos.row * sk * 2, pos.store ? (uint32_t)sk * 2u : 0u);
@@ -401,7 +524,6 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void softmax_fwd_kernel(SoftmaxArg
     }
     {
         const int len = pos.len;
-        const int plen = len + sh;  // the row's columns lie at the positions [sh, plen)
         float v[NCH][8];
 
         // ---- scale, mask, running maximum
@@ -409,15 +531,8 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void softmax_fwd_kernel(SoftmaxArg
 #pragma unroll
         for (int c = 0; c < NCH; ++c) {
             const int c0 = (wch + WPR * c) * kChunk;  // first position of the chunk (wave-uniform)
-            if (c0 < plen && (!kBnd || c0 + kChunk > lo)) {
-                const int col = c0 + lane * kVec - sh;  // first column of the lane, -1 in front of the row
-                if constexpr (kRag) {
-                    if (c0 + kChunk >= plen) {  // the chunk that holds the row end
-                        ragged_patch16(raw[c], c0 + lane * kVec, plen, tail_x);
-                        if constexpr ((FLAGS & kBias) != 0) ragged_patch16(rawb[c], c0 + lane * kVec, plen, tail_b);
-                        if constexpr (MASK == Mask::Bytes) ragged_patch_mask(mk[c], c0 + lane * kVec, plen, tail_m);
-                    }
-                }
+            if (rag.chunk_col(c0) < len && (!kBnd || c0 + kChunk > lo)) {
+                const int col = rag.col(c0);  // first column of the lane
                 unpack8<T>(raw[c], v[c]);
                 if constexpr ((FLAGS & kBias) != 0) {
                     float bv[8];
@@ -425,8 +540,8 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void softmax_fwd_kernel(SoftmaxArg
 #pragma unroll
                     for (int k = 0; k < 8; ++k) v[c][k] += bv[k];
                 }
-                // no lane of the wave crosses the row end (or holds the position in front of the row)
-                bool plain = (c0 + kChunk <= plen) && !(head && c == 0);
+                // no lane of the wave crosses the row end
+                bool plain = c0 + kChunk - rag.sh <= len;
                 if constexpr (kBnd) plain = plain && c0 >= lo;
                 if constexpr (MASK == Mask::Bytes) {
                     plain = plain && (__builtin_amdgcn_ballot_w64((mk[c].x | mk[c].y) != 0) == 0);
@@ -447,7 +562,6 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void softmax_fwd_kernel(SoftmaxArg
 #pragma unroll
                     for (int k = 0; k < 8; ++k) {
                         bool keep = (col + k) < len;
-                        if constexpr (kRag) keep = keep && (col + k) >= 0;
                         if constexpr (kBnd) keep = keep && (col + k) >= lo;
                         if constexpr (MASK == Mask::Bytes) {
                             const uint32_t w = (k < 4) ? mk[c].x : mk[c].y;
@@ -467,12 +581,10 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void softmax_fwd_kernel(SoftmaxArg
 #pragma unroll
         for (int c = 0; c < NCH; ++c) {
             const int c0 = (wch + WPR * c) * kChunk;
-            if (c0 < plen && (!kBnd || c0 + kChunk > lo)) {
+            if (rag.chunk_col(c0) < len && (!kBnd || c0 + kChunk > lo)) {
 #pragma unroll
-                for (int k = 0; k < 8; ++k) {
-                    v[c][k] = fast_exp2(v[c][k] - mx);
-                    sum += v[c][k];
-                }
+                for (int k = 0; k < 8; ++k) v[c][k] = fast_exp2(v[c][k] - mx);
+                sum = rag.add(sum, v[c], c0);
             }
         }
         if constexpr (MASK == Mask::Bytes) {
@@ -482,12 +594,10 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void softmax_fwd_kernel(SoftmaxArg
                 sum = 0.f;
 #pragma unroll
                 for (int c = 0; c < NCH; ++c) {
-                    const int col = (wch + WPR * c) * kChunk + lane * kVec - sh;
+                    const int c0 = (wch + WPR * c) * kChunk, col = rag.col(c0);
 #pragma unroll
-                    for (int k = 0; k < 8; ++k) {
-                        v[c][k] = ((col + k) < len && (col + k) >= 0) ? 1.f : 0.f;
-                        sum += v[c][k];
-                    }
+                    for (int k = 0; k < 8; ++k) v[c][k] = (col + k) < len ? 1.f : 0.f;
+                    sum = rag.add(sum, v[c], c0);
                 }
             }
         }
@@ -496,46 +606,40 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void softmax_fwd_kernel(SoftmaxArg
         const float inv = 1.0f / sum;
 
         // ---- normalise and store; chunks above the diagonal store zeros
-        char* y = static_cast<char*>(a.out) + (size_t)pos.row * sk * 2;
-        const rsrc_t ry = make_rsrc(y, pos.store ? (uint32_t)sk * 2u : 0u);
-        rsrc_t ry2 = ry;
-        if constexpr ((FLAGS & kDropout) != 0) {
-            ry2 = make_rsrc(static_cast<char*>(a.out2) + (size_t)pos.row * sk * 2, pos.store ? (uint32_t)sk * 2u : 0u);
-        }
+        const Rows<kStage, RPB> out(a, a.out, pos, rib, 0);
         u32x4 o[NCH];
 #pragma unroll
         for (int c = 0; c < NCH; ++c) {
             const int c0 = (wch + WPR * c) * kChunk;
             o[c] = u32x4{0, 0, 0, 0};
-            if (c0 < plen && (!kBnd || c0 + kChunk > lo)) {
+            if (rag.chunk_col(c0) < len && (!kBnd || c0 + kChunk > lo)) {
 #pragma unroll
                 for (int k = 0; k < 8; ++k) v[c][k] *= inv;
                 o[c] = pack8<T>(v[c]);
             }
-            buf_st128<kStNt>(ry, o[c], (c == 0 && first_lane) ? kOutOfRange : voff + c * WPR * kChunk * 2, 0);
-            if constexpr (kRag) {
-                if (c == 0 && head) ragged_head_store(ry, o[c], first_lane);
-                if (c0 < sk + sh && c0 + kChunk >= sk + sh)
-                    ragged_store16(ry, o[c], c0 + lane * kVec, sk + sh, (uint32_t)(sk - 1) * 2u);
-            }
+            out.template put<kStNt>(o[c], kRag ? rag.store_off(c0) : voff + c * WPR * kChunk * 2);
         }
         if constexpr ((FLAGS & kDropout) != 0) {
             // second output after the first: each stream is written in runs of whole rows
+            const Rows<kStage, RPB> out2(a, a.out2, pos, rib, 1);
 #pragma unroll
             for (int c = 0; c < NCH; ++c) {
                 const int c0 = (wch + WPR * c) * kChunk;
                 u32x4 o2 = u32x4{0, 0, 0, 0};
-                if (c0 < plen) {
-                    const uint32_t bits = keep_bits_row8<kRag>(drop, pos.row, sk, c0 + lane * kVec - sh);
+                if (rag.chunk_col(c0) < len) {
+                    const uint32_t bits = keep_bits_row8<kRag>(drop, pos.row, sk, rag.col(c0));
                     o2 = dropout8<T>(o[c], bits, drop.scale);
                 }
-                buf_st128<kStNt>(ry2, o2, (c == 0 && first_lane) ? kOutOfRange : voff + c * WPR * kChunk * 2, 0);
-                if constexpr (kRag) {
-                    if (c == 0 && head) ragged_head_store(ry2, o2, first_lane);
-                    if (c0 < sk + sh && c0 + kChunk >= sk + sh)
-                        ragged_store16(ry2, o2, c0 + lane * kVec, sk + sh, (uint32_t)(sk - 1) * 2u);
-                }
+                out2.template put<kStNt>(o2, kRag ? rag.store_off(c0) : voff + c * WPR * kChunk * 2);
             }
+            if constexpr (kStage) {
+                __syncthreads();
+                out.template flush<kStNt, kWave * WPR * RPB, NCH>();
+                out2.template flush<kStNt, kWave * WPR * RPB, NCH>();
+            }
+        } else if constexpr (kStage) {
+            __syncthreads();
+            out.template flush<kStNt, kWave * WPR * RPB, NCH>();
         }
     }
 }
@@ -548,7 +652,7 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void softmax_bwd_kernel(SoftmaxArg
     __shared__ float red_sum[WPR * RPB];
     constexpr bool kLdNt = (FLAGS & kNtLoad) != 0, kStNt = (FLAGS & kNtStore) != 0;
     constexpr bool kRag = (FLAGS & kRagged) != 0;
-    constexpr bool kBnd = (FLAGS & kBand) != 0;
+    constexpr bool kBnd = (FLAGS & kBand) != 0, kStage = (FLAGS & kStaged) != 0;
     static_assert(!kBnd || (MASK == Mask::Causal && (FLAGS & (kRagged | kDropout)) == 0),
                   "the sliding window comes with the plain causal row kernels only");
 
@@ -564,19 +668,13 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void softmax_bwd_kernel(SoftmaxArg
     if constexpr (kBnd) lo = max((int)pos.i - a.window, 0);
     const int lo8 = lo & ~(kVec - 1);
     const int wch = wir + lo / kChunk;
-    // kRagged: the row lies one position later on the lanes when it starts on an odd element; the
-    // position in front of it stays zero in both tensors and is never stored
-    int sh = 0;
-    if constexpr (kRag) sh = ragged_shift(a.in0, pos.row, sk);
-    const int voff = lane * 16 + wch * kChunk * 2 - 2 * sh;  // the range check ignores a scalar offset
-    const bool head = kRag && sh != 0 && wir == 0;  // wave-uniform: this wave holds the row start
-    const bool first_lane = head && lane == 0;      // its first access would begin in front of the row
+    const RaggedRow<kRag> rag(a.in0, pos.row, sk, lane, wir == 0);
+    const int voff = lane * 16 + wch * kChunk * 2;  // the range check ignores a scalar offset
     DropoutArgs drop = a.drop;
     if constexpr ((FLAGS & kDropout) != 0) drop = resolve(drop);
     u32x4 rg[NCH], rp[NCH];
-    uint32_t tail_g = 0, tail_p = 0;  // kRagged: what the range check drops at the row end
     {
-        const uint32_t bytes = (uint32_t)(kRag ? pos.len : (pos.len + kVec - 1) & ~(kVec - 1)) * 2u;
+        const uint32_t bytes = (uint32_t)(kRag ? sk : (pos.len + kVec - 1) & ~(kVec - 1)) * 2u;
         const rsrc_t bg = make_rsrc(static_cast<const char*>(a.in0) + (size_t)pos.row * sk * 2, bytes);
         const rsrc_t by = make_rsrc(static_cast<const char*>(a.in1) + (size_t)pos.row * sk * 2, bytes);
         // full rows (after a mask-tensor forward): the probabilities first, and no gradient for a lane
@@ -584,7 +682,11 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void softmax_bwd_kernel(SoftmaxArg
         constexpr bool kSkip = kSkipHidden && MASK == Mask::None && !kRag;
 #pragma unroll
         for (int c = 0; c < NCH; ++c) {
-            uint32_t off = (c == 0 && first_lane) ? kOutOfRange : voff + c * WPR * kChunk * 2;
+            uint32_t off = voff + c * WPR * kChunk * 2;
+            if constexpr (kRag) {
+                const int col = rag.col((wch + c * WPR) * kChunk);
+                off = col < pos.len ? (uint32_t)col * 2 : kOutOfRange;
+            }
             if constexpr (kBnd) off = ((int)off < lo8 * 2) ? kOutOfRange : off;  // in front of the band: nothing fetched
             rp[c] = buf_ld128<kLdNt>(by, off, 0);
             if constexpr (!kSkip) rg[c] = buf_ld128<kLdNt>(bg, off, 0);
@@ -594,15 +696,8 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void softmax_bwd_kernel(SoftmaxArg
             for (int c = 0; c < NCH; ++c)
                 rg[c] = buf_ld128<kLdNt>(bg, all_zero(rp[c]) ? kOutOfRange : voff + c * WPR * kChunk * 2, 0);
         }
-        if constexpr (kRag) {
-            tail_g = ragged_tail16(bg, pos.len, sh);
-            tail_p = ragged_tail16(by, pos.len, sh);
-            if (head) {
-                rg[0] |= ragged_head_load(bg, first_lane);
-                rp[0] |= ragged_head_load(by, first_lane);
-            }
-        }
     }
+    if constexpr (kRag) loads_first();
     if constexpr (kBnd) {
         // the zeros of the chunks that no wave holds.  dx may alias dy: those chunks lie outside the
         // band, where nothing is read
@@ -612,7 +707,6 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void softmax_bwd_kernel(SoftmaxArg
     {
         // dx may alias dy: a row is read and written by the same waves only, reads first
         const int len = pos.len;
-        const int plen = len + sh;  // the row's columns lie at the positions [sh, plen)
 
         // the row stays packed; it is unpacked once for the dot product and once for dx
         float dot = 0.f;
@@ -621,14 +715,8 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void softmax_bwd_kernel(SoftmaxArg
         for (int c = 0; c < NCH; ++c) {
             const int c0 = (wch + WPR * c) * kChunk;
             kb[c] = 0xffu;
-            if (c0 < plen && (!kBnd || c0 + kChunk > lo)) {
-                const int col = c0 + lane * kVec - sh;  // first column of the lane
-                if constexpr (kRag) {
-                    if (c0 + kChunk >= plen) {  // the chunk that holds the row end
-                        ragged_patch16(rg[c], c0 + lane * kVec, plen, tail_g);
-                        ragged_patch16(rp[c], c0 + lane * kVec, plen, tail_p);
-                    }
-                }
+            if (rag.chunk_col(c0) < len && (!kBnd || c0 + kChunk > lo)) {
+                const int col = rag.col(c0);  // first column of the lane
                 float gv[8], pv[8];
                 unpack8<T>(rg[c], gv);
                 unpack8<T>(rp[c], pv);
@@ -637,7 +725,7 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void softmax_bwd_kernel(SoftmaxArg
 #pragma unroll
                     for (int k = 0; k < 8; ++k) gv[k] = ((kb[c] >> k) & 1u) ? gv[k] * drop.scale : 0.f;
                 }
-                if (c0 + kChunk > plen) {
+                if (c0 + kChunk - rag.sh > len) {
                     // the lane holding the diagonal may have loaded columns past it
 #pragma unroll
                     for (int k = 0; k < 8; ++k)
@@ -650,6 +738,7 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void softmax_bwd_kernel(SoftmaxArg
                             if ((col + k) < lo) gv[k] = pv[k] = 0.f;
                     }
                 }
+                rag.own(gv, c0);
 #pragma unroll
                 for (int k = 0; k < 8; ++k) dot = fmaf(gv[k], pv[k], dot);
             }
@@ -657,34 +746,32 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void softmax_bwd_kernel(SoftmaxArg
         dot = wave_reduce<OpSum>(dot);
         dot = row_combine<OpSum, WPR, RPB>(dot, red_sum, wib, rib, lane);
 
-        char* dx = static_cast<char*>(a.out) + (size_t)pos.row * sk * 2;
-        const rsrc_t rdx = make_rsrc(dx, pos.store ? (uint32_t)sk * 2u : 0u);
+        const Rows<kStage, RPB> out(a, a.out, pos, rib, 0);
 #pragma unroll
         for (int c = 0; c < NCH; ++c) {
             const int c0 = (wch + WPR * c) * kChunk;
             u32x4 o = u32x4{0, 0, 0, 0};
-            if (c0 < plen && (!kBnd || c0 + kChunk > lo)) {
+            if (rag.chunk_col(c0) < len && (!kBnd || c0 + kChunk > lo)) {
                 float gv[8], pv[8];
                 unpack8<T>(rg[c], gv);
                 unpack8<T>(rp[c], pv);
-                const int col = c0 + lane * kVec - sh;
+                const int col = rag.col(c0);
 #pragma unroll
                 for (int k = 0; k < 8; ++k) {
                     if constexpr ((FLAGS & kDropout) != 0) gv[k] = ((kb[c] >> k) & 1u) ? gv[k] * drop.scale : 0.f;
                     gv[k] = a.scale * (pv[k] * (gv[k] - dot));
-                    if ((c0 + kChunk > plen) && (col + k) >= len) gv[k] = 0.f;
+                    if ((c0 + kChunk - rag.sh > len) && (col + k) >= len) gv[k] = 0.f;
                     if constexpr (kBnd) {
                         if (c0 < lo && (col + k) < lo) gv[k] = 0.f;
                     }
                 }
                 o = pack8<T>(gv);
             }
-            buf_st128<kStNt>(rdx, o, (c == 0 && first_lane) ? kOutOfRange : voff + c * WPR * kChunk * 2, 0);
-            if constexpr (kRag) {
-                if (c == 0 && head) ragged_head_store(rdx, o, first_lane);
-                if (c0 < sk + sh && c0 + kChunk >= sk + sh)
-                    ragged_store16(rdx, o, c0 + lane * kVec, sk + sh, (uint32_t)(sk - 1) * 2u);
-            }
+            out.template put<kStNt>(o, kRag ? rag.store_off(c0) : voff + c * WPR * kChunk * 2);
+        }
+        if constexpr (kStage) {
+            __syncthreads();
+            out.template flush<kStNt, kWave * WPR * RPB, NCH>();
         }
     }
 }
@@ -765,7 +852,6 @@ struct DirectSink {
         packed_st<NT>(out, v, off, active);
     }
 };
-struct __attribute__((packed, aligned(2))) Slot16 { u32x4 v; };  // 16 bytes at the alignment of an element
 struct StagedSink {
     char* lds;
     static __device__ __forceinline__ StagedSink at(void*, size_t, uint32_t, char* stage) { return {stage}; }

@@ -1,0 +1,148 @@
+"""Rows at any alignment through the row kernels: the lanes at the two ends of a row share columns with their
+neighbours, and one-wave rows leave through LDS in accesses aligned to cache lines.
+
+Against the fp32 expression, at the edges of the kernels' ranges (a last lane of 1 to 8 columns, a row end in the first lane
+of a chunk, the limits of the shapes), with tensors that begin at any element of a 16-byte slot, with a last block that is
+not full, in place, and with guard elements around every output: nothing outside of it is written.  The sums of a
+row are taken over the same terms in the same order whatever is folded in: zero slopes, a zero bias and dropout give
+the plain kernels' bits.
+"""
+import pytest
+import torch
+
+from gpt_neox_amd import _lib
+from oracle import torch_ref as R
+from bars import TOL, assert_grad
+
+pytestmark = pytest.mark.gpu
+
+GUARD = 64  # elements in front of and behind every output
+SCALE = 0.125
+# the limits of the shapes (672 and 944: staged; 1536 / 2048: chunks; 1856: two waves) and row ends in every place of a lane
+COLUMNS = [513, 520, 527, 671, 673, 943, 945, 1001, 1018, 1023, 1024, 1025, 1031, 1201, 1535, 1536, 1537, 1855, 1857, 2047, 2049, 4097]
+
+
+def at(offset, shape, dtype, device, fill=None, gen=None, std=1.0):
+    """A tensor that begins `offset` elements behind a 128-byte boundary, and the storage around it."""
+    n = 1
+    for d in shape:
+        n *= d
+    store = torch.full((GUARD + offset + n + GUARD,), 7.0, dtype=dtype, device=device)
+    t = store[GUARD + offset : GUARD + offset + n].view(shape)
+    if gen is not None:
+        t.normal_(0.0, std, generator=gen)
+    elif fill is not None:
+        t.copy_(fill)
+    return t, store
+
+
+def guarded(t, store):
+    lead = t.storage_offset()
+    return bool((store[:lead] == 7.0).all()) and bool((store[lead + t.numel() :] == 7.0).all())
+
+
+@pytest.mark.parametrize("sk", COLUMNS)
+@pytest.mark.parametrize("offsets", [(0, 0), (1, 0), (3, 5), (8, 1)])
+def test_ragged_rows(device, sk, offsets):
+    lib, stream = _lib.lib(), torch.cuda.current_stream().cuda_stream
+    dtype = (torch.float16, torch.bfloat16)[(sk + offsets[0]) % 2]
+    code = _lib.dtype_code(dtype)
+    gen = torch.Generator(device=device).manual_seed(sk)
+    b, heads, sq = 3, 1, 5  # fifteen rows: the last block of four is not full
+    rows = b * heads * sq
+    shape = (b, heads, sq, sk)
+    i, o = offsets
+    x, _ = at(i, shape, dtype, device, gen=gen, std=8.0)
+    g, _ = at(i, shape, dtype, device, gen=gen)
+    # causal rows of the full length: the last rows of a taller matrix
+    tall = (1, 1, sk, sk)
+    causal = torch.ones(sk, sk, dtype=torch.bool, device=device).triu_(1).view(tall)
+    xt, _ = at(i, tall, dtype, device, gen=gen, std=8.0)
+    gt, _ = at(i, tall, dtype, device, gen=gen)
+    lens = torch.tensor([sk, sk - 3, max(1, sk // 3)], device=device)
+    mask = (torch.arange(sk, device=device).view(1, 1, 1, sk) >= lens.view(b, 1, 1, 1)).expand(b, 1, sq, sk).contiguous()
+    mask[0, 0, 1] = True  # a row without a visible key
+    mask[0, 0, 2, ::3] = True
+
+    def forward(call, want_shape, inplace_of=None):
+        if inplace_of is None:
+            y, store = at(o, want_shape, dtype, device)
+        else:
+            y, store = at(i, want_shape, dtype, device, fill=inplace_of)
+        _lib.check(call(y))
+        assert guarded(y, store), (sk, offsets)
+        return y
+
+    cases = {
+        "causal": (xt, gt, causal, lambda y, src: lib.neox_causal_softmax_fwd(y.data_ptr(), src.data_ptr(), SCALE, 1, sk, sk, code, stream)),
+        "mask": (x, g, mask, lambda y, src: lib.neox_masked_softmax_fwd(
+            y.data_ptr(), src.data_ptr(), mask.data_ptr(), SCALE, b, heads, sq, sk, b, code, stream)),
+    }
+    for kind, (src, grad, hidden, call) in cases.items():
+        y = forward(lambda y: call(y, src), src.shape)
+        ref = R.softmax_fp32(src.cpu(), hidden.cpu(), SCALE).to(device)
+        assert (y.float() - ref).abs().max().item() <= TOL[dtype], (kind, sk, offsets)
+        seen = hidden.all(-1, keepdim=True)
+        assert (y[hidden.expand_as(y) & ~seen.expand_as(y)] == 0).all(), kind
+        inplace = forward(lambda y: call(y, y), src.shape, inplace_of=src)
+        if sk % 8 != 0 or i % 8 != 0 or o % 8 == 0:  # (else in place is aligned: another kernel, sums in another order)
+            assert torch.equal(inplace, y), kind
+        assert (inplace.float() - ref).abs().max().item() <= TOL[dtype], (kind, sk, offsets)
+        dx, store = at(o, src.shape, dtype, device)
+        same, same_store = at(i, src.shape, dtype, device, fill=grad)
+        for out, dy in ((dx, grad), (same, same)):
+            if kind == "causal":
+                _lib.check(lib.neox_causal_softmax_bwd(out.data_ptr(), dy.data_ptr(), y.data_ptr(), SCALE, 1, sk, sk, code, stream))
+            else:
+                _lib.check(lib.neox_masked_softmax_bwd(out.data_ptr(), dy.data_ptr(), y.data_ptr(), SCALE, rows, sk, code, stream))
+        assert guarded(dx, store) and guarded(same, same_store), (kind, sk, offsets)
+        assert torch.equal(dx, same), kind
+        yf, gf = y.float(), grad.float()
+        auto = SCALE * yf * (gf - (gf * yf).sum(-1, keepdim=True))
+        assert_grad(dx, auto, dtype, (kind, sk, offsets), y=y, g=grad, scale=SCALE)
+
+        # what is folded in leaves the sums as they are
+        shape4 = tuple(src.shape)
+        zero_bias, slopes = torch.zeros(shape4, dtype=dtype, device=device), torch.zeros(shape4[1], device=device)
+        for fold in ("alibi", "bias", "dropout"):
+            z, zs = at(o, src.shape, dtype, device)
+            extra = (slopes.data_ptr() if fold == "alibi" else None, zero_bias.data_ptr() if fold == "bias" else None, shape4[0])
+            p = 0.25 if fold == "dropout" else 0.0
+            drop, ds = at(o, src.shape, dtype, device)
+            if fold == "dropout":
+                if kind == "causal":
+                    _lib.check(lib.neox_causal_softmax_dropout_fwd(drop.data_ptr(), z.data_ptr(), src.data_ptr(), *extra, SCALE, p, 5, 0, None,
+                                                                   *shape4, code, stream))
+                else:
+                    _lib.check(lib.neox_masked_softmax_dropout_fwd(drop.data_ptr(), z.data_ptr(), src.data_ptr(), mask.data_ptr(), *extra,
+                                                                   SCALE, p, 5, 0, None, *shape4, b, code, stream))
+                keep = torch.empty(src.numel(), dtype=torch.uint8, device=device)
+                _lib.check(lib.neox_dropout_keep_mask(keep.data_ptr(), p, 5, 0, None, src.numel(), stream))
+                assert torch.equal(drop, torch.where(keep.view(src.shape).bool(), (y.float() * (1.0 / 0.75)).to(dtype), 0)), kind
+            elif kind == "causal":
+                if fold == "alibi":
+                    _lib.check(lib.neox_causal_softmax_alibi_fwd(z.data_ptr(), src.data_ptr(), extra[0], SCALE, *shape4, code, stream))
+                else:
+                    _lib.check(lib.neox_causal_softmax_bias_fwd(z.data_ptr(), src.data_ptr(), extra[1], None, SCALE, *shape4, shape4[0], code, stream))
+            elif fold == "alibi":
+                _lib.check(lib.neox_masked_softmax_alibi_fwd(z.data_ptr(), src.data_ptr(), mask.data_ptr(), extra[0], SCALE, *shape4, b, code, stream))
+            else:
+                _lib.check(lib.neox_masked_softmax_bias_fwd(z.data_ptr(), src.data_ptr(), mask.data_ptr(), extra[1], None, SCALE, *shape4, b,
+                                                            shape4[0], code, stream))
+            assert guarded(z, zs) and guarded(drop, ds), (kind, fold, sk)
+            assert torch.equal(z, y), (kind, fold, sk, offsets)
+
+
+@pytest.mark.parametrize("sk", [513, 1001, 1201, 1999, 3001])
+def test_one_ragged_row(device, sk):
+    # a single row: the lanes at its ends have no neighbouring row to share anything with
+    lib, stream = _lib.lib(), torch.cuda.current_stream().cuda_stream
+    gen = torch.Generator(device=device).manual_seed(sk)
+    x, _ = at(1, (1, 1, 1, sk), torch.float16, device, gen=gen, std=8.0)
+    mask = torch.zeros(1, 1, 1, sk, dtype=torch.bool, device=device)
+    mask[..., sk // 2 : sk // 2 + 9] = True
+    y, store = at(1, x.shape, torch.float16, device)
+    _lib.check(lib.neox_masked_softmax_fwd(y.data_ptr(), x.data_ptr(), mask.data_ptr(), SCALE, 1, 1, 1, sk, 1, _lib.NEOX_F16, stream))
+    assert guarded(y, store)
+    ref = R.softmax_fp32(x.cpu(), mask.cpu(), SCALE).to(device)
+    assert (y.float() - ref).abs().max().item() <= TOL[torch.float16]
