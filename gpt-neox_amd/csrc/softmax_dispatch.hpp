@@ -14,8 +14,9 @@
 //   chunks <= 16   8 waves per row, 512-thread block                 (sk <= 8192)
 //   chunks <= 32   16 waves per row, 1024-thread block               (sk <= 16384)
 //                  forward, in the lower 3/4 of each of these three ranges (7/8 of the last):
-//                  half as many waves with 3 (4) chunks each; causal backward likewise at
-//                  8193-12288 columns; mask-tensor forward at 513-2048 columns (unless the call
+//                  half as many waves with 3 (4) chunks each; backward (the last range: causal) likewise at
+//                  2049-3072, 4097-6144 (full rows: 4608) and 8193-12288 columns; mask-tensor forward at 513-2048
+//                  columns (unless the call
 //                  knows where its rows end) and causal forward at 1025-1408: packed kernel, two
 //                  rows of two chunks or one row of three or four chunks per wave
 //   chunks <= 64   16 waves per row with 3 or 4 chunks per wave      (sk <= 32768)
@@ -85,7 +86,7 @@ static hipError_t launch_shape(const SoftmaxArgs& a0, hipStream_t st) {
     constexpr int FLAGS = kDefaultFlags | EXTRA;
     constexpr bool staged = (EXTRA & kStaged) != 0;  // a block's rows then are one run: rows in order
     const SoftmaxArgs a = with_xcd_mapping(a0, staged || (WPR == 1 && unit_bytes > 4096) ? 0 : unit_bytes, RPB, grid.x);
-    const uint32_t lds = staged ? stage_bytes(RPB, (uint32_t)a0.sk) * (!BWD && (EXTRA & kDropout) != 0 ? 2 : 1) : 0;
+    const uint32_t lds = staged ? stage_bytes(RPB, (uint32_t)a0.sk) : 0;
     if constexpr (BWD) {
         hipLaunchKernelGGL((softmax_bwd_kernel<T, NCH, WPR, RPB, M, FLAGS>), grid, block, lds, st, a);
     } else {
@@ -283,6 +284,13 @@ static std::optional<hipError_t> dispatch_aligned(const SoftmaxArgs& a, bool vec
         const bool fits32 = a.bias == nullptr || a.bias_bytes != 0;
         if (chunks == 3 && a.sk <= 1408 && fits32) return launch_packed_shape<T, M, BWD, EXTRA, kWave, 1, 3>(a, st);
     }
+    if constexpr (BWD && M == Mask::Causal && (EXTRA & kDropout) != 0) {
+        // causal backward with dropout, 1025-1344 columns: one wave per row with three chunks, two rows per block; the Philox rounds of
+        // a fourth chunk slot are work for nothing.  us per launch, fp16, two waves per row -> one: [113,1088,1088] 104.9 -> 93.0, [81,1280,1280]
+        // 96.8 -> 90.7, [67,1408,1408] 94.0 -> 90.3, [61,1472,1472] 90.7 -> 90.1, but [8,1408,1408] 14.8 -> 15.3; without dropout +1...+3 % throughout,
+        // and with few rows [1,1280,1280] 4.5 -> 5.0, [3,1280,1280] 6.6 -> 7.4, [4,1088,1088] 7.7 -> 7.3
+        if (chunks == 3 && a.sk <= 1344 && a.rows >= 4608) return launch_shape<T, M, BWD, EXTRA, 3, 1, 2>(a, st);
+    }
     if constexpr (BWD && M == Mask::None) {
         // full rows up to 2048 columns: straight-line packed kernel, R x C = 4 accesses per tensor
         if (chunks == 2) return launch_packed_shape<T, M, BWD, EXTRA, kWave, 2, 2>(a, st);
@@ -325,9 +333,13 @@ static bool two_causal_rows(const SoftmaxArgs& a, int chunks) {
 //   70.3 -> 70.9, [33,2001,2001] 69.3 -> 74.7, the others there 0...-4 %
 // with ALiBi [60,1049,1049] 44.8 -> 36.3, [20,1801,1801] 36.4 -> 36.1, with a bias 47.7 -> 41.2 and 41.2 -> 40.6, with dropout 76.9 ->
 // 67.0 and 64.3 -> 64.7, its backward 65.4 -> 58.7 and 56.1 -> 53.9.  All feature sets take the same shape: the same sums.
-// (two_waves_ragged: what keeps two waves for the longest of them.)
+// The backward pass with few rows keeps two waves: full rows [1,1601,1601] 6.0 -> 6.3, [4,1601,1601] 13.8 -> 14.1, causal [1,1601,1601]
+// 4.9 -> 5.1, [2,1601,1601] 7.5 -> 6.8, [1,1301,1301] level.
 template <Mask M, bool BWD>
-constexpr bool two_waves_ragged = !BWD && M == Mask::Causal;
+static bool one_wave_ragged(const SoftmaxArgs& a, int chunks) {
+    if constexpr (!BWD) return M != Mask::Causal || a.sk <= 1856;
+    return M == Mask::None ? a.rows >= 8192 : chunks == 3 || a.rows >= 2048;
+}
 
 template <typename T, Mask M, bool BWD, int EXTRA>
 static hipError_t dispatch_rows(const SoftmaxArgs& a, bool vec_ok, hipStream_t st) {
@@ -360,7 +372,8 @@ static hipError_t dispatch_rows(const SoftmaxArgs& a, bool vec_ok, hipStream_t s
                 // elements, direct -> staged: forward [92,851,851] 36.9 -> 37.5, [82,901,901] 36.9 -> 36.8, [74,951,951] 36.6 -> 36.2,
                 // [64,1022,1022] 36.7 -> 36.1, backward [185,601,601] 50.0 both, [136,701,701] 49.6 -> 48.8, [65,1009,1009] 48.4 -> 47.1;
                 // with dropout behind throughout ([96,1001,1001] 94.2 -> 96.1 and 86.6 -> 90.0)
-                if (a.sk >= (BWD ? 672 : 944)) return launch_shape<T, M, BWD, EXTRA | kStaged, 2, 1, 4>(a, st);
+                // ([4,1001,1001] forward 4.73 -> 4.82, [1,1001,1001] 3.55 -> 3.62: not with few rows)
+                if (a.sk >= (BWD ? 672 : 944) && a.rows >= 8192) return launch_shape<T, M, BWD, EXTRA | kStaged, 2, 1, 4>(a, st);
             }
             return launch_shape<T, M, BWD, EXTRA, 2, 1, 4>(a, st);
         }
@@ -378,12 +391,19 @@ static hipError_t dispatch_rows(const SoftmaxArgs& a, bool vec_ok, hipStream_t s
             // mask-tensor forward with dropout, [8,7,1049,1049] 95.4 and 99.3, [8,3,1601,1601] 84.2 and 88.0
             constexpr bool staged = (EXTRA & kDropout) == 0 || (!BWD && M == Mask::Causal);
             constexpr int FL = EXTRA | (staged ? kStaged : 0);
-            if (chunks == 3) return launch_shape<T, M, BWD, FL, 3, 1, 4>(a, st);
-            if (chunks == 4 && (!two_waves_ragged<M, BWD> || a.sk <= 1856)) return launch_shape<T, M, BWD, FL, 4, 1, 4>(a, st);
-        } else {
+            if (chunks <= 4 && one_wave_ragged<M, BWD>(a, chunks)) {
+                // with dropout, few rows: [3,1701,1701] 13.1 us with two waves, 11.2 staged, 10.2 not; [4,1801,1801] 17.3, 15.4, 18.1;
+                // [1,1601,1601] 7.2, 7.8, 6.7
+                if constexpr (staged && (EXTRA & kDropout) != 0) {
+                    if (a.rows < 6400) return chunks == 3 ? launch_shape<T, M, BWD, EXTRA, 3, 1, 4>(a, st) : launch_shape<T, M, BWD, EXTRA, 4, 1, 4>(a, st);
+                }
+                return chunks == 3 ? launch_shape<T, M, BWD, FL, 3, 1, 4>(a, st) : launch_shape<T, M, BWD, FL, 4, 1, 4>(a, st);
+            }
+        }
+        if constexpr (!ragged || (BWD && M == Mask::None)) {
             if (chunks == 3) return launch_shape<T, M, BWD, EXTRA, 2, 2, 2>(a, st);
         }
-        if constexpr (!ragged || two_waves_ragged<M, BWD>) {
+        if constexpr (!ragged || BWD || M == Mask::Causal) {
             if (chunks == 4) {
                 // the causal forward with two output streams (dropout) measured 3 % faster with 2 rows
                 if constexpr (!BWD && M == Mask::Causal && (EXTRA & kDropout) != 0)
@@ -396,17 +416,36 @@ static hipError_t dispatch_rows(const SoftmaxArgs& a, bool vec_ok, hipStream_t s
         // Forward, rows that would leave a quarter or more of the 2-chunk shape's slots empty:
         // half as many waves with 3 or 4 chunks each.  Measured in an interleaved comparison:
         // +20-50 % just above a power of two (2056, 4104, 8200 columns), +4-15 % up to 3/4 (7/8 with
-        // 4 chunks) of the range, while full rows lose 2-3 % with 4 chunks per wave and the
-        // backward pass gains nothing.
+        // 4 chunks) of the range, while full rows lose 2-3 % with 4 chunks per wave.
         if (chunks <= 6) return launch_shape<T, M, BWD, EXTRA, 3, 2, 2>(a, st);
         if (chunks > 8 && chunks <= 12) return launch_shape<T, M, BWD, EXTRA, 3, 4, 1>(a, st);
         if (chunks > 16 && chunks <= 24) return launch_shape<T, M, BWD, EXTRA, 3, 8, 1>(a, st);
         if (chunks > 24 && chunks <= 28) return launch_shape<T, M, BWD, EXTRA, 4, 8, 1>(a, st);
     }
+    if constexpr (BWD && (EXTRA & kBand) == 0) {
+        // Backward likewise, where it gains: rows of five and six chunks in two waves, rows of nine and more in four.  us per launch,
+        // fp16, 2^27 elements, two chunks per wave -> three, causal / full rows / both with dropout:
+        //   [30,2112,2112] 88.9 -> 88.1 / 87.8 -> 81.6 / 102.7 -> 90.4 / 119.6 -> 104.4, [20,2560,2560] 87.9 -> 86.5 / 82.2 -> 82.6 /
+        //     93.3 -> 87.8 / 102.0 -> 96.3, [14,3072,3072] 88.6 -> 86.7 / 61.7 -> 61.1 / 90.6 -> 87.5 / 70.2 -> 67.7; ragged [31,2051,2051]
+        //     93.9 -> 92.1, its results staged 89.9, with dropout 118.6 -> 106.7; [14,3071,3071] 91.5 -> 93.2, staged 89.6
+        //   [7,4160,4160] 88.5 -> 80.1 / 98.3 -> 83.1 / 95.8 -> 83.5 / 135.6 -> 114.2, [5,5120,5120] 89.8 -> 87.5 / 103.8 -> 102.9 / 95.8 -> 88.7 /
+        //     126.2 -> 110.5, [3,6144,6144] 75.6 -> 74.8 / 88.8 -> 91.1 / 78.6 -> 75.5 / 110.3 -> 107.6
+        //   with few rows: causal [1,2112,2112] 5.9 -> 6.1, with dropout [2,2112,2112] 10.0 -> 10.9, [4,2112,2112] level, full rows [1,2112,2112] 8.0
+        //     -> 7.5, ragged [1,2901,2901] 11.7 -> 11.9, [4,2901,2901] 35.2 -> 35.7
+        // Full rows without dropout: only if the call knows where the rows of several samples end (the figures above); without a hidden tail
+        // [1,30,2112,2112] 124.7 -> 127.5, [1,8,4608,4608] 158.3 -> 163.7, [1,8,5120,5120] 194.1 -> 203.9 (with dropout [1,8,5120,5120]
+        // 212.9 -> 199.9, [1,8,6144,6144] 291.1 -> 290.1).
+        constexpr bool ends = M == Mask::None && (EXTRA & kDropout) == 0;
+        bool enough = !ends || (a.row_end != nullptr && !a.mask_bcast && a.rows > a.by_mask_batch.d);  // (several samples)
+        const bool four = enough && chunks > 8 && chunks <= (M == Mask::Causal ? 12 : ends ? 9 : 10);
+        if (M == Mask::Causal) enough = a.rows >= 4608;
+        if (EXTRA == kRagged && M == Mask::None) enough = enough && a.rows >= 8192 && a.sk <= 2304;
+        if (chunks <= 6 && enough) return launch_shape<T, M, BWD, EXTRA | (EXTRA == kRagged ? kStaged : 0), 3, 2, 2>(a, st);
+        if (four) return launch_shape<T, M, BWD, EXTRA, 3, 4, 1>(a, st);
+    }
     if constexpr (BWD && M == Mask::Causal) {
         // Causal backward just above 8192 columns: 8 waves with 3 chunks each instead of 16 with 2, of
-        // which up to half would hold nothing (-13 % at 8200 columns, -8 % at 10240, -4 % at 12288).  The
-        // same step at the shorter ranges and for the full-row backward measured -3...+5 %: not taken.
+        // which up to half would hold nothing (-13 % at 8200 columns, -8 % at 10240, -4 % at 12288).
         if (chunks > 16 && chunks <= 24) return launch_shape<T, M, BWD, EXTRA, 3, 8, 1>(a, st);
     }
     if constexpr ((EXTRA & kBand) != 0) {

@@ -367,14 +367,14 @@ struct RaggedRow<true> {
 // arithmetic, causal rows of 1001 columns, runs at 5.2 TB/s that way and at 5.6 staged, full rows at 5.9 and 6.2.
 struct __attribute__((packed, aligned(2))) Slot16 { u32x4 v; };  // 16 bytes at the alignment of an element
 constexpr int kLine = 128;
-// LDS of one output of a block of `rows` rows
+// LDS of a block of `rows` rows
 __host__ __device__ constexpr uint32_t stage_bytes(uint32_t rows, uint32_t sk) { return (rows * sk * 2 + kLine + 31) & ~15u; }
 extern __shared__ __attribute__((aligned(16))) char lds_stage[];
 
 template <bool ST, int RPB>
 struct Rows {
     rsrc_t row;
-    __device__ __forceinline__ Rows(const SoftmaxArgs& a, void* out, const RowPos& pos, int, int) {
+    __device__ __forceinline__ Rows(const SoftmaxArgs& a, void* out, const RowPos& pos, int) {
         row = make_rsrc(static_cast<char*>(out) + (size_t)pos.row * a.sk * 2, pos.store ? (uint32_t)a.sk * 2u : 0u);
     }
     template <bool NT>
@@ -388,13 +388,13 @@ struct Rows<true, RPB> {
     uint32_t end;    // of the run, counted from that line
     char* row;       // the wave's row in LDS (a surplus row: behind the run, where nothing is taken from)
     uint32_t spare;  // 16 bytes for the lanes behind the row, counted from `row`
-    __device__ __forceinline__ Rows(const SoftmaxArgs& a, void* out, const RowPos&, int rib, int which) {
+    __device__ __forceinline__ Rows(const SoftmaxArgs& a, void* out, const RowPos&, int rib) {
         const uint32_t row0 = blockIdx.x * RPB, size = stage_bytes(RPB, a.sk);
         mem = static_cast<char*>(out) + (size_t)row0 * a.sk * 2;
         head = (uint32_t)(reinterpret_cast<uintptr_t>(mem) & (kLine - 1));
         mem -= head;
         end = head + min((uint32_t)RPB, a.rows - row0) * a.sk * 2;
-        stage = lds_stage + which * size;
+        stage = lds_stage;
         row = stage + head + rib * a.sk * 2;
         spare = size - 16 - (uint32_t)(row - stage);
     }
@@ -606,7 +606,7 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void softmax_fwd_kernel(SoftmaxArg
         const float inv = 1.0f / sum;
 
         // ---- normalise and store; chunks above the diagonal store zeros
-        const Rows<kStage, RPB> out(a, a.out, pos, rib, 0);
+        const Rows<kStage, RPB> out(a, a.out, pos, rib);
         u32x4 o[NCH];
 #pragma unroll
         for (int c = 0; c < NCH; ++c) {
@@ -619,9 +619,14 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void softmax_fwd_kernel(SoftmaxArg
             }
             out.template put<kStNt>(o[c], kRag ? rag.store_off(c0) : voff + c * WPR * kChunk * 2);
         }
+        if constexpr (kStage) {
+            __syncthreads();
+            out.template flush<kStNt, kWave * WPR * RPB, NCH>();
+            if constexpr ((FLAGS & kDropout) != 0) __syncthreads();
+        }
         if constexpr ((FLAGS & kDropout) != 0) {
             // second output after the first: each stream is written in runs of whole rows
-            const Rows<kStage, RPB> out2(a, a.out2, pos, rib, 1);
+            const Rows<kStage, RPB> out2(a, a.out2, pos, rib);
 #pragma unroll
             for (int c = 0; c < NCH; ++c) {
                 const int c0 = (wch + WPR * c) * kChunk;
@@ -634,12 +639,8 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void softmax_fwd_kernel(SoftmaxArg
             }
             if constexpr (kStage) {
                 __syncthreads();
-                out.template flush<kStNt, kWave * WPR * RPB, NCH>();
                 out2.template flush<kStNt, kWave * WPR * RPB, NCH>();
             }
-        } else if constexpr (kStage) {
-            __syncthreads();
-            out.template flush<kStNt, kWave * WPR * RPB, NCH>();
         }
     }
 }
@@ -746,7 +747,7 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void softmax_bwd_kernel(SoftmaxArg
         dot = wave_reduce<OpSum>(dot);
         dot = row_combine<OpSum, WPR, RPB>(dot, red_sum, wib, rib, lane);
 
-        const Rows<kStage, RPB> out(a, a.out, pos, rib, 0);
+        const Rows<kStage, RPB> out(a, a.out, pos, rib);
 #pragma unroll
         for (int c = 0; c < NCH; ++c) {
             const int c0 = (wch + WPR * c) * kChunk;
