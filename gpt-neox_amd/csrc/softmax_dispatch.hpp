@@ -15,7 +15,7 @@
 //   chunks <= 32   16 waves per row, 1024-thread block               (sk <= 16384)
 //                  forward, in the lower 3/4 of each of these three ranges (7/8 of the last):
 //                  half as many waves with 3 (4) chunks each; backward (the last range: causal) likewise at
-//                  2049-3072, 4097-6144 (full rows: 4608) and 8193-12288 columns; mask-tensor forward at 513-2048
+//                  2049-3072 (full rows: 2560), 4097-6144 (4608) and 8193-12288 columns; mask-tensor forward at 513-2048
 //                  columns (unless the call
 //                  knows where its rows end) and causal forward at 1025-1408: packed kernel, two
 //                  rows of two chunks or one row of three or four chunks per wave
@@ -375,7 +375,17 @@ static hipError_t dispatch_rows(const SoftmaxArgs& a, bool vec_ok, hipStream_t s
                 // ([4,1001,1001] forward 4.73 -> 4.82, [1,1001,1001] 3.55 -> 3.62: not with few rows)
                 if (a.sk >= (BWD ? 672 : 944) && a.rows >= 8192) return launch_shape<T, M, BWD, EXTRA | kStaged, 2, 1, 4>(a, st);
             }
-            return launch_shape<T, M, BWD, EXTRA, 2, 1, 4>(a, st);
+            if constexpr (M == Mask::Causal && (EXTRA & (kRagged | kBand)) == 0) {
+                // Both chunks' loads in front of the first one's arithmetic.  us per launch, fp16, without -> with: forward [4,960,960] 5.0 -> 3.8,
+                // [16,640,640] 6.7 -> 5.9, [404,576,576] 74.2 -> 72.0, [128,1024,1024] 65.6 -> 64.5; with dropout [8,832,832] 8.2 -> 6.4, its
+                // backward [4,768,768] 5.2 -> 4.6, [227,768,768] 104.6 -> 101.8; backward [4,832,832] 5.0 -> 4.1, [64,640,640] 21.8 -> 20.0,
+                // [404,576,576] 97.5 -> 92.0, [193,832,832] 90.6 -> 89.8, but [8,896,896] 6.7 -> 7.0, [128,1024,1024] 86.0 -> 87.9 (two input
+                // streams, more of their loads at once); [4,1024,1024] 5.5 -> 5.4.  (With a mask tensor or a window 0...+6 %: not there.)
+                const bool early = !BWD || (EXTRA & kDropout) != 0 || a.sk <= 880 || a.rows <= 4608;
+                if (early) return launch_shape<T, M, BWD, EXTRA | kEarly, 2, 1, 4>(a, st);
+            }
+            if constexpr (!(M == Mask::Causal && (EXTRA & (kRagged | kBand)) == 0) || (BWD && (EXTRA & kDropout) == 0))
+                return launch_shape<T, M, BWD, EXTRA, 2, 1, 4>(a, st);
         }
         if constexpr ((EXTRA & kBand) != 0) {
             // rows that are mostly zeros in front of and behind the band: twice the waves, one chunk of the band each.
@@ -439,6 +449,7 @@ static hipError_t dispatch_rows(const SoftmaxArgs& a, bool vec_ok, hipStream_t s
         bool enough = !ends || (a.row_end != nullptr && !a.mask_bcast && a.rows > a.by_mask_batch.d);  // (several samples)
         const bool four = enough && chunks > 8 && chunks <= (M == Mask::Causal ? 12 : ends ? 9 : 10);
         if (M == Mask::Causal) enough = a.rows >= 4608;
+        if (ends && chunks == 6) enough = false;  // [8,5,3000,3000] 259.5 -> 267, [8,2,2816,2816] 98.2 -> 98.7
         if (EXTRA == kRagged && M == Mask::None) enough = enough && a.rows >= 8192 && a.sk <= 2304;
         if (chunks <= 6 && enough) return launch_shape<T, M, BWD, EXTRA | (EXTRA == kRagged ? kStaged : 0), 3, 2, 2>(a, st);
         if (four) return launch_shape<T, M, BWD, EXTRA, 3, 4, 1>(a, st);

@@ -98,6 +98,8 @@ constexpr int kRagged = 32;
 constexpr int kBand = 64;
 // Ragged row kernels only: the block's results go through LDS (see Rows).
 constexpr int kStaged = 128;
+// Row kernels: loads_first, which kRagged has anyway.
+constexpr int kEarly = 256;
 constexpr int kDefaultFlags = kNtLoad | kNtStore;
 
 // kRagged: 1 if the row starts on an odd element (2 mod 4 bytes) of the tensor at `base` and sk is
@@ -516,7 +518,7 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void softmax_fwd_kernel(SoftmaxArg
             for (int c = 0; c < NCH; ++c) rawb[c] = buf_ld128<false>(rb, lane_off(c, 2), 0);
         }
     }
-    if constexpr (kRag) loads_first();
+    if constexpr (kRag || (FLAGS & kEarly) != 0) loads_first();
     if constexpr (kBnd) {
         // while the loads are in flight: the zeros of the chunks that no wave holds
         const rsrc_t rz = make_rsrc(static_cast<char*>(a.out) + (size_t)pos.row * sk * 2, pos.store ? (uint32_t)sk * 2u : 0u);
@@ -698,7 +700,7 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void softmax_bwd_kernel(SoftmaxArg
                 rg[c] = buf_ld128<kLdNt>(bg, all_zero(rp[c]) ? kOutOfRange : voff + c * WPR * kChunk * 2, 0);
         }
     }
-    if constexpr (kRag) loads_first();
+    if constexpr (kRag || (FLAGS & kEarly) != 0) loads_first();
     if constexpr (kBnd) {
         // the zeros of the chunks that no wave holds.  dx may alias dy: those chunks lie outside the
         // band, where nothing is read
