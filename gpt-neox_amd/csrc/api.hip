@@ -198,7 +198,7 @@ struct SoftmaxCall {
     int launch(bool backward, Mask m, void* stream) const {
         const bool vec = vec_ok && a.sk % kVec == 0;
         int flags = backward ? (features & kDropout) : features;
-        if (!vec && a.sk >= kVec && a.sk < kMaxStagedRow) flags |= kRagged;
+        if ((!vec && a.sk >= kVec && a.sk < kMaxStagedRow) || (vec && through_lds(backward, m))) flags |= kRagged;
         const hipError_t e = backward ? launch_softmax_bwd(flags, a, m, dtype, vec, (hipStream_t)stream)
                                       : launch_softmax_fwd(flags, a, m, dtype, vec, (hipStream_t)stream);
         return check_launch(e, what);
@@ -206,6 +206,28 @@ struct SoftmaxCall {
 
   private:
     bool misaligned_ = false;
+
+    // Aligned rows that are no whole number of cache lines, many of them: by the kRagged unit too, whose one-wave kernels store a
+    // block's rows in accesses aligned to lines (see Rows), where the row kernels store parts of lines at both ends of every access.
+    // us per launch, fp16, 2^27 elements, aligned unit -> ragged unit:
+    //   causal forward   [319,648,648] 43.2 -> 42.6, [134,1000,1000] 71.4 -> 68.8, [126,1032,1032] 74.7 -> 69.3, [67,1416,1416] -2.2 %, [51,1608,1608]
+    //                    -1.4 %, [440,552,552] +1.6 %; with ALiBi or dropout -2...-17 % at 1025-1480 columns, +7...-2 % below (the same sums
+    //                    either way), [57,1528,1528] with dropout +3 % (other sums: neither goes)
+    //   causal backward  520-3064 columns -1...-7 %: [496,520,520] -6.4 %, [134,1000,1000] -4.4 %, [31,2056,2056] -4.6 %; with dropout +1...+7 %
+    //   mask tensor with known row ends: forward 832-2048 columns 0...-8 %, [8,26,712,712] -1.6 %, [8,25,800,800] +1.2 %, [8,61,520,520] +5 %;
+    //                    backward 513-2048 columns -0.3...-8 %; without the ends the aligned kernels fetch no hidden key: +5...+14 %
+    // Few rows do not fill the staged kernels' longer chain: [9,1032,1032] backward +3 %, mask-tensor +3 and +8 %, [9,1656,1656] +1 %.
+    bool through_lds(bool backward, Mask m) const {
+        if (a.rows < 32768 || a.sk <= kChunk || a.sk % (kLine / 2) == 0) return false;
+        const bool plain = (features & (kAlibi | kBias | kDropout)) == 0;
+        if (backward) {
+            if ((features & kDropout) != 0) return false;
+            if (m == Mask::Causal) return a.sk <= 3072;
+            return a.row_end != nullptr && a.sk <= 2048;
+        }
+        if (m == Mask::Causal) return a.sk <= 1480 && a.sk >= (plain ? 640 : 1025);
+        return plain && a.row_end != nullptr && a.sk >= 832 && a.sk <= 2048;
+    }
 
     void rows(int64_t n, int sq, int sk) {
         if ((status = check_rows(n, sq, sk, what)) != NEOX_OK) return;
