@@ -14,8 +14,8 @@
 //   chunks <= 16   8 waves per row, 512-thread block                 (sk <= 8192)
 //   chunks <= 32   16 waves per row, 1024-thread block               (sk <= 16384)
 //                  forward, in the lower 3/4 of each of these three ranges (7/8 of the last):
-//                  half as many waves with 3 (4) chunks each; backward (the last range: causal) likewise at
-//                  2049-3072 (full rows: 2560), 4097-6144 (4608) and 8193-12288 columns; mask-tensor forward at 513-2048
+//                  half as many waves with 3 (4) chunks each; backward (causal, or with dropout) likewise at
+//                  2049-3072, 4097-6144 and 8193-12288 columns; mask-tensor forward at 513-2048
 //                  columns (unless the call
 //                  knows where its rows end) and causal forward at 1025-1408: packed kernel, two
 //                  rows of two chunks or one row of three or four chunks per wave
@@ -26,11 +26,11 @@
 //                  the same packed, one- to sixteen-wave row and LDS-staged kernels with the kRagged flag; three and
 //                  four chunks (causal forward: up to 1856 columns) in one wave, results of one-wave rows staged
 //                  in LDS (kStaged)
-//   sliding window (kBand) the one- to sixteen-wave row kernels, aligned rows of 513-32768 columns, by the
-//                  chunks the band can touch
+//   sliding window (kBand) the row kernels, aligned rows of 513-32768 columns: dispatch_band_rows
 //   anything else  element-wise kernels (rows shorter than 8 columns or beyond 81408)
 #pragma once
 
+#include <algorithm>
 #include <optional>
 #include <type_traits>
 
@@ -344,14 +344,7 @@ static bool one_wave_ragged(const SoftmaxArgs& a, int chunks) {
 template <typename T, Mask M, bool BWD, int EXTRA>
 static hipError_t dispatch_rows(const SoftmaxArgs& a, bool vec_ok, hipStream_t st) {
     int chunks = (a.sk + kChunk - 1) / kChunk;
-    if constexpr ((EXTRA & kBand) != 0) {
-        // sliding-window rows: the row kernels below only (aligned rows of two chunks or more), and the
-        // kernel shape goes by the chunks a band can touch -- w + 1 keys lie in at most w / 512 + 2
-        // chunks -- not by the row length: the waves hold the band, the rest of the row is zeros
-        if (!vec_ok || chunks < 2 || a.sk > kMaxRegisterRow) return hipErrorInvalidValue;  // the caller checks
-        const int band_chunks = a.window / kChunk + 2;
-        if (band_chunks < chunks) chunks = band_chunks;
-    } else if constexpr ((EXTRA & kRagged) != 0) {
+    if constexpr ((EXTRA & kRagged) != 0) {
         // rows at any alignment: the packed kernels up to 512 columns, the row kernels below beyond
         if (a.sk < kVec || a.sk >= kMaxLdsRow) return hipErrorInvalidValue;  // the caller checks
         if (a.sk >= kMaxRegisterRow) return launch_lds<T, M, BWD, EXTRA>(a, st);
@@ -375,7 +368,7 @@ static hipError_t dispatch_rows(const SoftmaxArgs& a, bool vec_ok, hipStream_t s
                 // ([4,1001,1001] forward 4.73 -> 4.82, [1,1001,1001] 3.55 -> 3.62: not with few rows)
                 if (a.sk >= (BWD ? 672 : 944) && a.rows >= 8192) return launch_shape<T, M, BWD, EXTRA | kStaged, 2, 1, 4>(a, st);
             }
-            if constexpr (M == Mask::Causal && (EXTRA & (kRagged | kBand)) == 0) {
+            if constexpr (M == Mask::Causal && (EXTRA & kRagged) == 0) {
                 // Both chunks' loads in front of the first one's arithmetic.  us per launch, fp16, without -> with: forward [4,960,960] 5.0 -> 3.8,
                 // [16,640,640] 6.7 -> 5.9, [404,576,576] 74.2 -> 72.0, [128,1024,1024] 65.6 -> 64.5; with dropout [8,832,832] 8.2 -> 6.4, its
                 // backward [4,768,768] 5.2 -> 4.6, [227,768,768] 104.6 -> 101.8; backward [4,832,832] 5.0 -> 4.1, [64,640,640] 21.8 -> 20.0,
@@ -384,16 +377,8 @@ static hipError_t dispatch_rows(const SoftmaxArgs& a, bool vec_ok, hipStream_t s
                 const bool early = !BWD || (EXTRA & kDropout) != 0 || a.sk <= 880 || a.rows <= 4608;
                 if (early) return launch_shape<T, M, BWD, EXTRA | kEarly, 2, 1, 4>(a, st);
             }
-            if constexpr (!(M == Mask::Causal && (EXTRA & (kRagged | kBand)) == 0) || (BWD && (EXTRA & kDropout) == 0))
+            if constexpr (!(M == Mask::Causal && (EXTRA & kRagged) == 0) || (BWD && (EXTRA & kDropout) == 0))
                 return launch_shape<T, M, BWD, EXTRA, 2, 1, 4>(a, st);
-        }
-        if constexpr ((EXTRA & kBand) != 0) {
-            // rows that are mostly zeros in front of and behind the band: twice the waves, one chunk of the band each.
-            // us per launch forward / backward, two chunks per wave -> one: [8,8192,8192] window 1024 220 -> 207 / 241 -> 236,
-            // [20,5000,5000] window 1250 252 -> 236 / 294 -> 274, [4,12288,12288] 1500 272 -> 243 / 280 -> 270, [3,14336,14336] 1024
-            // 273 -> 260 / 268 -> 254; behind at 3000 columns (+2 / -3 %) and beyond 28 chunks: [2,15360,15360] 1024 200 -> 204 /
-            // 207 -> 203, [2,16384,16384] 1500 210 -> 232 / 223 -> 232, [1,32768,32768] 1024 408 -> 446 / 431 -> 460
-            if (a.sk > 4096 && a.sk <= 28 * kChunk && (chunks == 3 || chunks == 4)) return launch_shape<T, M, BWD, EXTRA, 1, 4, 1>(a, st);
         }
         constexpr bool ragged = (EXTRA & kRagged) != 0;
         if constexpr (ragged) {
@@ -422,7 +407,7 @@ static hipError_t dispatch_rows(const SoftmaxArgs& a, bool vec_ok, hipStream_t s
             }
         }
     }
-    if constexpr (!BWD && (EXTRA & kBand) == 0) {
+    if constexpr (!BWD) {
         // Forward, rows that would leave a quarter or more of the 2-chunk shape's slots empty:
         // half as many waves with 3 or 4 chunks each.  Measured in an interleaved comparison:
         // +20-50 % just above a power of two (2056, 4104, 8200 columns), +4-15 % up to 3/4 (7/8 with
@@ -432,7 +417,7 @@ static hipError_t dispatch_rows(const SoftmaxArgs& a, bool vec_ok, hipStream_t s
         if (chunks > 16 && chunks <= 24) return launch_shape<T, M, BWD, EXTRA, 3, 8, 1>(a, st);
         if (chunks > 24 && chunks <= 28) return launch_shape<T, M, BWD, EXTRA, 4, 8, 1>(a, st);
     }
-    if constexpr (BWD && (EXTRA & kBand) == 0) {
+    if constexpr (BWD) {
         // Backward likewise, where it gains: rows of five and six chunks in two waves, rows of nine and more in four.  us per launch,
         // fp16, 2^27 elements, two chunks per wave -> three, causal / full rows / both with dropout:
         //   [30,2112,2112] 88.9 -> 88.1 / 87.8 -> 81.6 / 102.7 -> 90.4 / 119.6 -> 104.4, [20,2560,2560] 87.9 -> 86.5 / 82.2 -> 82.6 /
@@ -442,15 +427,12 @@ static hipError_t dispatch_rows(const SoftmaxArgs& a, bool vec_ok, hipStream_t s
         //     126.2 -> 110.5, [3,6144,6144] 75.6 -> 74.8 / 88.8 -> 91.1 / 78.6 -> 75.5 / 110.3 -> 107.6
         //   with few rows: causal [1,2112,2112] 5.9 -> 6.1, with dropout [2,2112,2112] 10.0 -> 10.9, [4,2112,2112] level, full rows [1,2112,2112] 8.0
         //     -> 7.5, ragged [1,2901,2901] 11.7 -> 11.9, [4,2901,2901] 35.2 -> 35.7
-        // Full rows without dropout: only if the call knows where the rows of several samples end (the figures above); without a hidden tail
-        // [1,30,2112,2112] 124.7 -> 127.5, [1,8,4608,4608] 158.3 -> 163.7, [1,8,5120,5120] 194.1 -> 203.9 (with dropout [1,8,5120,5120]
-        // 212.9 -> 199.9, [1,8,6144,6144] 291.1 -> 290.1).
-        constexpr bool ends = M == Mask::None && (EXTRA & kDropout) == 0;
-        bool enough = !ends || (a.row_end != nullptr && !a.mask_bcast && a.rows > a.by_mask_batch.d);  // (several samples)
-        const bool four = enough && chunks > 8 && chunks <= (M == Mask::Causal ? 12 : ends ? 9 : 10);
-        if (M == Mask::Causal) enough = a.rows >= 4608;
-        if (ends && chunks == 6) enough = false;  // [8,5,3000,3000] 259.5 -> 267, [8,2,2816,2816] 98.2 -> 98.7
-        if (EXTRA == kRagged && M == Mask::None) enough = enough && a.rows >= 8192 && a.sk <= 2304;
+        // Aligned full rows without dropout: not at all.  They gain where the padding hides much of a sample (the figures above) and lose where
+        // nothing is hidden, [1,30,2112,2112] 124.7 -> 127.5, [1,8,4608,4608] 158.3 -> 163.7, [1,8,5120,5120] 194.1 -> 203.9, and a call
+        // that knows where its rows end must sum in the order of one that does not.
+        constexpr bool full = M == Mask::None && EXTRA == 0;
+        const bool enough = !full && (M == Mask::Causal ? a.rows >= 4608 : EXTRA != kRagged || (a.rows >= 8192 && a.sk <= 2304));
+        const bool four = chunks > 8 && (M == Mask::Causal ? chunks <= 12 : EXTRA == kRagged ? chunks == 9 : !full && chunks <= 10);
         if (chunks <= 6 && enough) return launch_shape<T, M, BWD, EXTRA | (EXTRA == kRagged ? kStaged : 0), 3, 2, 2>(a, st);
         if (four) return launch_shape<T, M, BWD, EXTRA, 3, 4, 1>(a, st);
     }
@@ -459,13 +441,7 @@ static hipError_t dispatch_rows(const SoftmaxArgs& a, bool vec_ok, hipStream_t s
         // which up to half would hold nothing (-13 % at 8200 columns, -8 % at 10240, -4 % at 12288).
         if (chunks > 16 && chunks <= 24) return launch_shape<T, M, BWD, EXTRA, 3, 8, 1>(a, st);
     }
-    if constexpr ((EXTRA & kBand) != 0) {
-        // rows of two 4 KiB pieces: two per block, in the order of with_xcd_mapping ([32,4096,4096] window 2048:
-        // 248 -> 232 us forward, 315 -> 306 backward; window 1600 239 -> 222 and 298 -> 281).  Without that order the shape
-        // loses: on an output off the 4 KiB boundary 263 -> 284 and 341 -> 354, 3600 columns 219 -> 226 and 284 -> 297.
-        if (chunks <= 6 && two_piece_rows(a)) return launch_shape<T, M, BWD, EXTRA, 3, 2, 2>(a, st);
-    }
-    if constexpr (M == Mask::Causal && (EXTRA & kBand) == 0 && !(BWD && (EXTRA & kDropout) != 0)) {
+    if constexpr (M == Mask::Causal && !(BWD && (EXTRA & kDropout) != 0)) {
         if (chunks >= 7 && chunks <= 8 && two_causal_rows<BWD, EXTRA>(a, chunks)) return launch_shape<T, M, BWD, EXTRA, 2, 4, 2>(a, st);
     }
     if (chunks <= 8) return launch_shape<T, M, BWD, EXTRA, 2, 4, 1>(a, st);
@@ -475,11 +451,79 @@ static hipError_t dispatch_rows(const SoftmaxArgs& a, bool vec_ok, hipStream_t s
     return launch_shape<T, M, BWD, EXTRA, 4, 16, 1>(a, st);
 }
 
-// Sliding-window causal softmax (EXTRA = kBand): causal rows only.
+// Sliding-window causal softmax: aligned causal rows of two chunks or more.  The shape goes by the chunks the band can
+// touch -- w + 1 keys lie in at most w / 512 + 2 of them, `chunks` -- and by those of the row: the waves hold the band, the rest of the
+// row is zeros, which they store as well (band_zero_fill).  TB/s by algorithmic bytes, bf16, 2^27 elements, [columns, window], the shape
+// of the rule against the one that the band alone would call for (chunks / 2 waves with two chunks, from 4097 columns on
+// chunks waves with one).  With few rows fewer waves per row or more of them lose 2-10 % ([1,2048,2048] window 256 backward 3.6 -> 3.9 us,
+// [4,1536,1536] 384 forward 5.5 -> 5.9): `many`.
+//   forward   rows of three chunks: one wave, [1152,576] 4.54 -> 5.82, [1536,768] 5.55 -> 5.89, [1536,256] 5.37 -> 5.46, [1152,288] 5.46 -> 5.50
+//     of four: two waves with two rows per block, [2048,1024] 5.99 -> 6.14, [2048,600] 5.74 -> 5.97
+//     of five to eight: one wave at two chunks, [2560,256] 5.08 -> 5.29, [3072,400] 5.19 -> 5.30; two waves with three chunks each at
+//       three to six, [3072,1000] 5.67 -> 5.78, [3072,1400] 5.70 -> 5.97, [3072,1600] 5.43 -> 6.03, [2560,1600] 5.16 -> 5.96, but [2560,700]
+//       5.63 -> 5.61; with four from 3073 columns on at five and six, [3584,1792] 5.56 -> 5.82
+//   backward  one chunk per wave: [2048,384] 5.88 -> 6.17, [2560,400] 5.41 -> 5.52, [1472,368] 5.45 -> 5.59, [1536,128] level; [3072,768]
+//     5.63 -> 5.72, [3584,896] 5.52 -> 5.76, [3072,1100] 5.70 -> 5.89, [2560,1280] 5.84 -> 5.92, but [2560,700] 5.69 -> 5.5; [8192,1600] 5.62 -> 5.81,
+//     [8192,3000] 5.73 -> 5.93, [7168,1792] 5.55 -> 5.72, [6144,3072] 5.83 -> 5.94, but [5120,2560] 5.87 -> 5.79
+//   4096 columns, rows of two 4 KiB pieces, two per block in the order of with_xcd_mapping: [4096,256] 5.4 -> 5.78 and backward 5.32 -> 5.80,
+//     [4096,1024] 5.86 -> 5.96 (forward), [4096,2048] 5.65 -> 6.15 and 5.99 -> 6.13, [4096,2560] 5.81 -> 6.21 and 6.13 -> 6.22; three waves' worth
+//     at three chunks [4096,1000] 5.86 -> 5.97, [4096,512] -1 %.  Off the 4 KiB boundary that order does not apply: as other lengths.
+//   beyond 4096 columns one chunk per wave up to four chunks, [8192,256] 5.36 -> 5.68 and 5.36 -> 5.49, [5000,1250] 252 -> 236 us and 294 -> 274,
+//     (forward at two chunks: from 16 chunks of the row on, [4608,400] 46.2 -> 52.4), up to 28 chunks of the row: [15360,1024] 200 -> 204 us, [16384,1500] 210 -> 232, [32768,1024] 408 -> 446
+template <typename T, bool BWD>
+static hipError_t dispatch_band_rows(const SoftmaxArgs& a, hipStream_t st) {
+    constexpr Mask M = Mask::Causal;
+    constexpr int B = kBand;
+    const int row = (a.sk + kChunk - 1) / kChunk, chunks = std::min(a.window / kChunk + 2, row);
+    const bool many = a.rows >= 8192;
+    if (row <= 2) return launch_shape<T, M, BWD, B, 2, 1, 4>(a, st);
+    if (two_piece_rows(a) && (chunks > 2 || many)) {
+        if (chunks == 2) return launch_shape<T, M, BWD, B, 1, 2, 2>(a, st);
+        if (chunks == 3 && a.window < 640) return launch_shape<T, M, BWD, B, 2, 2, 2>(a, st);
+        if (chunks <= 4 && (BWD || (chunks == 4 && !many))) return launch_shape<T, M, BWD, B, 2, 2, 4>(a, st);
+        if constexpr (!BWD) {
+            if (chunks == 3) return launch_shape<T, M, BWD, B, 3, 2, 2>(a, st);
+        }
+        return launch_shape<T, M, BWD, B, 4, 2, 2>(a, st);
+    }
+    if (row <= 8) {
+        if constexpr (!BWD) {
+            if (row == 3 && (chunks == 3 || (a.window >= 256 && a.rows >= 32768))) return launch_shape<T, M, BWD, B, 3, 1, 4>(a, st);
+            if (chunks == 2 && (row <= 4 || !many)) return launch_shape<T, M, BWD, B, 2, 1, 4>(a, st);
+            if (chunks == 2) return launch_shape<T, M, BWD, B, 4, 1, 4>(a, st);
+            if (row == 4 || (chunks == 3 && (row == 5 || !many))) return launch_shape<T, M, BWD, B, 2, 2, 2>(a, st);
+            if (chunks == 4 && !many) return launch_shape<T, M, BWD, B, 2, 2, 4>(a, st);
+            if (chunks <= 4 || (chunks <= 6 && row <= 6)) return launch_shape<T, M, BWD, B, 3, 2, 2>(a, st);
+            if (chunks <= 6 && row == 7) return launch_shape<T, M, BWD, B, 4, 2, 2>(a, st);
+        } else {
+            if (chunks == 2 && a.sk > 1408 && a.window >= 192 && many) return launch_shape<T, M, BWD, B, 1, 2, 2>(a, st);
+            if (chunks == 2) return launch_shape<T, M, BWD, B, 2, 1, 4>(a, st);
+            if (many && ((chunks == 3 && row >= 6) || (chunks == 4 && row >= 5))) return launch_shape<T, M, BWD, B, 1, 4, 1>(a, st);
+            if (chunks == 3) return launch_shape<T, M, BWD, B, 2, 2, 2>(a, st);
+            if (chunks == 4) return launch_shape<T, M, BWD, B, 2, 2, 4>(a, st);
+        }
+        return launch_shape<T, M, BWD, B, 2, 4, 1>(a, st);
+    }
+    if (chunks <= 4) {
+        if (row <= 28 && (chunks > 2 || (BWD ? many : row >= 16))) return launch_shape<T, M, BWD, B, 1, 4, 1>(a, st);
+        if (chunks == 2) return launch_shape<T, M, BWD, B, 2, 1, 4>(a, st);
+        return chunks == 3 ? launch_shape<T, M, BWD, B, 2, 2, 2>(a, st) : launch_shape<T, M, BWD, B, 2, 2, 4>(a, st);
+    }
+    if constexpr (BWD) {
+        if (chunks <= 8 && row >= 12 && row <= 16) return launch_shape<T, M, BWD, B, 1, 8, 1>(a, st);
+        if (chunks > 16 && chunks <= 24) return launch_shape<T, M, BWD, B, 3, 8, 1>(a, st);
+    }
+    if (chunks <= 8) return launch_shape<T, M, BWD, B, 2, 4, 1>(a, st);
+    if (chunks <= 16) return launch_shape<T, M, BWD, B, 2, 8, 1>(a, st);
+    if (chunks <= 32) return launch_shape<T, M, BWD, B, 2, 16, 1>(a, st);
+    if (chunks <= 48) return launch_shape<T, M, BWD, B, 3, 16, 1>(a, st);
+    return launch_shape<T, M, BWD, B, 4, 16, 1>(a, st);
+}
+
 template <bool BWD>
 static hipError_t dispatch_band(const SoftmaxArgs& a, int dtype, bool vec_ok, hipStream_t st) {
-    return dtype == NEOX_F16 ? dispatch_rows<F16, Mask::Causal, BWD, kBand>(a, vec_ok, st)
-                             : dispatch_rows<BF16, Mask::Causal, BWD, kBand>(a, vec_ok, st);
+    if (!vec_ok || a.sk <= kChunk || a.sk > kMaxRegisterRow) return hipErrorInvalidValue;  // the caller checks
+    return dtype == NEOX_F16 ? dispatch_band_rows<F16, BWD>(a, st) : dispatch_band_rows<BF16, BWD>(a, st);
 }
 
 template <bool BWD, int EXTRA = 0>
