@@ -430,11 +430,12 @@ static hipError_t dispatch_rows(const SoftmaxArgs& a, bool vec_ok, hipStream_t s
         // Aligned full rows without dropout: not at all.  They gain where the padding hides much of a sample (the figures above) and lose where
         // nothing is hidden, [1,30,2112,2112] 124.7 -> 127.5, [1,8,4608,4608] 158.3 -> 163.7, [1,8,5120,5120] 194.1 -> 203.9, and a call
         // that knows where its rows end must sum in the order of one that does not.
-        constexpr bool full = M == Mask::None && EXTRA == 0;
-        const bool enough = !full && (M == Mask::Causal ? a.rows >= 4608 : EXTRA != kRagged || (a.rows >= 8192 && a.sk <= 2304));
-        const bool four = chunks > 8 && (M == Mask::Causal ? chunks <= 12 : EXTRA == kRagged ? chunks == 9 : !full && chunks <= 10);
-        if (chunks <= 6 && enough) return launch_shape<T, M, BWD, EXTRA | (EXTRA == kRagged ? kStaged : 0), 3, 2, 2>(a, st);
-        if (four) return launch_shape<T, M, BWD, EXTRA, 3, 4, 1>(a, st);
+        if constexpr (M == Mask::Causal || EXTRA != 0) {
+            const bool enough = M == Mask::Causal ? a.rows >= 4608 : EXTRA != kRagged || (a.rows >= 8192 && a.sk <= 2304);
+            if (chunks <= 6 && enough) return launch_shape<T, M, BWD, EXTRA | (EXTRA == kRagged ? kStaged : 0), 3, 2, 2>(a, st);
+            constexpr int most = M == Mask::Causal ? 12 : EXTRA == kRagged ? 9 : 10;
+            if (chunks > 8 && chunks <= most) return launch_shape<T, M, BWD, EXTRA, 3, 4, 1>(a, st);
+        }
     }
     if constexpr (BWD && M == Mask::Causal) {
         // Causal backward just above 8192 columns: 8 waves with 3 chunks each instead of 16 with 2, of

@@ -39,10 +39,9 @@ def check(x, y, g, dx, hidden, dtype, what):
                                          (3072, 1400, 3), (3584, 1200, 3), (3584, 1792, 1), (4096, 200, 2), (4096, 200, 1), (4096, 600, 1),
                                          (4096, 700, 2), (4096, 1100, 1), (4096, 2600, 1), (4608, 400, 2), (6144, 3000, 1), (8192, 256, 1),
                                          (8192, 1600, 1)])
-def test_sliding_window_shapes_by_rows(device, s, w, batches):
-    lib, stream = _lib.lib(), torch.cuda.current_stream().cuda_stream
-    dtype = DTYPES[(s // 8 + w) % 2]
-    code = _lib.dtype_code(dtype)
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_sliding_window_shapes_by_rows(device, s, w, batches, dtype):
+    lib, stream, code = _lib.lib(), torch.cuda.current_stream().cuda_stream, _lib.dtype_code(dtype)
     x, g = normal((batches, s, s), dtype, device, s, 8.0), normal((batches, s, s), dtype, device, w)
     y, dx = torch.empty_like(x), torch.empty_like(x)
     _lib.check(lib.neox_sliding_window_softmax_fwd(y.data_ptr(), x.data_ptr(), SCALE, batches, s, s, w, code, stream))
@@ -55,10 +54,9 @@ def test_sliding_window_shapes_by_rows(device, s, w, batches):
 @pytest.mark.parametrize("s,batches", [(576, 1), (888, 6), (1024, 5), (1088, 5), (1088, 4), (2112, 3), (2112, 2), (4160, 1), (520, 64), (520, 63),
                                        (1000, 33), (1032, 32), (1416, 24), (1480, 23), (1488, 23), (2056, 16), (3064, 11), (1001, 9), (1001, 8), (1301, 5), (1301, 4),
                                        (1601, 2), (1601, 1), (1801, 4), (1801, 3), (2051, 3), (2051, 2), (4101, 1)])
-def test_causal_shapes_by_rows(device, s, batches):
-    lib, stream = _lib.lib(), torch.cuda.current_stream().cuda_stream
-    dtype = DTYPES[(s + batches) % 2]
-    code = _lib.dtype_code(dtype)
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_causal_shapes_by_rows(device, s, batches, dtype):
+    lib, stream, code = _lib.lib(), torch.cuda.current_stream().cuda_stream, _lib.dtype_code(dtype)
     x, g = normal((batches, s, s), dtype, device, s, 8.0), normal((batches, s, s), dtype, device, s + 1)
     y, dx, z, drop = (torch.empty_like(x) for _ in range(4))
     _lib.check(lib.neox_causal_softmax_fwd(y.data_ptr(), x.data_ptr(), SCALE, batches, s, s, code, stream))
@@ -97,3 +95,48 @@ def test_row_ends_of_many_rows(device, s, heads):
     assert torch.equal(masked_ext.backward(g.clone(), y, SCALE), hinted)
     for i in range(b):
         check(x[i], y[i], g[i], hinted[i], mask[i, 0], dtype, (s, heads, i))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("s,heads", [(1301, 5), (1301, 2), (1601, 4), (1601, 2)])
+def test_features_of_one_wave_rows(device, s, heads, dtype):
+    # every combination of what folds into the causal forward pass, 6400 rows or fewer: zero slopes and a zero bias give the
+    # plain bits, and the dropped output follows from them
+    lib, stream, code = _lib.lib(), torch.cuda.current_stream().cuda_stream, _lib.dtype_code(dtype)
+    x = normal((1, heads, s, s), dtype, device, s, 8.0)
+    y, z, drop = (torch.empty_like(x) for _ in range(3))
+    _lib.check(lib.neox_causal_softmax_fwd(y.data_ptr(), x.data_ptr(), SCALE, heads, s, s, code, stream))
+    slopes, bias = torch.zeros(heads, device=device), torch.zeros_like(x)
+    keep = torch.empty(x.numel(), dtype=torch.uint8, device=device)
+    _lib.check(lib.neox_dropout_keep_mask(keep.data_ptr(), 0.25, 9, 0, None, x.numel(), stream))
+    want = torch.where(keep.view(x.shape).bool(), (y.float() * (1.0 / 0.75)).to(dtype), 0)
+    for sl in (None, slopes.data_ptr()):
+        for bi in (None, bias.data_ptr()):
+            z.fill_(7.0)
+            if bi is not None:
+                _lib.check(lib.neox_causal_softmax_bias_fwd(z.data_ptr(), x.data_ptr(), bi, sl, SCALE, 1, heads, s, s, 1, code, stream))
+                assert torch.equal(z, y)
+            z.fill_(7.0)
+            _lib.check(lib.neox_causal_softmax_dropout_fwd(drop.data_ptr(), z.data_ptr(), x.data_ptr(), sl, bi, 1 if bi else 0, SCALE, 0.25, 9, 0,
+                                                           None, 1, heads, s, s, code, stream))
+            assert torch.equal(z, y) and torch.equal(drop, want)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("s,batches", [(1301, 7), (1301, 1), (1601, 6), (1601, 1), (2051, 4), (2112, 1), (4160, 1)])
+def test_full_row_backward_by_rows(device, s, batches, dtype):
+    # plain and with dropout, 8192 rows or fewer
+    lib, stream, code = _lib.lib(), torch.cuda.current_stream().cuda_stream, _lib.dtype_code(dtype)
+    y = torch.softmax(normal((batches, s, s), torch.float32, device, s, 2.0), -1).to(dtype)
+    g, dx = normal((batches, s, s), dtype, device, s + 1), torch.empty(batches, s, s, dtype=dtype, device=device)
+    keep = torch.empty(g.numel(), dtype=torch.uint8, device=device)
+    _lib.check(lib.neox_dropout_keep_mask(keep.data_ptr(), 0.25, 3, 0, None, g.numel(), stream))
+    kept = torch.where(keep.view(g.shape).bool(), g.float() * (1.0 / 0.75), 0)
+    for p, gf in ((0.0, g.float()), (0.25, kept)):
+        if p:
+            _lib.check(lib.neox_masked_softmax_dropout_bwd(dx.data_ptr(), g.data_ptr(), y.data_ptr(), SCALE, p, 3, 0, None, batches * s, s, code, stream))
+        else:
+            _lib.check(lib.neox_masked_softmax_bwd(dx.data_ptr(), g.data_ptr(), y.data_ptr(), SCALE, batches * s, s, code, stream))
+        for i in {0, batches - 1}:
+            yf = y[i].float()
+            assert_grad(dx[i], SCALE * yf * (gf[i] - (gf[i] * yf).sum(-1, keepdim=True)), dtype, (s, p, i), y=y[i], g=gf[i], scale=SCALE)
