@@ -226,7 +226,8 @@ struct SoftmaxCall {
             return a.row_end != nullptr && a.sk <= 2048;
         }
         if (m == Mask::Causal) return a.sk <= 1480 && a.sk >= (plain ? 640 : 1025);
-        return plain && a.row_end != nullptr && a.sk >= 832 && a.sk <= 2048;
+        // (above two chunks the call without the ends sums in one wave per row, like the ragged kernels, only if 32 bits address the mask)
+        return plain && a.row_end != nullptr && a.sk >= 832 && a.sk <= 2048 && (a.sk <= 2 * kChunk || a.mask_bytes != 0);
     }
 
     void rows(int64_t n, int sq, int sk) {

@@ -339,3 +339,21 @@ def test_hint_on_another_stream_than_the_scans(device, monkeypatch):
             assert torch.equal(m(x, mask), want)
     side.synchronize()
     assert seen["hinted"] == 4
+
+
+@pytest.mark.parametrize("sk", [1000, 1032, 1608])
+def test_hint_beside_a_mask_beyond_4_gib(device, sk):
+    # aligned rows that are no whole cache lines, so many that the mask needs 64-bit addresses: the kernels that a call
+    # without the hint takes then sum a row over two waves above 1024 columns, and the hint must not change that
+    sq = 2**32 // sk + 8
+    x = torch.empty((1, 1, sq, sk), dtype=torch.float16, device=device).normal_(0.0, 4.0, generator=gen(device, sk))
+    mask = torch.zeros((1, 1, sq, sk), dtype=torch.bool, device=device)
+    end = sk // 2 + 5
+    mask[..., end:] = True
+    ends = torch.full((sq,), end, dtype=torch.int32, device=device)
+    y = masked_ext.forward(x, mask, 0.25)
+    hinted = masked_ext.forward(x, mask, 0.25, row_end=ends)
+    for a, b in zip(hinted[0, 0].split(2**19), y[0, 0].split(2**19)):  # (a whole comparison needs a tensor of its own)
+        assert torch.equal(a, b)
+    for rows in (slice(0, 64), slice(sq - 64, sq)):
+        assert max_err(y[0, 0, rows], R.softmax_fp32(x[0, 0, rows], mask[0, 0, rows], 0.25)) <= TOL[torch.float16]
