@@ -236,9 +236,10 @@ __device__ __forceinline__ uint32_t keep_bits_row8(const DropoutArgs& d, uint32_
 // each go the same way in groups of 4 blocks (group_shift 2): an XCD then keeps to two pieces in eight.
 // Returns the unit index for unit l of block b; the identity for the last, incomplete group.
 //
-// FLAT, the row kernels: no branch, behind which the kernel's other arguments would be fetched a round trip later.  The packed kernels,
-// which ask for them behind a test of the row anyway, are faster with it where a call has few rows (mask tensor and ALiBi, fp16
-// [544,544] 4.0 us against 4.2, [8,469,469] 4.8 against 4.9).
+// FLAT, ragged rows with dropout: no branch, behind which the kernel's other arguments would be fetched a round trip later.  Those
+// kernels are 0.3-1 % faster without it, the others with it where a call has few rows, us with -> without: sliding window backward
+// [10,744,744] 5.7 -> 6.2, [15,536,536] 5.3 -> 5.7, causal forward with ALiBi [2,2004,2004] 5.9 -> 6.5, [3416,3416] 8.6 -> 8.9, dropout backward
+// [3,1344,1344] 6.3 -> 6.8, row ends [6,944,944] 5.4 -> 5.65; packed kernels, mask tensor and ALiBi [544,544] 4.0 -> 4.2, [8,469,469] 4.8 -> 4.9.
 template <bool FLAT>
 __device__ __forceinline__ uint32_t xcd_slot(uint32_t b, uint32_t l, uint32_t U, const SoftmaxArgs& a) {
     if constexpr (!FLAT) {
@@ -474,7 +475,8 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void softmax_fwd_kernel(SoftmaxArg
     const float ninf = -__builtin_inff();
     // byte offset of the lane inside the row, first chunk of its wave.  Everything goes into
     // the per-lane offset: the hardware's range check does not see the scalar offset operand.
-    const RowPos pos = locate<MASK>(xcd_slot<true>(blockIdx.x, rib, RPB, a), a);
+    constexpr bool kFlat = kRag && (FLAGS & kDropout) != 0;
+    const RowPos pos = locate<MASK>(xcd_slot<kFlat>(blockIdx.x, rib, RPB, a), a);
     const RaggedRow<kRag> rag(a.in0, pos.row, sk, lane, wir == 0);
     // kBand: first visible key of the row, and the start of the 128-bit access that holds it.  The
     // waves' chunks are counted from the chunk that holds that key (wch instead of wir), so that a
@@ -687,7 +689,8 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void softmax_bwd_kernel(SoftmaxArg
     const int rib = wib / WPR;
     const int wir = wib % WPR;
     const int sk = a.sk;
-    const RowPos pos = locate<MASK>(xcd_slot<true>(blockIdx.x, rib, RPB, a), a);
+    constexpr bool kFlat = kRag && (FLAGS & kDropout) != 0;
+    const RowPos pos = locate<MASK>(xcd_slot<kFlat>(blockIdx.x, rib, RPB, a), a);
     // kBand: first visible key of the row, the start of the 128-bit access that holds it, and the
     // wave's first chunk of the row counted from the chunk that holds that key (see the forward kernel)
     int lo = 0;
