@@ -289,6 +289,17 @@ __device__ __forceinline__ void loads_first() {
     __builtin_amdgcn_sched_barrier(0);
 }
 
+// Ragged backward pass of eight and sixteen waves per row: what the compiler has unpacked before this point it unpacks again behind it,
+// instead of holding the row in fp32 over the reduction.  That took 72 registers a lane (bf16, two chunks) and 72 to 120 (three and
+// four chunks), with which a CU runs one block of 16 waves and not two.  us per launch, held in fp32 -> packed: bf16 row ends
+// [8490,8490] 104 -> 77, full rows [4194,16001] 79 -> 67, causal [8573,8573] 58.8 -> 51.9, [16383,16383] 215 -> 181, fp16 and bf16
+// [20001,20001] 321 -> 283.  Fewer waves, or two chunks in fp16 (56 registers either way): 0...+3 %.
+template <int N>
+__device__ __forceinline__ void keep_packed(u32x4 (&v)[N]) {
+#pragma unroll
+    for (int c = 0; c < N; ++c) asm volatile("" : "+v"(v[c]));
+}
+
 // Combine a per-wave partial across the WPR waves of a row.
 template <typename Op, int WPR, int RPB>
 __device__ __forceinline__ float row_combine(float v, float* red, int wib, int rib, int lane) {
@@ -774,6 +785,10 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void softmax_bwd_kernel(SoftmaxArg
         }
         dot = wave_reduce<OpSum>(dot);
         dot = row_combine<OpSum, WPR, RPB>(dot, red_sum, wib, rib, lane);
+        if constexpr (kRag && WPR >= 8 && (FLAGS & kDropout) == 0 && (NCH > 2 || std::is_same<T, BF16>::value)) {
+            keep_packed(rg);
+            keep_packed(rp);
+        }
 
         const Rows<kStage, RPB> out(a, a.out, pos, rib);
 #pragma unroll
