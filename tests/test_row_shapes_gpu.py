@@ -16,6 +16,11 @@ SCALE = 0.125
 DTYPES = [torch.float16, torch.bfloat16]
 
 
+def unwritten(like):
+    """An output that holds what no kernel writes: every store has to be this call's own."""
+    return torch.full_like(like, 7.0)
+
+
 def normal(shape, dtype, device, seed, std=1.0):
     return torch.empty(shape, dtype=dtype, device=device).normal_(0.0, std, generator=torch.Generator(device=device).manual_seed(seed))
 
@@ -43,7 +48,7 @@ def check(x, y, g, dx, hidden, dtype, what):
 def test_sliding_window_shapes_by_rows(device, s, w, batches, dtype):
     lib, stream, code = _lib.lib(), torch.cuda.current_stream().cuda_stream, _lib.dtype_code(dtype)
     x, g = normal((batches, s, s), dtype, device, s, 8.0), normal((batches, s, s), dtype, device, w)
-    y, dx = torch.empty_like(x), torch.empty_like(x)
+    y, dx = unwritten(x), unwritten(x)
     _lib.check(lib.neox_sliding_window_softmax_fwd(y.data_ptr(), x.data_ptr(), SCALE, batches, s, s, w, code, stream))
     _lib.check(lib.neox_sliding_window_softmax_bwd(dx.data_ptr(), g.data_ptr(), y.data_ptr(), SCALE, batches, s, s, w, code, stream))
     check(x, y, g, dx, R.get_attn_mask(s, device, sliding_window_width=w)[0, 0], dtype, (s, w))
@@ -58,7 +63,7 @@ def test_sliding_window_shapes_by_rows(device, s, w, batches, dtype):
 def test_causal_shapes_by_rows(device, s, batches, dtype):
     lib, stream, code = _lib.lib(), torch.cuda.current_stream().cuda_stream, _lib.dtype_code(dtype)
     x, g = normal((batches, s, s), dtype, device, s, 8.0), normal((batches, s, s), dtype, device, s + 1)
-    y, dx, z, drop = (torch.empty_like(x) for _ in range(4))
+    y, dx, z, drop = (unwritten(x) for _ in range(4))
     _lib.check(lib.neox_causal_softmax_fwd(y.data_ptr(), x.data_ptr(), SCALE, batches, s, s, code, stream))
     _lib.check(lib.neox_causal_softmax_bwd(dx.data_ptr(), g.data_ptr(), y.data_ptr(), SCALE, batches, s, s, code, stream))
     hidden = torch.ones(s, s, dtype=torch.bool, device=device).triu_(1)
@@ -71,12 +76,14 @@ def test_causal_shapes_by_rows(device, s, batches, dtype):
     _lib.check(lib.neox_dropout_keep_mask(keep.data_ptr(), 0.25, 7, 0, None, x.numel(), stream))
     keep = keep.view(x.shape).bool()
     assert torch.equal(drop, torch.where(keep, (y.float() * (1.0 / 0.75)).to(dtype), 0))
+    dx.fill_(7.0)
     _lib.check(lib.neox_causal_softmax_dropout_bwd(dx.data_ptr(), g.data_ptr(), y.data_ptr(), SCALE, 0.25, 7, 0, None, batches, s, s, code, stream))
     for i in {0, batches - 1}:
         yf, gf = y[i].float(), torch.where(keep[i], g[i].float() * (1.0 / 0.75), 0)
         assert_grad(dx[i], SCALE * yf * (gf - (gf * yf).sum(-1, keepdim=True)), dtype, (s, i), y=y[i], g=gf, scale=SCALE)
     # slopes of zero: the same sums
     slopes = torch.zeros(batches, device=device)
+    z.fill_(7.0)
     _lib.check(lib.neox_causal_softmax_alibi_fwd(z.data_ptr(), x.data_ptr(), slopes.data_ptr(), SCALE, 1, batches, s, s, code, stream))
     assert torch.equal(z, y)
 
@@ -104,7 +111,7 @@ def test_features_of_one_wave_rows(device, s, heads, dtype):
     # plain bits, and the dropped output follows from them
     lib, stream, code = _lib.lib(), torch.cuda.current_stream().cuda_stream, _lib.dtype_code(dtype)
     x = normal((1, heads, s, s), dtype, device, s, 8.0)
-    y, z, drop = (torch.empty_like(x) for _ in range(3))
+    y, z, drop = (unwritten(x) for _ in range(3))
     _lib.check(lib.neox_causal_softmax_fwd(y.data_ptr(), x.data_ptr(), SCALE, heads, s, s, code, stream))
     slopes, bias = torch.zeros(heads, device=device), torch.zeros_like(x)
     keep = torch.empty(x.numel(), dtype=torch.uint8, device=device)
@@ -117,6 +124,7 @@ def test_features_of_one_wave_rows(device, s, heads, dtype):
                 _lib.check(lib.neox_causal_softmax_bias_fwd(z.data_ptr(), x.data_ptr(), bi, sl, SCALE, 1, heads, s, s, 1, code, stream))
                 assert torch.equal(z, y)
             z.fill_(7.0)
+            drop.fill_(7.0)
             _lib.check(lib.neox_causal_softmax_dropout_fwd(drop.data_ptr(), z.data_ptr(), x.data_ptr(), sl, bi, 1 if bi else 0, SCALE, 0.25, 9, 0,
                                                            None, 1, heads, s, s, code, stream))
             assert torch.equal(z, y) and torch.equal(drop, want)
@@ -128,11 +136,12 @@ def test_full_row_backward_by_rows(device, s, batches, dtype):
     # plain and with dropout, 8192 rows or fewer
     lib, stream, code = _lib.lib(), torch.cuda.current_stream().cuda_stream, _lib.dtype_code(dtype)
     y = torch.softmax(normal((batches, s, s), torch.float32, device, s, 2.0), -1).to(dtype)
-    g, dx = normal((batches, s, s), dtype, device, s + 1), torch.empty(batches, s, s, dtype=dtype, device=device)
+    g, dx = normal((batches, s, s), dtype, device, s + 1), unwritten(y)
     keep = torch.empty(g.numel(), dtype=torch.uint8, device=device)
     _lib.check(lib.neox_dropout_keep_mask(keep.data_ptr(), 0.25, 3, 0, None, g.numel(), stream))
     kept = torch.where(keep.view(g.shape).bool(), g.float() * (1.0 / 0.75), 0)
     for p, gf in ((0.0, g.float()), (0.25, kept)):
+        dx.fill_(7.0)
         if p:
             _lib.check(lib.neox_masked_softmax_dropout_bwd(dx.data_ptr(), g.data_ptr(), y.data_ptr(), SCALE, p, 3, 0, None, batches * s, s, code, stream))
         else:
