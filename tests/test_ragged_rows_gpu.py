@@ -18,7 +18,8 @@ pytestmark = pytest.mark.gpu
 
 GUARD = 64  # elements in front of and behind every output
 SCALE = 0.125
-# the limits of the shapes (672 and 944: staged; 1536 / 2048: chunks; 1856: two waves) and row ends in every place of a lane
+# the limits of the shapes (1536 / 2048: chunks; 1856: two waves) and row ends in every place of a lane; the shapes that want
+# many rows: test_staged_rows_of_many_rows and what follows it
 COLUMNS = [513, 520, 527, 671, 673, 943, 945, 1001, 1018, 1023, 1024, 1025, 1031, 1201, 1535, 1536, 1537, 1855, 1857, 2047, 2049, 4097]
 
 
@@ -131,6 +132,114 @@ def test_ragged_rows(device, sk, offsets):
                                                             shape4[0], code, stream))
             assert guarded(z, zs) and guarded(drop, ds), (kind, fold, sk)
             assert torch.equal(z, y), (kind, fold, sk, offsets)
+
+
+class Written:
+    """Calls that write guarded outputs: every element of each is written, nothing around it is."""
+
+    def __init__(self, dtype, device, what):
+        self.dtype, self.device, self.what = dtype, device, what
+
+    def __call__(self, call, shape, offset, fill=None, outputs=1):
+        outs = [at(offset, shape, self.dtype, self.device, fill=fill) for _ in range(outputs)]
+        _lib.check(call(*(t for t, _ in outs)))
+        for t, store in outs:
+            assert guarded(t, store), self.what
+            assert not (t == 7.0).any(), self.what  # no probability, and no gradient of these sizes, is 7
+        return outs[0][0] if outputs == 1 else [t for t, _ in outs]
+
+
+def check_backward(written, run, y, g, offsets, dtype):
+    """dx into a tensor of its own and over the gradient: the same bits, within the bar of the closed form."""
+    i, o = offsets
+    dx = written(lambda dx: run(dx, g), g.shape, o)
+    assert torch.equal(written(lambda t: run(t, t), g.shape, i, fill=g), dx), written.what
+    yf, gf = y.float(), g.float()
+    assert_grad(dx, SCALE * yf * (gf - (gf * yf).sum(-1, keepdim=True)), dtype, written.what, y=y, g=g, scale=SCALE)
+
+
+# 8193 rows: where the results of rows of two chunks leave through LDS (from 672 columns on in the backward pass, from 944 in the forward
+# pass), and those of two waves per row in the backward pass (2049 to 2304 columns); the last block holds a single row
+@pytest.mark.parametrize("sk", [671, 673, 943, 945, 1001, 1023, 1535, 2047, 2051, 2303])
+@pytest.mark.parametrize("offsets", [(0, 0), (1, 0), (3, 5), (8, 1)])
+def test_staged_rows_of_many_rows(device, sk, offsets):
+    lib, stream = _lib.lib(), torch.cuda.current_stream().cuda_stream
+    dtype = (torch.float16, torch.bfloat16)[(sk // 2 + offsets[0]) % 2]
+    code, gen = _lib.dtype_code(dtype), torch.Generator(device=device).manual_seed(sk)
+    b, sq = 3, 2731
+    shape, (i, o) = (b, 1, sq, sk), offsets
+    x, _ = at(i, shape, dtype, device, gen=gen, std=8.0)
+    g, _ = at(i, shape, dtype, device, gen=gen)
+    lens = torch.tensor([sk, sk - 3, sk // 3], device=device)
+    mask = (torch.arange(sk, device=device).view(1, 1, 1, sk) >= lens.view(b, 1, 1, 1)).expand(shape).contiguous()
+    mask[0, 0, 1] = True  # a row without a visible key
+    written = Written(dtype, device, (sk, offsets))
+
+    def forward(y, src):
+        return lib.neox_masked_softmax_fwd(y.data_ptr(), src.data_ptr(), mask.data_ptr(), SCALE, b, 1, sq, sk, b, code, stream)
+
+    y = written(lambda y: forward(y, x), shape, o)
+    assert (y.float() - R.softmax_fp32(x, mask, SCALE)).abs().max().item() <= TOL[dtype]
+    assert torch.equal(written(lambda t: forward(t, t), shape, i, fill=x), y)
+    check_backward(written, lambda dx, dy: lib.neox_masked_softmax_bwd(dx.data_ptr(), dy.data_ptr(), y.data_ptr(), SCALE, b * sq, sk, code, stream),
+                   y, g, offsets, dtype)
+
+
+# causal rows, as many as it takes: 6400 for the two outputs of dropout through LDS, 4608 for two staged waves per row in the backward
+# pass; the last block is not full
+@pytest.mark.parametrize("sk,n", [(1301, 5), (1601, 5), (1855, 5), (2051, 3), (3071, 3)])
+@pytest.mark.parametrize("offsets", [(0, 0), (1, 0), (3, 5), (8, 1)])
+def test_staged_causal_rows_of_many_rows(device, sk, n, offsets):
+    lib, stream = _lib.lib(), torch.cuda.current_stream().cuda_stream
+    dtype = (torch.float16, torch.bfloat16)[(sk // 2 + offsets[0]) % 2]
+    code, gen = _lib.dtype_code(dtype), torch.Generator(device=device).manual_seed(sk)
+    shape, (i, o) = (n, sk, sk), offsets
+    x, _ = at(i, shape, dtype, device, gen=gen, std=8.0)
+    g, _ = at(i, shape, dtype, device, gen=gen)
+    hidden = torch.ones(sk, sk, dtype=torch.bool, device=device).triu_(1)
+    written = Written(dtype, device, (sk, offsets))
+    y = written(lambda y: lib.neox_causal_softmax_fwd(y.data_ptr(), x.data_ptr(), SCALE, n, sk, sk, code, stream), shape, o)
+    assert (y.float() - R.softmax_fp32(x[None], hidden[None, None], SCALE)[0]).abs().max().item() <= TOL[dtype]
+    assert torch.equal(written(lambda t: lib.neox_causal_softmax_fwd(t.data_ptr(), t.data_ptr(), SCALE, n, sk, sk, code, stream), shape, i, fill=x), y)
+
+    def dropped(drop, z):
+        return lib.neox_causal_softmax_dropout_fwd(drop.data_ptr(), z.data_ptr(), x.data_ptr(), None, None, 0, SCALE, 0.25, 5, 0, None,
+                                                   1, n, sk, sk, code, stream)
+
+    drop, z = written(dropped, shape, o, outputs=2)
+    keep = torch.empty(x.numel(), dtype=torch.uint8, device=device)
+    _lib.check(lib.neox_dropout_keep_mask(keep.data_ptr(), 0.25, 5, 0, None, x.numel(), stream))
+    assert torch.equal(z, y)
+    assert torch.equal(drop, torch.where(keep.view(shape).bool(), (y.float() * (1.0 / 0.75)).to(dtype), 0))
+    check_backward(written, lambda dx, dy: lib.neox_causal_softmax_bwd(dx.data_ptr(), dy.data_ptr(), y.data_ptr(), SCALE, n, sk, sk, code, stream),
+                   y, g, offsets, dtype)
+
+
+# aligned rows that are no whole cache lines, 32768 and more of them: the same kernels.  The last block is not full where rows
+# are not a multiple of the length (mask tensor with known row ends)
+@pytest.mark.parametrize("sk", [840, 1000, 1032, 1544, 2040])
+@pytest.mark.parametrize("offsets", [(0, 0), (8, 24)])
+def test_aligned_rows_through_lds(device, sk, offsets):
+    lib, stream = _lib.lib(), torch.cuda.current_stream().cuda_stream
+    dtype = (torch.float16, torch.bfloat16)[(sk // 8 + offsets[0]) % 2]
+    code, gen = _lib.dtype_code(dtype), torch.Generator(device=device).manual_seed(sk)
+    sq = 32769
+    shape, (i, o) = (1, 1, sq, sk), offsets
+    x, _ = at(i, shape, dtype, device, gen=gen, std=8.0)
+    g, _ = at(i, shape, dtype, device, gen=gen)
+    lens = sk - torch.arange(sq, device=device, dtype=torch.int32) % 37
+    mask = (torch.arange(sk, device=device).view(1, sk) >= lens.view(sq, 1)).view(shape)
+    written = Written(dtype, device, (sk, offsets))
+
+    def forward(y, src):
+        return lib.neox_masked_softmax_ends_fwd(None, y.data_ptr(), src.data_ptr(), mask.data_ptr(), lens.data_ptr(), None, None, 0, SCALE, 0.0,
+                                                0, 0, None, 1, 1, sq, sk, 1, code, stream)
+
+    y = written(lambda y: forward(y, x), shape, o)
+    assert (y.float() - R.softmax_fp32(x, mask, SCALE)).abs().max().item() <= TOL[dtype]
+    assert torch.equal(written(lambda t: forward(t, t), shape, i, fill=x), y)
+    check_backward(written, lambda dx, dy: lib.neox_masked_softmax_ends_bwd(dx.data_ptr(), dy.data_ptr(), y.data_ptr(), lens.data_ptr(), SCALE, 0,
+                                                                            0.0, 0, 0, None, 1, 1, sq, sk, 1, code, stream), y, g, offsets, dtype)
 
 
 @pytest.mark.parametrize("sk", [513, 1001, 1201, 1999, 3001])
