@@ -321,7 +321,11 @@ __device__ __forceinline__ float row_combine(float v, float* red, int wib, int r
 // that would reach behind it is moved back to end with the row.  Such a lane shares columns with its neighbour: both
 // compute and store the same bits for them, and only one counts them in the row's sums.  Every lane so makes one 128-bit
 // access per tensor, inside the row.
-template <bool RAG>
+// CLIP, the backward pass with dropout, which stores its rows itself: in rows of an even length, whose last access ends with a
+// whole dword, the buffer's range check ends the row instead and no lane is moved back (the lane's columns behind the row are
+// zero like those behind `len`; the same sums).  The lane that two lanes store cost full rows 2-4 %, us per launch, fp16, moved -> clipped:
+// [64,804,804] 57.8 -> 55.8, [110,724,724] -3.5 %, [32,660,660] -2.5 %, [64,1020,1020] -7 %; odd lengths level.
+template <bool RAG, bool CLIP = false>
 struct RaggedRow {  // aligned rows
     static constexpr int sh = 0;
     int lane;
@@ -336,21 +340,25 @@ struct RaggedRow {  // aligned rows
     __device__ __forceinline__ void own(float (&)[8], int) const {}
     __device__ __forceinline__ uint32_t store_off(int) const { return 0; }
 };
-template <>
-struct RaggedRow<true> {
+template <bool CLIP>
+struct RaggedRow<true, CLIP> {
     int sh, sk, lane;
+    int last;    // the last column that an access may start at
     bool first;  // the wave holds the row's first chunk, moved by sh
     __device__ __forceinline__ RaggedRow(const void* base, uint32_t row, int sk_, int lane_, bool first_wave)
-        : sh(ragged_shift(base, row, sk_)), sk(sk_), lane(lane_), first(sh != 0 && first_wave) {}
+        : sh(ragged_shift(base, row, sk_)), sk(sk_), lane(lane_), last(CLIP && (sk_ & 1) == 0 ? sk_ - 1 : sk_ - kVec),
+          first(sh != 0 && first_wave) {}
     // first column of the lane's access; a lane behind the row: one that no row has
     __device__ __forceinline__ int col(int c0) const {
         const int own = c0 + lane * kVec - sh;
-        return own < sk ? min(max(own, 0), sk - kVec) : 0x3fffffff;
+        return own < sk ? min(max(own, 0), last) : 0x3fffffff;
     }
     // the first column that any lane of the chunk holds (wave-uniform)
-    __device__ __forceinline__ int chunk_col(int c0) const { return c0 - sh < sk ? min(c0 - sh, sk - kVec) : sk; }
+    __device__ __forceinline__ int chunk_col(int c0) const { return c0 - sh < sk ? min(c0 - sh, last) : sk; }
     // the lane moved back is in this chunk (wave-uniform)
-    __device__ __forceinline__ bool moved_back(int c0) const { return c0 + kChunk - sh > sk && ((sk + sh) & (kVec - 1)) != 0; }
+    __device__ __forceinline__ bool moved_back(int c0) const {
+        return c0 + kChunk - sh > sk && ((sk + sh) & (kVec - 1)) != 0 && !(CLIP && (sk & 1) == 0);
+    }
     // columns of the lane that the lane before it counts
     __device__ __forceinline__ int back(int c0) const {
         const int own = c0 + lane * kVec - sh;
@@ -710,7 +718,7 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void softmax_bwd_kernel(SoftmaxArg
     if constexpr (kBnd) lo = max((int)pos.i - a.window, 0);
     const int lo8 = lo & ~(kVec - 1);
     const int wch = wir + lo / kChunk;
-    const RaggedRow<kRag> rag(a.in0, pos.row, sk, lane, wir == 0);
+    const RaggedRow<kRag, (FLAGS & kDropout) != 0 && !kStage> rag(a.in0, pos.row, sk, lane, wir == 0);
     const int voff = lane * 16 + wch * kChunk * 2;  // the range check ignores a scalar offset
     DropoutArgs drop = a.drop;
     if constexpr ((FLAGS & kDropout) != 0) drop = resolve(drop);

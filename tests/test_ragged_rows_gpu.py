@@ -242,6 +242,38 @@ def test_aligned_rows_through_lds(device, sk, offsets):
                                                                             0.0, 0, 0, None, 1, 1, sq, sk, 1, code, stream), y, g, offsets, dtype)
 
 
+# the backward pass with dropout ends a row of an even length by the range check, one of an odd length by a lane that is moved
+# back: one to sixteen waves per row, fifteen full rows or a causal matrix
+@pytest.mark.parametrize("sk", [514, 516, 517, 804, 1020, 1022, 1030, 1031, 1604, 2052, 4100, 4102, 8204, 16386])
+@pytest.mark.parametrize("offsets", [(0, 0), (1, 0), (3, 5), (8, 1)])
+def test_dropout_backward_of_even_rows(device, sk, offsets):
+    lib, stream = _lib.lib(), torch.cuda.current_stream().cuda_stream
+    dtype = (torch.float16, torch.bfloat16)[(sk // 2 + offsets[0]) % 2]
+    code, gen = _lib.dtype_code(dtype), torch.Generator(device=device).manual_seed(sk)
+    i, o = offsets
+    written = Written(dtype, device, (sk, offsets))
+    for causal, shape in ((False, (15, sk)), (True, (sk, sk))):
+        if causal and sk > 4100:
+            continue
+        probs = torch.empty(shape, device=device).normal_(0.0, 2.0, generator=gen)
+        if causal:
+            probs = probs.masked_fill(torch.ones(shape, dtype=torch.bool, device=device).triu_(1), float("-inf"))
+        y, _ = at(i, shape, dtype, device, fill=torch.softmax(probs, -1))
+        g, _ = at(i, shape, dtype, device, gen=gen)
+        keep = torch.empty(g.numel(), dtype=torch.uint8, device=device)
+        _lib.check(lib.neox_dropout_keep_mask(keep.data_ptr(), 0.25, 5, 0, None, g.numel(), stream))
+        gf, yf = torch.where(keep.view(shape).bool(), g.float() * (1.0 / 0.75), 0), y.float()
+
+        def backward(dx, dy):
+            if causal:
+                return lib.neox_causal_softmax_dropout_bwd(dx.data_ptr(), dy.data_ptr(), y.data_ptr(), SCALE, 0.25, 5, 0, None, 1, *shape, code, stream)
+            return lib.neox_masked_softmax_dropout_bwd(dx.data_ptr(), dy.data_ptr(), y.data_ptr(), SCALE, 0.25, 5, 0, None, *shape, code, stream)
+
+        dx = written(lambda dx: backward(dx, g), shape, o)
+        assert_grad(dx, SCALE * yf * (gf - (gf * yf).sum(-1, keepdim=True)), dtype, (sk, offsets, causal), y=y, g=gf, scale=SCALE)
+        assert torch.equal(written(lambda t: backward(t, t), shape, i, fill=g), dx)
+
+
 @pytest.mark.parametrize("sk", [513, 1001, 1201, 1999, 3001])
 def test_one_ragged_row(device, sk):
     # a single row: the lanes at its ends have no neighbouring row to share anything with
