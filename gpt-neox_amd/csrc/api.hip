@@ -207,25 +207,29 @@ struct SoftmaxCall {
   private:
     bool misaligned_ = false;
 
-    // Aligned rows that are no whole number of cache lines, many of them: by the kRagged unit too, whose one-wave kernels store a
-    // block's rows in accesses aligned to lines (see Rows), where the row kernels store parts of lines at both ends of every access.
-    // us per launch, fp16, 2^27 elements, aligned unit -> ragged unit:
-    //   causal forward   [319,648,648] 43.2 -> 42.6, [134,1000,1000] 71.4 -> 68.8, [126,1032,1032] 74.7 -> 69.3, [67,1416,1416] -2.2 %, [51,1608,1608]
-    //                    -1.4 %, [440,552,552] +1.6 %; with ALiBi or dropout -2...-17 % at 1025-1480 columns, +7...-2 % below (the same sums
-    //                    either way), [57,1528,1528] with dropout +3 % (other sums: neither goes)
-    //   causal backward  520-3064 columns -1...-7 %: [496,520,520] -6.4 %, [134,1000,1000] -4.4 %, [31,2056,2056] -4.6 %; with dropout +1...+7 %
-    //   mask tensor with known row ends: forward 832-2048 columns 0...-8 %, [8,26,712,712] -1.6 %, [8,25,800,800] +1.2 %, [8,61,520,520] +5 %;
-    //                    backward 513-2048 columns -0.3...-8 %; without the ends the aligned kernels fetch no hidden key: +5...+14 %
-    // Few rows do not fill the staged kernels' longer chain: [9,1032,1032] backward +3 %, mask-tensor +3 and +8 %, [9,1656,1656] +1 %.
+    // Aligned rows that are no whole number of cache lines, many of them: by the kRagged unit too, most of whose kernels for up to
+    // 3072 columns store a block's rows in accesses aligned to lines (see Rows), where the row kernels store parts of lines at both
+    // ends of every access.  % per launch of the aligned unit against the ragged one, fp16 / bf16, 2^26 elements, buffers changing:
+    //   causal forward   [75,944,944] level, [67,1000,1000] +2.0, [63,1032,1032] +6.1, [47,1192,1192] +3.9, [33,1416,1416] +2.1, [30,1480,1480]
+    //                    +1.4, [102,808,808] -1.1 / -0.6 (not staged there); with ALiBi, a bias or dropout at 1032-1400 columns +2...+19, below
+    //                    -7...+2, [57,1528,1528] with dropout -3 (other sums: neither goes)
+    //   causal backward  [145,680,680] +3.1 / +1.4, [82,904,904] +4.1 / +3.9, [63,1032,1032] +1.6 / +5.3, [30,1480,1480] +1.0 / +1.2, [17,2040,2040]
+    //                    +2.8 / +2.6; two staged waves per row above 2048, [11,3064,3064] +4.2 / +3.8; not staged below 672 columns, [248,520,520]
+    //                    0 / -1.7; with dropout -7...-1
+    //   mask tensor with known row ends: forward [82,904,904] +0.1 / +0.7, [28,1544,1544] +8.6 / +10.9, [8,26,712,712] +1.6, [8,25,800,800] -1.2,
+    //                    [8,61,520,520] -5; backward [248,520,520] +5.6 / +3.7, [96,840,840] +3.2 / +3.7, [18,2040,2040] +6.4 / +6.8: the ragged unit
+    //                    ends the rows where the aligned one reads the probabilities to see what is hidden, also where it does not
+    //                    stage; without the ends the aligned kernels fetch no hidden key: -5...-14
+    // Few rows do not fill the staged kernels' longer chain: [9,1032,1032] backward -3 %, mask-tensor -3 and -8 %, [9,1656,1656] -1 %.
     bool through_lds(bool backward, Mask m) const {
         if (a.rows < 32768 || a.sk <= kChunk || a.sk % (kLine / 2) == 0) return false;
         const bool plain = (features & (kAlibi | kBias | kDropout)) == 0;
         if (backward) {
             if ((features & kDropout) != 0) return false;
-            if (m == Mask::Causal) return a.sk <= 3072;
+            if (m == Mask::Causal) return a.sk >= 672 && a.sk <= 3072;
             return a.row_end != nullptr && a.sk <= 2048;
         }
-        if (m == Mask::Causal) return a.sk <= 1480 && a.sk >= (plain ? 640 : 1025);
+        if (m == Mask::Causal) return a.sk <= 1480 && a.sk >= (plain ? 944 : 1025);
         // (above two chunks the call without the ends sums in one wave per row, like the ragged kernels, only if 32 bits address the mask)
         return plain && a.row_end != nullptr && a.sk >= 832 && a.sk <= 2048 && (a.sk <= 2 * kChunk || a.mask_bytes != 0);
     }

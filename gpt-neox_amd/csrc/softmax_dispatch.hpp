@@ -324,6 +324,23 @@ static bool two_causal_rows(const SoftmaxArgs& a, int chunks) {
     else return (EXTRA & kDropout) != 0 && a.sk % 8 == 4;
 }
 
+// Ragged rows of two chunks: the block's results through LDS (see Rows) where the call is large enough to be bound by what its stores
+// do to the lines; below, the barrier and the detour cost more.  % per launch of direct against staged, fp16 / bf16, buffers changing:
+//   causal forward       [40,945,945] -4.5 / -4.4, [64,1001,1001] -2.2 / -1.8, [128,1023,1023] +0.6 / +0.9, [250,1001,1001] +3.5 / +2.0
+//   mask-tensor forward  [40,961,961] -1.8, [64,1001,1001] +0.3 / +0.5, [128,945,945] +1.1 / +0.8, [200,1001,1001] +2.5 / +2.6; [9,1001,1001] -9
+//   full-row backward    [24,673,673] -0.7 / -3.1, [64,673,673] +2.0 / -0.1, [24,901,901] +1.2 / +0.9, [16,805,805] -0.2 / -1.2, [32,1001,1001] +2.9 / +1.9
+//   causal backward      [128,673,673] -0.3 / -1.9, [128,769,769] +1.9 / +0.2, [48,805,805] -0.9 / -1.1, [64,901,901] +0.9 / +0.6, [16,901,901] -2.1 / -2.6
+// Aligned rows that come here (through_lds, 32768 of them and more) begin and end on 16 bytes: causal forward [34,968,968] -0.6, [80,1000,1000]
+// +2.5, backward [52,776,776] +1.5, [140,840,840] +2.9, [52,648,648] 0.
+// With dropout behind throughout ([96,1001,1001] 94.2 -> 96.1 us and 86.6 -> 90.0).
+template <Mask M, bool BWD>
+static bool staged_two_chunks(const SoftmaxArgs& a, bool vec_ok) {
+    if (vec_ok) return a.sk >= (BWD ? 672 : 944);
+    if constexpr (!BWD) return a.sk >= 944 && a.rows >= (M == Mask::Causal ? 131072u : 65536u);
+    if constexpr (M == Mask::Causal) return a.sk >= 896 ? a.rows >= 40960 : a.sk >= 720 && a.rows >= 98304;
+    return a.sk >= 672 && a.rows >= (a.sk >= 768 ? 18432u : 40960u);
+}
+
 // Ragged rows of three or four chunks: one wave per row instead of two, four rows per block, the results through LDS.
 // (Two waves leave a quarter of their slots empty at three chunks and meet at barriers; staged on top, they lose 5-13 %.)  us per
 // launch, fp16, 2^27 elements, two waves -> one, forward / backward / mask-tensor forward with padding / its backward:
@@ -361,12 +378,7 @@ static hipError_t dispatch_rows(const SoftmaxArgs& a, bool vec_ok, hipStream_t s
     if constexpr (!(BWD && M == Mask::None && (EXTRA & kRagged) == 0)) {
         if (chunks == 2) {
             if constexpr (EXTRA == kRagged) {
-                // the block's results through LDS where the rows fill most of their two chunks (see Rows); us per launch, fp16, 2^26
-                // elements, direct -> staged: forward [92,851,851] 36.9 -> 37.5, [82,901,901] 36.9 -> 36.8, [74,951,951] 36.6 -> 36.2,
-                // [64,1022,1022] 36.7 -> 36.1, backward [185,601,601] 50.0 both, [136,701,701] 49.6 -> 48.8, [65,1009,1009] 48.4 -> 47.1;
-                // with dropout behind throughout ([96,1001,1001] 94.2 -> 96.1 and 86.6 -> 90.0)
-                // ([4,1001,1001] forward 4.73 -> 4.82, [1,1001,1001] 3.55 -> 3.62: not with few rows)
-                if (a.sk >= (BWD ? 672 : 944) && a.rows >= 8192) return launch_shape<T, M, BWD, EXTRA | kStaged, 2, 1, 4>(a, st);
+                if (staged_two_chunks<M, BWD>(a, vec_ok)) return launch_shape<T, M, BWD, EXTRA | kStaged, 2, 1, 4>(a, st);
             }
             if constexpr (M == Mask::Causal && (EXTRA & kRagged) == 0) {
                 // Both chunks' loads in front of the first one's arithmetic.  us per launch, fp16, without -> with: forward [4,960,960] 5.0 -> 3.8,

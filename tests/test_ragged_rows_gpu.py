@@ -158,15 +158,17 @@ def check_backward(written, run, y, g, offsets, dtype):
     assert_grad(dx, SCALE * yf * (gf - (gf * yf).sum(-1, keepdim=True)), dtype, written.what, y=y, g=g, scale=SCALE)
 
 
-# 8193 rows: where the results of rows of two chunks leave through LDS (from 672 columns on in the backward pass, from 944 in the forward
-# pass), and those of two waves per row in the backward pass (2049 to 2304 columns); the last block holds a single row
-@pytest.mark.parametrize("sk", [671, 673, 943, 945, 1001, 1023, 1535, 2047, 2051, 2303])
+# as many rows as it takes for the results to leave through LDS, and one case on the other side of each limit: of two chunks in the
+# backward pass (40960 rows from 672 columns on, 18432 from 768) and in the forward pass (65536 from 944), and of two waves per row in
+# the backward pass (8192, 2049 to 2304 columns); the last block is not full
+@pytest.mark.parametrize("sk,sq", [(671, 13655), (673, 13655), (673, 6145), (767, 6145), (769, 6145), (1023, 6143), (943, 21847), (945, 21847), (1001, 21847),
+                                   (1001, 21845), (1535, 2731), (2047, 2731), (2051, 2731), (2303, 2731)])
 @pytest.mark.parametrize("offsets", [(0, 0), (1, 0), (3, 5), (8, 1)])
-def test_staged_rows_of_many_rows(device, sk, offsets):
+def test_staged_rows_of_many_rows(device, sk, sq, offsets):
     lib, stream = _lib.lib(), torch.cuda.current_stream().cuda_stream
     dtype = (torch.float16, torch.bfloat16)[(sk // 2 + offsets[0]) % 2]
     code, gen = _lib.dtype_code(dtype), torch.Generator(device=device).manual_seed(sk)
-    b, sq = 3, 2731
+    b = 3
     shape, (i, o) = (b, 1, sq, sk), offsets
     x, _ = at(i, shape, dtype, device, gen=gen, std=8.0)
     g, _ = at(i, shape, dtype, device, gen=gen)
@@ -185,9 +187,9 @@ def test_staged_rows_of_many_rows(device, sk, offsets):
                    y, g, offsets, dtype)
 
 
-# causal rows, as many as it takes: 6400 for the two outputs of dropout through LDS, 4608 for two staged waves per row in the backward
-# pass; the last block is not full
-@pytest.mark.parametrize("sk,n", [(1301, 5), (1601, 5), (1855, 5), (2051, 3), (3071, 3)])
+# causal rows likewise: 131072 for two chunks in the forward pass (from 944 columns on), 98304 and 40960 in the backward pass (720, 896);
+# 6400 for the two outputs of dropout, 4608 for two staged waves per row in the backward pass
+@pytest.mark.parametrize("sk,n", [(725, 137), (905, 46), (1001, 131), (1001, 129), (1301, 5), (1601, 5), (1855, 5), (2051, 3), (3071, 3)])
 @pytest.mark.parametrize("offsets", [(0, 0), (1, 0), (3, 5), (8, 1)])
 def test_staged_causal_rows_of_many_rows(device, sk, n, offsets):
     lib, stream = _lib.lib(), torch.cuda.current_stream().cuda_stream
