@@ -14,9 +14,10 @@
 //   chunks <= 16   8 waves per row, 512-thread block                 (sk <= 8192)
 //   chunks <= 32   16 waves per row, 1024-thread block               (sk <= 16384)
 //                  forward, in the lower 3/4 of each of these three ranges (7/8 of the last):
-//                  half as many waves with 3 (4) chunks each; backward (causal, or with dropout) likewise at
-//                  2049-3072, 4097-6144 and 8193-12288 columns; mask-tensor forward at 513-2048
-//                  columns (unless the call
+//                  half as many waves with 3 (4) chunks each; backward likewise, causal at 2049-3072 (if there
+//                  are rows enough), 4097-6144 and 8193-12288 columns, full rows with dropout at 2049-3072 and
+//                  4097-6144 (ragged ones to 5120), ragged full rows without at 2049-2304 (8192 rows and
+//                  more) and 4097-4608; mask-tensor forward at 513-2048 columns (unless the call
 //                  knows where its rows end) and causal forward at 1025-1408: packed kernel, two
 //                  rows of two chunks or one row of three or four chunks per wave
 //   chunks <= 64   16 waves per row with 3 or 4 chunks per wave      (sk <= 32768)
@@ -437,15 +438,30 @@ static hipError_t dispatch_rows(const SoftmaxArgs& a, bool vec_ok, hipStream_t s
         //     93.9 -> 92.1, its results staged 89.9, with dropout 118.6 -> 106.7; [14,3071,3071] 91.5 -> 93.2, staged 89.6
         //   [7,4160,4160] 88.5 -> 80.1 / 98.3 -> 83.1 / 95.8 -> 83.5 / 135.6 -> 114.2, [5,5120,5120] 89.8 -> 87.5 / 103.8 -> 102.9 / 95.8 -> 88.7 /
         //     126.2 -> 110.5, [3,6144,6144] 75.6 -> 74.8 / 88.8 -> 91.1 / 78.6 -> 75.5 / 110.3 -> 107.6
-        //   with few rows: causal [1,2112,2112] 5.9 -> 6.1, with dropout [2,2112,2112] 10.0 -> 10.9, [4,2112,2112] level, full rows [1,2112,2112] 8.0
-        //     -> 7.5, ragged [1,2901,2901] 11.7 -> 11.9, [4,2901,2901] 35.2 -> 35.7
+        //   full rows with dropout to the end of the range, [2,5600,5600] -5.4 %, [1,5888,5888] -5 %, [4,5632,5632] 120.9 -> 110.1, but ragged ones
+        //     beyond ten chunks [2,5131,5131] +0.6 %, [1,5635,5635] +1.3 %, [3,5891,5891] -1.6 %
+        //   with few rows: causal [1,2112,2112] 5.9 -> 6.1, with dropout [2,2112,2112] 10.0 -> 10.9, [3,2192,2192] +3.4 % (fp16), +5.4 % (bf16),
+        //     [4,2432,2432] -2.8 and -0.7 %, [3,2728,2728] +2 %, [6,2728,2728] -1 %; without dropout [2,2688,2688] 0 and +2 %, [3,2496,2496] -0.6 %;
+        //     full rows [1,2112,2112] 8.0 -> 7.5, ragged [1,2901,2901] 11.7 -> 11.9, [4,2901,2901] 35.2 -> 35.7
+        //   aligned causal rows that nearly fill six chunks, where the smaller number of waves is all that is left of it, by what part of a
+        //     line they end on, fp16 / bf16: [6,2848,2848] and [6,2912,2912] (half a line) -1...-3 %, [6,2984,2984] and [6,3048,3048] +1.7...+3.5 / +0.4...+2,
+        //     whole lines [6,2944,2944] +1.9 / -0.4 and [6,3008,3008] +1.9 / 0, full [6,3072,3072] -1.6 / -2.7; with dropout +0.5...+2.3 on parts of a
+        //     line, -0.7...-4 on halves and whole lines (from 32768 rows on they go to the ragged unit, -2...-7 %)
         // Aligned full rows without dropout: not at all.  They gain where the padding hides much of a sample (the figures above) and lose where
         // nothing is hidden, [1,30,2112,2112] 124.7 -> 127.5, [1,8,4608,4608] 158.3 -> 163.7, [1,8,5120,5120] 194.1 -> 203.9, and a call
         // that knows where its rows end must sum in the order of one that does not.
         if constexpr (M == Mask::Causal || EXTRA != 0) {
-            const bool enough = M == Mask::Causal ? a.rows >= 4608 : EXTRA != kRagged || (a.rows >= 8192 && a.sk <= 2304);
+            constexpr bool drop = (EXTRA & kDropout) != 0;
+            bool enough = EXTRA != kRagged || (a.rows >= 8192 && a.sk <= 2304);
+            if constexpr (M == Mask::Causal) {
+                enough = a.rows >= 4608;
+                if constexpr ((EXTRA & kRagged) == 0) {
+                    const bool ends = a.sk % (kLine / 4) == 0 && (drop || a.sk % (kLine / 2) != 0 || a.sk == 6 * kChunk);
+                    enough = a.rows >= (drop ? 9216u : 6144u) && (a.sk <= 2816 || ends);
+                }
+            }
             if (chunks <= 6 && enough) return launch_shape<T, M, BWD, EXTRA | (EXTRA == kRagged ? kStaged : 0), 3, 2, 2>(a, st);
-            constexpr int most = M == Mask::Causal ? 12 : EXTRA == kRagged ? 9 : 10;
+            constexpr int most = M == Mask::Causal || EXTRA == kDropout ? 12 : EXTRA == kRagged ? 9 : 10;
             if (chunks > 8 && chunks <= most) return launch_shape<T, M, BWD, EXTRA, 3, 4, 1>(a, st);
         }
     }
