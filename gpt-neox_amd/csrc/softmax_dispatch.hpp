@@ -352,11 +352,11 @@ static bool staged_two_chunks(const SoftmaxArgs& a, bool vec_ok) {
 // with ALiBi [60,1049,1049] 44.8 -> 36.3, [20,1801,1801] 36.4 -> 36.1, with a bias 47.7 -> 41.2 and 41.2 -> 40.6, with dropout 76.9 ->
 // 67.0 and 64.3 -> 64.7, its backward 65.4 -> 58.7 and 56.1 -> 53.9.  All feature sets take the same shape: the same sums.
 // The backward pass with few rows keeps two waves: full rows [1,1601,1601] 6.0 -> 6.3, [4,1601,1601] 13.8 -> 14.1, causal [1,1601,1601]
-// 4.9 -> 5.1, [2,1601,1601] 7.5 -> 6.8, [1,1301,1301] level.
+// 4.9 -> 5.1, [2,1601,1601] 7.5 -> 6.8, [1,1301,1301] level; with dropout [2,1868,1868] +3.8 %, [2,1900,1900] +3.5 %, [3,1868,1868] -14 %, [2,1707,1707] -10 %.
 template <Mask M, bool BWD>
-static bool one_wave_ragged(const SoftmaxArgs& a, int chunks) {
+static bool one_wave_ragged(const SoftmaxArgs& a, int chunks, bool dropout) {
     if constexpr (!BWD) return M != Mask::Causal || a.sk <= 1856;
-    return M == Mask::None ? a.rows >= 8192 : chunks == 3 || a.rows >= 2048;
+    return M == Mask::None ? a.rows >= 8192 : chunks == 3 || a.rows >= (dropout && a.sk > 1792 ? 4096u : 2048u);
 }
 
 template <typename T, Mask M, bool BWD, int EXTRA>
@@ -399,7 +399,7 @@ static hipError_t dispatch_rows(const SoftmaxArgs& a, bool vec_ok, hipStream_t s
             // mask-tensor forward with dropout, [8,7,1049,1049] 95.4 and 99.3, [8,3,1601,1601] 84.2 and 88.0
             constexpr bool staged = (EXTRA & kDropout) == 0 || (!BWD && M == Mask::Causal);
             constexpr int FL = EXTRA | (staged ? kStaged : 0);
-            if (chunks <= 4 && one_wave_ragged<M, BWD>(a, chunks)) {
+            if (chunks <= 4 && one_wave_ragged<M, BWD>(a, chunks, (EXTRA & kDropout) != 0)) {
                 // with dropout, few rows: [3,1701,1701] 13.1 us with two waves, 11.2 staged, 10.2 not; [4,1801,1801] 17.3, 15.4, 18.1;
                 // [1,1601,1601] 7.2, 7.8, 6.7
                 if constexpr (staged && (EXTRA & kDropout) != 0) {
