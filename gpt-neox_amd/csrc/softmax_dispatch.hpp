@@ -25,8 +25,8 @@
 //                  blocks per CU (sk <= 40448), or in all of it       (sk <= 81408)
 //   ragged rows    (sk % 8 != 0 or pointers not 16-byte aligned; 8 <= sk < 81408)
 //                  the same packed, one- to sixteen-wave row and LDS-staged kernels with the kRagged flag; three and
-//                  four chunks (causal forward: up to 1856 columns) in one wave, results of one-wave rows staged
-//                  in LDS (kStaged)
+//                  four chunks (causal forward: up to 1856 columns) in one wave, results of one-wave rows and of
+//                  the backward pass in two waves staged in LDS where it pays (kStaged)
 //   sliding window (kBand) the row kernels, aligned rows of 513-32768 columns: dispatch_band_rows
 //   anything else  element-wise kernels (rows shorter than 8 columns or beyond 81408)
 #pragma once
@@ -484,21 +484,26 @@ static hipError_t dispatch_rows(const SoftmaxArgs& a, bool vec_ok, hipStream_t s
 // touch -- w + 1 keys lie in at most w / 512 + 2 of them, `chunks` -- and by those of the row: the waves hold the band, the rest of the
 // row is zeros, which they store as well (band_zero_fill).  TB/s by algorithmic bytes, bf16, 2^27 elements, [columns, window], the shape
 // of the rule against the one that the band alone would call for (chunks / 2 waves with two chunks, from 4097 columns on
-// chunks waves with one).  With few rows fewer waves per row or more of them lose 2-10 % ([1,2048,2048] window 256 backward 3.6 -> 3.9 us,
-// [4,1536,1536] 384 forward 5.5 -> 5.9): `many`.
+// chunks waves with one).  With few rows other shapes lose 2-10 %, in the forward pass those with fewer waves per row, in the backward pass
+// those with one chunk per wave ([1,2048,2048] window 256 backward 3.6 -> 3.9 us, [4,1536,1536] 384 forward 5.5 -> 5.9): `many`.
 //   forward   rows of three chunks: one wave, [1152,576] 4.54 -> 5.82, [1536,768] 5.55 -> 5.89, [1536,256] 5.37 -> 5.46, [1152,288] 5.46 -> 5.50
 //     of four: two waves with two rows per block, [2048,1024] 5.99 -> 6.14, [2048,600] 5.74 -> 5.97
-//     of five to eight: one wave at two chunks, [2560,256] 5.08 -> 5.29, [3072,400] 5.19 -> 5.30; two waves with three chunks each at
-//       three to six, [3072,1000] 5.67 -> 5.78, [3072,1400] 5.70 -> 5.97, [3072,1600] 5.43 -> 6.03, [2560,1600] 5.16 -> 5.96, but [2560,700]
+//     of five to eight: one wave at two chunks, [2560,256] 5.08 -> 5.29, [3072,400] 5.19 -> 5.30, with four chunks up to 2560 columns or for
+//       windows of 256 and more (us, four -> two: [5,3072,3072] 142 -2 %, [5,3584,3584] 180 -2 %, [8,3072,3072] 256 +1 %); two waves with
+//       three chunks each at three to six, [3072,1000] 5.67 -> 5.78, [3072,1400] 5.70 -> 5.97, [3072,1600] 5.43 -> 6.03, [2560,1600] 5.16 -> 5.96, but [2560,700]
 //       5.63 -> 5.61; with four from 3073 columns on at five and six, [3584,1792] 5.56 -> 5.82
-//   backward  one chunk per wave: [2048,384] 5.88 -> 6.17, [2560,400] 5.41 -> 5.52, [1472,368] 5.45 -> 5.59, [1536,128] level; [3072,768]
+//   backward  one chunk per wave: [2048,384] 5.88 -> 6.17, [2560,400] 5.41 -> 5.52, [1472,368] 5.45 -> 5.59, [1536,128] level (rows of three chunks
+//       that end on half or whole lines, window 200: [12,1472,1472] +4 %, [24,1504,1504] +4 %, [12,1536,1536] +3 %; 300 0...-2 %, [12,1512,1512] 200 -1.7 %); [3072,768]
 //     5.63 -> 5.72, [3584,896] 5.52 -> 5.76, [3072,1100] 5.70 -> 5.89, [2560,1280] 5.84 -> 5.92, but [2560,700] 5.69 -> 5.5; [8192,1600] 5.62 -> 5.81,
 //     [8192,3000] 5.73 -> 5.93, [7168,1792] 5.55 -> 5.72, [6144,3072] 5.83 -> 5.94, but [5120,2560] 5.87 -> 5.79
 //   4096 columns, rows of two 4 KiB pieces, two per block in the order of with_xcd_mapping: [4096,256] 5.4 -> 5.78 and backward 5.32 -> 5.80,
 //     [4096,1024] 5.86 -> 5.96 (forward), [4096,2048] 5.65 -> 6.15 and 5.99 -> 6.13, [4096,2560] 5.81 -> 6.21 and 6.13 -> 6.22; three waves' worth
 //     at three chunks [4096,1000] 5.86 -> 5.97, [4096,512] -1 %.  Off the 4 KiB boundary that order does not apply: as other lengths.
-//   beyond 4096 columns one chunk per wave up to four chunks, [8192,256] 5.36 -> 5.68 and 5.36 -> 5.49, [5000,1250] 252 -> 236 us and 294 -> 274,
-//     (forward at two chunks: from 16 chunks of the row on, [4608,400] 46.2 -> 52.4), up to 28 chunks of the row: [15360,1024] 200 -> 204 us, [16384,1500] 210 -> 232, [32768,1024] 408 -> 446
+//   beyond 4096 columns one chunk per wave up to four chunks, [8192,256] 5.36 -> 5.68 (forward), [5000,1250] 252 -> 236 us and 294 -> 274,
+//     (forward at two chunks: from 16 chunks of the row on, [4608,400] 46.2 -> 52.4; backward at two chunks up to 16 only where rows end inside a
+//     line, us, fp16, window 256: [2,5000,5000] -12 %, [2,6160,6160] -12 %, but [2,5088,5088] +6 %, [2,6144,6144] +7 %, [2,7136,7136] +9 %, [2,8192,8192]
+//     +5 %; [2,9216,9216] -10 %; five to eight chunks in the backward pass with few rows too, [1,7680,7680] 3000 -5 %, [1,8184,8184] 2600 -8 %),
+//     up to 28 chunks of the row: [15360,1024] 200 -> 204 us, [16384,1500] 210 -> 232, [32768,1024] 408 -> 446
 template <typename T, bool BWD>
 static hipError_t dispatch_band_rows(const SoftmaxArgs& a, hipStream_t st) {
     constexpr Mask M = Mask::Causal;
@@ -518,14 +523,15 @@ static hipError_t dispatch_band_rows(const SoftmaxArgs& a, hipStream_t st) {
     if (row <= 8) {
         if constexpr (!BWD) {
             if (row == 3 && (chunks == 3 || (a.window >= 256 && a.rows >= 32768))) return launch_shape<T, M, BWD, B, 3, 1, 4>(a, st);
-            if (chunks == 2 && (row <= 4 || !many)) return launch_shape<T, M, BWD, B, 2, 1, 4>(a, st);
+            if (chunks == 2 && (row <= 4 || !many || (row > 5 && a.window < 256))) return launch_shape<T, M, BWD, B, 2, 1, 4>(a, st);
             if (chunks == 2) return launch_shape<T, M, BWD, B, 4, 1, 4>(a, st);
             if (row == 4 || (chunks == 3 && (row == 5 || !many))) return launch_shape<T, M, BWD, B, 2, 2, 2>(a, st);
             if (chunks == 4 && !many) return launch_shape<T, M, BWD, B, 2, 2, 4>(a, st);
             if (chunks <= 4 || (chunks <= 6 && row <= 6)) return launch_shape<T, M, BWD, B, 3, 2, 2>(a, st);
             if (chunks <= 6 && row == 7) return launch_shape<T, M, BWD, B, 4, 2, 2>(a, st);
         } else {
-            if (chunks == 2 && a.sk > 1408 && a.window >= 192 && many) return launch_shape<T, M, BWD, B, 1, 2, 2>(a, st);
+            const int narrow = row == 3 && a.sk % (kLine / 4) == 0 ? 256 : 192;
+            if (chunks == 2 && a.sk > 1408 && a.window >= narrow && many) return launch_shape<T, M, BWD, B, 1, 2, 2>(a, st);
             if (chunks == 2) return launch_shape<T, M, BWD, B, 2, 1, 4>(a, st);
             if (many && ((chunks == 3 && row >= 6) || (chunks == 4 && row >= 5))) return launch_shape<T, M, BWD, B, 1, 4, 1>(a, st);
             if (chunks == 3) return launch_shape<T, M, BWD, B, 2, 2, 2>(a, st);
@@ -534,7 +540,8 @@ static hipError_t dispatch_band_rows(const SoftmaxArgs& a, hipStream_t st) {
         return launch_shape<T, M, BWD, B, 2, 4, 1>(a, st);
     }
     if (chunks <= 4) {
-        if (row <= 28 && (chunks > 2 || (BWD ? many : row >= 16))) return launch_shape<T, M, BWD, B, 1, 4, 1>(a, st);
+        const bool two = BWD ? many && (row > 16 || a.sk % (kLine / 4) != 0) : row >= 16;
+        if (row <= 28 && (chunks > 2 || two)) return launch_shape<T, M, BWD, B, 1, 4, 1>(a, st);
         if (chunks == 2) return launch_shape<T, M, BWD, B, 2, 1, 4>(a, st);
         return chunks == 3 ? launch_shape<T, M, BWD, B, 2, 2, 2>(a, st) : launch_shape<T, M, BWD, B, 2, 2, 4>(a, st);
     }

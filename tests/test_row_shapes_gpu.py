@@ -42,7 +42,7 @@ def check(x, y, g, dx, hidden, dtype, what):
 @pytest.mark.parametrize("s,w,batches", [(1152, 288, 29), (1152, 288, 2), (1152, 576, 1), (1472, 368, 6), (2048, 384, 4), (2048, 600, 1),
                                          (2048, 1024, 1), (2560, 256, 4), (2560, 700, 1), (2560, 1600, 1), (3072, 600, 3), (3072, 600, 2),
                                          (3072, 1400, 3), (3584, 1200, 3), (3584, 1792, 1), (4096, 200, 2), (4096, 200, 1), (4096, 600, 1),
-                                         (4096, 700, 2), (4096, 1100, 1), (4096, 2600, 1), (4608, 400, 2), (6144, 3000, 1), (8192, 256, 1),
+                                         (4096, 700, 2), (4096, 1100, 1), (4096, 2600, 1), (4608, 400, 2), (4616, 400, 2), (1504, 200, 6), (1504, 300, 6), (2816, 200, 3), (9216, 200, 1), (6144, 3000, 1), (8192, 256, 1),
                                          (8192, 1600, 1)])
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_sliding_window_shapes_by_rows(device, s, w, batches, dtype):
