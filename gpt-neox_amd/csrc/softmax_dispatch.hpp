@@ -286,11 +286,14 @@ static std::optional<hipError_t> dispatch_aligned(const SoftmaxArgs& a, bool vec
         if (chunks == 3 && a.sk <= 1408 && fits32) return launch_packed_shape<T, M, BWD, EXTRA, kWave, 1, 3>(a, st);
     }
     if constexpr (BWD && M == Mask::Causal && (EXTRA & kDropout) != 0) {
-        // causal backward with dropout, 1025-1344 columns: one wave per row with three chunks, two rows per block; the Philox rounds of
-        // a fourth chunk slot are work for nothing.  us per launch, fp16, two waves per row -> one: [113,1088,1088] 104.9 -> 93.0, [81,1280,1280]
-        // 96.8 -> 90.7, [67,1408,1408] 94.0 -> 90.3, [61,1472,1472] 90.7 -> 90.1, but [8,1408,1408] 14.8 -> 15.3; without dropout +1...+3 % throughout,
-        // and with few rows [1,1280,1280] 4.5 -> 5.0, [3,1280,1280] 6.6 -> 7.4, [4,1088,1088] 7.7 -> 7.3
-        if (chunks == 3 && a.sk <= 1344 && a.rows >= 4608) return launch_shape<T, M, BWD, EXTRA, 3, 1, 2>(a, st);
+        // causal backward with dropout, 1025-1344 columns, many rows: one wave per row with three chunks, two rows per block; the Philox rounds
+        // of a fourth chunk slot are work for nothing.  us per launch, fp16, two waves per row -> one: [113,1088,1088] 104.9 -> 93.0, [81,1280,1280]
+        // 96.8 -> 90.7; %, fp16 / bf16, buffers changing: [9,1056,1056] +1.2 / +1.5, [12,1280,1280] -0.4 / +2.6, [19,1152,1152] -3.5 / +0.3, [28,1088,1088]
+        // -6.9 / -1.9, [28,1248,1248] -2.9 / +1.5, [40,1280,1280] -5.5 / -1.9; above 1280 columns [19,1304,1304] +1.8 / +4.3, [40,1336,1336] +2.5 / +3.2, whole
+        // and half lines [40,1312,1312] -3.8 / +0.1, [64,1344,1344] -7.0 / -2.8, beyond [67,1408,1408] 94.0 -> 90.3 us, but [8,1408,1408] 14.8 -> 15.3;
+        // without dropout +1...+3 % throughout
+        constexpr uint32_t least = std::is_same<T, F16>::value ? 18432 : 36864;
+        if (chunks == 3 && a.rows >= least && a.sk <= (a.sk % (kLine / 4) == 0 ? 1344 : 1280)) return launch_shape<T, M, BWD, EXTRA, 3, 1, 2>(a, st);
     }
     if constexpr (BWD && M == Mask::None) {
         // full rows up to 2048 columns: straight-line packed kernel, R x C = 4 accesses per tensor
