@@ -595,8 +595,11 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void softmax_fwd_kernel(SoftmaxArg
                 // a conversion.  us per launch, in the branches -> in front: window 160 of 640 columns [327,640,640] 77.7 -> 73.8 (with the
                 // one comparison), [510,513,513] fp16 82.7 -> 81.1, with ALiBi 86.3 -> 84.6; aligned rows with mask bytes,
                 // [8,50,576,576] 82.5 -> 92.6: in the branches.  So are aligned bf16 rows of several waves with ALiBi, which convert either way:
-                // [2720,2720] 5.03 in the branches, 5.14 in front, [2848,2848] 5.14 and 5.29 (fp16 level, with a window 0-4 % for in front).
-                constexpr bool kBranches = std::is_same<T, BF16>::value && (FLAGS & kAlibi) != 0 && WPR > 1;
+                // [2720,2720] 5.03 in the branches, 5.14 in front, [2848,2848] 5.14 and 5.29 (fp16 level, with a window 0-4 % for in front),
+                // and rows of eight waves with three and four chunks with dropout, [9128,9128] 81.8 and 83.6, [2,9216,9216] -2.2 and -3.1 % (two
+                // chunks 0...+1 %).
+                constexpr bool kBranches = (std::is_same<T, BF16>::value && (FLAGS & kAlibi) != 0 && WPR > 1) ||
+                                           ((FLAGS & (kAlibi | kBias | kDropout)) == kDropout && WPR == 8 && NCH > 2);
                 if constexpr (kRag || (MASK != Mask::Bytes && !kBranches)) {
 #pragma unroll
                     for (int k = 0; k < 8; ++k) v[c][k] = fmaf(v[c][k], a.scale, bias[k]);  // bias 0: the plain product
