@@ -464,8 +464,14 @@ static hipError_t dispatch_rows(const SoftmaxArgs& a, bool vec_ok, hipStream_t s
                 }
             }
             if (chunks <= 6 && enough) return launch_shape<T, M, BWD, EXTRA | (EXTRA == kRagged ? kStaged : 0), 3, 2, 2>(a, st);
+            //   likewise aligned causal rows of eleven and twelve chunks, fp16 / bf16: [2,5440,5440] -1.8 / -7.0, [2,5888,5888] -0.7 / -6.2, [2,6144,6144] -0.3 / -5.1
+            //     (whole lines), [2,5328,5328] +1.5 / -3.4, [3,5840,5840] +1.6 / -1.5, [2,6008,6008] +2.1 / -1.7, [2,6112,6112] +0.9 / -1.9; with dropout [2,5440,5440] -4.6 /
+            //     -4.7, [2,5344,5344] -0.7 / -1.4, [2,5744,5744] +1.6 / +0.9, [1,5840,5840] +2.6 / +2.3, [2,6032,6032] +1.8 / +0.4
             constexpr int most = M == Mask::Causal || EXTRA == kDropout ? 12 : EXTRA == kRagged ? 9 : 10;
-            if (chunks > 8 && chunks <= most) return launch_shape<T, M, BWD, EXTRA, 3, 4, 1>(a, st);
+            bool pays = true;
+            if constexpr (M == Mask::Causal && (EXTRA & kRagged) == 0 && (drop || std::is_same<T, F16>::value))
+                pays = a.sk <= (drop ? 5632 : 5120) || a.sk % (kLine / 2) == 0;
+            if (chunks > 8 && chunks <= most && pays) return launch_shape<T, M, BWD, EXTRA, 3, 4, 1>(a, st);
         }
     }
     if constexpr (BWD && M == Mask::Causal) {
