@@ -329,20 +329,38 @@ static bool two_causal_rows(const SoftmaxArgs& a, int chunks) {
 }
 
 // Ragged rows of two chunks: the block's results through LDS (see Rows) where the call is large enough to be bound by what its stores
-// do to the lines; below, the barrier and the detour cost more.  % per launch of direct against staged, fp16 / bf16, buffers changing:
-//   causal forward       [40,945,945] -4.5 / -4.4, [64,1001,1001] -2.2 / -1.8, [128,1023,1023] +0.6 / +0.9, [250,1001,1001] +3.5 / +2.0
-//   mask-tensor forward  [40,961,961] -1.8, [64,1001,1001] +0.3 / +0.5, [128,945,945] +1.1 / +0.8, [200,1001,1001] +2.5 / +2.6; [9,1001,1001] -9
-//   full-row backward    [24,673,673] -0.7 / -3.1, [64,673,673] +2.0 / -0.1, [24,901,901] +1.2 / +0.9, [16,805,805] -0.2 / -1.2, [32,1001,1001] +2.9 / +1.9
-//   causal backward      [128,673,673] -0.3 / -1.9, [128,769,769] +1.9 / +0.2, [48,805,805] -0.9 / -1.1, [64,901,901] +0.9 / +0.6, [16,901,901] -2.1 / -2.6
+// do to the lines; below, the barrier and the detour cost more.  Rows of an even length, which begin on whole dwords, gain earlier.
+// % per launch of direct against staged by thousands of rows, both kernels in turn in one process, buffers changing, fp16 / bf16:
+//   causal forward       945: 45 -1.4 / -0.2, 60 -0.2 / -0.5, 75 +0.7 / -0.2, 120 +1.4 / +1.1; 1001: 24 -1.4 / -1.8, 48 -0.5 / -0.7, 64 +1.1 / +1.1, 96 +1.7 / +1.5,
+//                        128 +2.1 / +2.0; 946: 30 -0.5 / -2.0, 45 +1.9 / +0.5; 962: 46 -0.2 / +0.2, 61 +1.3 / +1.2; 1002: 24 -0.7 / 0, 48 +1.6 / +0.7
+//   mask-tensor forward  945: 45 -0.5 / -0.5, 60 -1.2 / -1.2; 1001: 48 -2.3 / -2.2, 64 -1.6 / -1.6; 1021: 49 -3.9 / -3.5; 1022: 16 -0.2 / -1.0, 32 +1.1 / +1.0, 49 +1.6 /
+//                        +1.2; 1023: 24 -0.4 / -1.6, 32 +0.7 / 0, 65 +2.7 / +2.4; other lengths from 65536 rows on, [128,945,945] +1.1 / +0.8, [200,1001,1001] +2.5 / +2.6
+//   causal backward      673: 64 -0.1 / -0.7, 86 +0.8 / +0.3; 721: 57 +0.2 / -0.3, 92 +1.5 / +1.1; 769: 24 -0.5 / -1.3, 36 +1.3 / -0.9, 49 +1.4 / -0.6, 61 +1.7 / +0.8; 865: 20
+//                        -1.1 / -2.0, 41 +0.8 / -0.9, 55 +1.3 / +1.0; 897: 21 -0.1 / -0.2, 28 +1.0 / +0.5; 1001: 16 +0.2 / +1.0, 24 +2.2 / +0.9, 32 +1.3 / +2.3; 674: 32 +0.3 /
+//                        -0.1, 53 +0.6 / +0.8; 722: 23 -1.1 / -1.0, 46 +1.1 / +1.0; 802: 25 +0.8 / +0.3, 38 +0.8 / +1.3
+//   full-row backward    673: 16 -0.3 / -2.6, 32 +0.5 / -0.3; 721: 23 +1.4 / -0.1, 34 +2.5 / -0.6; 674: 10 +0.2 / +2.1, 16 +2.6 / -1.0, 32 +2.6 / +1.7; 746: 11 +2.4 / +1.0, 35 +3.2 /
+//                        +2.8; from
+//                        768 columns on [24,901,901] +1.2 / +0.9, [16,805,805] -0.2 / -1.2, [32,1001,1001] +2.9 / +1.9
 // Aligned rows that come here (through_lds, 32768 of them and more) begin and end on 16 bytes: causal forward [34,968,968] -0.6, [80,1000,1000]
 // +2.5, backward [52,776,776] +1.5, [140,840,840] +2.9, [52,648,648] 0.
 // With dropout behind throughout ([96,1001,1001] 94.2 -> 96.1 us and 86.6 -> 90.0).
 template <Mask M, bool BWD>
 static bool staged_two_chunks(const SoftmaxArgs& a, bool vec_ok) {
     if (vec_ok) return a.sk >= (BWD ? 672 : 944);
-    if constexpr (!BWD) return a.sk >= 944 && a.rows >= (M == Mask::Causal ? 131072u : 65536u);
-    if constexpr (M == Mask::Causal) return a.sk >= 896 ? a.rows >= 40960 : a.sk >= 720 && a.rows >= 98304;
-    return a.sk >= 672 && a.rows >= (a.sk >= 768 ? 18432u : 40960u);
+    const bool odd = (a.sk & 1) != 0;
+    uint32_t least;
+    if constexpr (!BWD) {
+        if (a.sk < 944) return false;
+        least = M == Mask::Causal ? (odd ? 64000 : 45000) : a.sk >= 1022 ? 32768 : 65536;
+    } else {
+        if (a.sk < 672) return false;
+        if constexpr (M == Mask::Causal) {
+            least = a.sk >= 960 ? 20480 : a.sk >= 896 ? 27648 : a.sk >= 760 ? (odd ? 45056 : 32768) : odd ? 81920 : 49152;
+        } else {
+            least = a.sk >= 768 ? 18432 : odd ? 28672 : 8192;
+        }
+    }
+    return a.rows >= least;
 }
 
 // Ragged rows of three or four chunks: one wave per row instead of two, four rows per block, the results through LDS.
