@@ -288,11 +288,15 @@ static std::optional<hipError_t> dispatch_aligned(const SoftmaxArgs& a, bool vec
     if constexpr (BWD && M == Mask::Causal && (EXTRA & kDropout) != 0) {
         // causal backward with dropout, 1025-1344 columns, many rows: one wave per row with three chunks, two rows per block; the Philox rounds
         // of a fourth chunk slot are work for nothing.  us per launch, fp16, two waves per row -> one: [113,1088,1088] 104.9 -> 93.0, [81,1280,1280]
-        // 96.8 -> 90.7; %, fp16 / bf16, buffers changing: [9,1056,1056] +1.2 / +1.5, [12,1280,1280] -0.4 / +2.6, [19,1152,1152] -3.5 / +0.3, [28,1088,1088]
-        // -6.9 / -1.9, [28,1248,1248] -2.9 / +1.5, [40,1280,1280] -5.5 / -1.9; above 1280 columns [19,1304,1304] +1.8 / +4.3, [40,1336,1336] +2.5 / +3.2, whole
-        // and half lines [40,1312,1312] -3.8 / +0.1, [64,1344,1344] -7.0 / -2.8, beyond [67,1408,1408] 94.0 -> 90.3 us, but [8,1408,1408] 14.8 -> 15.3;
-        // without dropout +1...+3 % throughout
-        constexpr uint32_t least = std::is_same<T, F16>::value ? 18432 : 36864;
+        // 96.8 -> 90.7; % of two waves against one, by matrices, both kernels in turn in one process, buffers changing:
+        //   fp16  1056: 5 +2.8, 6 +4.9, 8 +1.4, 12 +3.1, 16 +4.4; 1088: 6 +7.0, 8 +1.4, 14 +4.4; 1120: 5 +2.4, 7 -0.5, 8 -0.6, 14 +1.6; 1152: 6 +4.8, 8 -0.4, 14 +3.4;
+        //         1184: 5 +3.9, 7 -2.2, 10 -0.3, 14 +1.4; 1248: 6 -3.8, 10 -2.2, 16 +0.1; 1304: 10 -3.1, 20 -2.1, 28 +1.8; 1336: 20 -2.5, 34 -1.5
+        //   bf16  1032: 6 -6.3, 20 0, 28 +0.9; 1056: 6 -5.0, 14 +1.0, 20 +1.8, 28 +3.0; 1088: 6 -3.8, 20 +1.6, 28 +2.3; 1152: 6 -4.0, 20 +0.5, 28 +1.8; 1200: 10 -3.7, 28
+        //         -1.0; 1248: 10 -4.1, 28 -0.7; 1336: 28 -3.8
+        // above 1280 columns [40,1336,1336] -2.5 / -3.2, whole and half lines [40,1312,1312] +3.8 / -0.1, [64,1344,1344] +7.0 / +2.8; beyond [67,1408,1408]
+        // 94.0 -> 90.3 us, but [8,1408,1408] 14.8 -> 15.3; without dropout one wave is 1-3 % slower throughout
+        const bool f16 = std::is_same<T, F16>::value;
+        const uint32_t least = a.sk <= 1152 ? (f16 ? 4608 : 20480) : f16 ? 18432 : 36864;
         if (chunks == 3 && a.rows >= least && a.sk <= (a.sk % (kLine / 4) == 0 ? 1344 : 1280)) return launch_shape<T, M, BWD, EXTRA, 3, 1, 2>(a, st);
     }
     if constexpr (BWD && M == Mask::None) {

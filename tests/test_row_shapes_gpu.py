@@ -56,7 +56,7 @@ def test_sliding_window_shapes_by_rows(device, s, w, batches, dtype):
 
 # 513-1024 columns with the loads in front or not; above 1024, 2048 and 4096 columns in the backward pass; rows that are no whole
 # cache lines, 32768 of them or fewer; odd rows, 2048 / 4608 / 6400 / 8192 of them or fewer
-@pytest.mark.parametrize("s,batches", [(576, 1), (888, 6), (1024, 5), (1088, 5), (1088, 4), (1088, 16), (1088, 17), (1088, 33), (1088, 34), (1304, 29), (2112, 3), (2112, 2), (2112, 5), (2824, 4), (2848, 3), (2848, 4), (2944, 4), (3072, 3), (4160, 1), (5136, 1), (5696, 1), (5704, 1), (520, 64), (520, 63),
+@pytest.mark.parametrize("s,batches", [(576, 1), (888, 6), (1024, 5), (1088, 5), (1088, 4), (1088, 16), (1088, 17), (1088, 33), (1088, 34), (1088, 18), (1088, 19), (1184, 15), (1184, 16), (1184, 31), (1184, 32), (1304, 29), (2112, 3), (2112, 2), (2112, 5), (2824, 4), (2848, 3), (2848, 4), (2944, 4), (3072, 3), (4160, 1), (5136, 1), (5696, 1), (5704, 1), (520, 64), (520, 63),
                                        (1000, 33), (1032, 32), (1416, 24), (1480, 23), (1488, 23), (2056, 16), (3064, 11), (1001, 9), (1001, 8), (1301, 5), (1301, 4),
                                        (1601, 2), (1601, 1), (1801, 4), (1801, 3), (1801, 2), (2051, 3), (2051, 2), (4101, 1)])
 @pytest.mark.parametrize("dtype", DTYPES)
