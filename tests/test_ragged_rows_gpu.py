@@ -161,8 +161,10 @@ def check_backward(written, run, y, g, offsets, dtype):
 # as many rows as it takes for the results to leave through LDS, and one case on the other side of each limit: of two chunks in the
 # backward pass (from 672 columns on 8192 rows of an even and 28672 of an odd length, 18432 from 768) and in the forward pass (from 944
 # columns on 65536, 32768 from 1022), and of two waves per row in the backward pass (8192, 2049 to 2304 columns); the last block is not full
-@pytest.mark.parametrize("sk,sq", [(671, 13655), (673, 13655), (673, 6145), (767, 6145), (769, 6145), (1023, 6143), (943, 21847), (945, 21847), (1001, 21847),
-                                   (1001, 21845), (673, 9557), (721, 9559), (722, 2729), (722, 2731), (1021, 10923), (1022, 10921), (1022, 10923), (1535, 2731), (2047, 2731), (2051, 2731), (2303, 2731)])
+@pytest.mark.parametrize("sk,sq", [(671, 13655), (673, 13655), (673, 6145), (767, 6145), (769, 6145), (1023, 6143), (943, 21847),
+                                   (945, 21847), (1001, 21847), (1001, 21845), (673, 9557), (721, 9559), (722, 2729), (722, 2731),
+                                   (1021, 10923), (1022, 10921), (1022, 10923), (1535, 2731), (2047, 2731), (2051, 2731),
+                                   (2303, 2731)])
 @pytest.mark.parametrize("offsets", [(0, 0), (1, 0), (3, 5), (8, 1)])
 def test_staged_rows_of_many_rows(device, sk, sq, offsets):
     lib, stream = _lib.lib(), torch.cuda.current_stream().cuda_stream
@@ -189,8 +191,9 @@ def test_staged_rows_of_many_rows(device, sk, sq, offsets):
 
 # causal rows likewise: for two chunks in the forward pass 64000 of an odd and 45000 of an even length (from 944 columns on), in the backward
 # pass 81920 and 49152 (672), 45056 and 32768 (760), 27648 (896) and 20480 (960); 6400 for the two outputs of dropout, 4608 for two staged waves per row in the backward pass
-@pytest.mark.parametrize("sk,n", [(725, 137), (905, 46), (1001, 131), (1001, 129), (673, 121), (673, 122), (674, 73), (769, 58), (769, 59), (802, 41), (905, 30), (905, 31),
-                                  (969, 21), (969, 22), (1001, 63), (1001, 65), (1002, 44), (1002, 45), (1301, 5), (1601, 5), (1855, 5), (2051, 3), (3071, 3)])
+@pytest.mark.parametrize("sk,n", [(725, 137), (905, 46), (1001, 131), (1001, 129), (673, 121), (673, 122), (674, 73), (769, 58),
+                                  (769, 59), (802, 41), (905, 30), (905, 31), (969, 21), (969, 22), (1001, 63), (1001, 65),
+                                  (1002, 44), (1002, 45), (1301, 5), (1601, 5), (1855, 5), (2051, 3), (3071, 3)])
 @pytest.mark.parametrize("offsets", [(0, 0), (1, 0), (3, 5), (8, 1)])
 def test_staged_causal_rows_of_many_rows(device, sk, n, offsets):
     lib, stream = _lib.lib(), torch.cuda.current_stream().cuda_stream

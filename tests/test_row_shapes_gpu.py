@@ -39,11 +39,12 @@ def check(x, y, g, dx, hidden, dtype, what):
 
 
 # rows of three to seven chunks and more, bands of two chunks and more, 8192 rows and more or fewer
-@pytest.mark.parametrize("s,w,batches", [(1152, 288, 29), (1152, 288, 2), (1152, 576, 1), (1472, 368, 6), (2048, 384, 4), (2048, 600, 1),
-                                         (2048, 1024, 1), (2560, 256, 4), (2560, 700, 1), (2560, 1600, 1), (3072, 600, 3), (3072, 600, 2),
-                                         (3072, 1400, 3), (3584, 1200, 3), (3584, 1792, 1), (4096, 200, 2), (4096, 200, 1), (4096, 600, 1),
-                                         (4096, 700, 2), (4096, 1100, 1), (4096, 2600, 1), (4608, 400, 2), (4616, 400, 2), (1504, 200, 6), (1504, 300, 6), (2816, 200, 3), (9216, 200, 1), (6144, 3000, 1), (8192, 256, 1),
-                                         (8192, 1600, 1)])
+@pytest.mark.parametrize("s,w,batches", [(1152, 288, 29), (1152, 288, 2), (1152, 576, 1), (1472, 368, 6), (2048, 384, 4),
+                                         (2048, 600, 1), (2048, 1024, 1), (2560, 256, 4), (2560, 700, 1), (2560, 1600, 1),
+                                         (3072, 600, 3), (3072, 600, 2), (3072, 1400, 3), (3584, 1200, 3), (3584, 1792, 1),
+                                         (4096, 200, 2), (4096, 200, 1), (4096, 600, 1), (4096, 700, 2), (4096, 1100, 1),
+                                         (4096, 2600, 1), (4608, 400, 2), (4616, 400, 2), (1504, 200, 6), (1504, 300, 6),
+                                         (2816, 200, 3), (9216, 200, 1), (6144, 3000, 1), (8192, 256, 1), (8192, 1600, 1)])
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_sliding_window_shapes_by_rows(device, s, w, batches, dtype):
     lib, stream, code = _lib.lib(), torch.cuda.current_stream().cuda_stream, _lib.dtype_code(dtype)
@@ -56,9 +57,13 @@ def test_sliding_window_shapes_by_rows(device, s, w, batches, dtype):
 
 # 513-1024 columns with the loads in front or not; above 1024, 2048 and 4096 columns in the backward pass; rows that are no whole
 # cache lines, 32768 of them or fewer; odd rows, 2048 / 4608 / 6400 / 8192 of them or fewer
-@pytest.mark.parametrize("s,batches", [(576, 1), (888, 6), (1024, 5), (1088, 5), (1088, 4), (1088, 16), (1088, 17), (1088, 33), (1088, 34), (1088, 18), (1088, 19), (1184, 15), (1184, 16), (1184, 31), (1184, 32), (1304, 29), (2112, 3), (2112, 2), (2112, 5), (2824, 4), (2848, 3), (2848, 4), (2944, 4), (3072, 3), (4160, 1), (5136, 1), (5696, 1), (5704, 1), (520, 64), (520, 63),
-                                       (1000, 33), (1032, 32), (1416, 24), (1480, 23), (1488, 23), (2056, 16), (3064, 11), (1001, 9), (1001, 8), (1301, 5), (1301, 4),
-                                       (1601, 2), (1601, 1), (1801, 4), (1801, 3), (1801, 2), (2051, 3), (2051, 2), (4101, 1)])
+@pytest.mark.parametrize("s,batches", [(576, 1), (888, 6), (1024, 5), (1088, 5), (1088, 4), (1088, 16), (1088, 17), (1088, 33),
+                                       (1088, 34), (1088, 18), (1088, 19), (1184, 15), (1184, 16), (1184, 31), (1184, 32),
+                                       (1304, 29), (2112, 3), (2112, 2), (2112, 5), (2824, 4), (2848, 3), (2848, 4), (2944, 4),
+                                       (3072, 3), (4160, 1), (5136, 1), (5696, 1), (5704, 1), (520, 64), (520, 63), (1000, 33),
+                                       (1032, 32), (1416, 24), (1480, 23), (1488, 23), (2056, 16), (3064, 11), (1001, 9), (1001, 8),
+                                       (1301, 5), (1301, 4), (1601, 2), (1601, 1), (1801, 4), (1801, 3), (1801, 2), (2051, 3),
+                                       (2051, 2), (4101, 1)])
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_causal_shapes_by_rows(device, s, batches, dtype):
     lib, stream, code = _lib.lib(), torch.cuda.current_stream().cuda_stream, _lib.dtype_code(dtype)
